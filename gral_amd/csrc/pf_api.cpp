@@ -707,6 +707,21 @@ extern "C" int gral_pf_prepare(gral_pf_handle *h, const gral_pf_params *p) {
         if ((rc = dalloc(h, &fs, (size_t)SYNC_BLOCK0 + 5 * (size_t)d.sync_stride))) return rc;
         HIPCHK(h, hipMemsetAsync(fs, 0, sizeof(int) * ((size_t)SYNC_BLOCK0 + 5 * (size_t)d.sync_stride), h->stream));
         d.sync = fs;
+        d.nact = 1;
+        d.nlow = 0;
+        for (int i = 1; i <= h->nii; ++i)
+            for (int j = 1; j <= h->njj; ++j) {
+                const size_t c = h->i2(i, j);
+                if (h->adv[c] != 1) continue;
+                d.nact = std::max(d.nact, h->vi[c] - h->kk[c]);
+                if (h->cutk[c] != 0) d.nlow = std::max(d.nlow, (int)h->kk[c]);
+            }
+        d.hand_cols = std::max(h->nii, h->njj);
+        if (d.tiled) {
+            d.hand_words = (size_t)(std::max(h->nii, h->njj) / STRIP_ROWS_MIN + 1) * d.hand_cols * d.nkp;
+            if ((rc = dalloc(h, &d.hand, 2 * d.hand_words))) return rc;
+            HIPCHK(h, hipMemsetAsync(d.hand, 0, 2 * d.hand_words * sizeof(unsigned long long), h->stream));
+        }
     }
     d.planes = nullptr;
     d.rec3 = nullptr;

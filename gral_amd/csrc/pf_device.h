@@ -45,6 +45,10 @@ struct DomT {
     int tiled;                       // 2: strip-pipelined sweeps, 0: one launch per anti-diagonal
     P<int> sync;                     // strip sweeps: [64] header (sticky error flag at 0), then 4 blocks
     int sync_stride;                 //   of sync_stride ints (ticket, unused, progress per strip)
+    P<unsigned long long> hand;      // values handed from strip to strip: {value, tag} words [2][strip][hand_cols][nkp]
+    size_t hand_words;               // words of one of the two
+    int hand_cols;
+    int nact, nlow;                  // largest VI - KKART, and KKART + 1 - KSTART, of the active columns
     P<float> planes;                 // [cells][12 (U, V) or 8 (W)] mixing-length coefficient records
     P<float> rec3;                   // [cells][3]  C, TERMP and P of the same cells
     P<float> wcol;                   // [columns] wall term of the U / V sweep at KKART+1
@@ -176,6 +180,7 @@ struct MomAdj {
 
 #define SYNC_BLOCK0 64               // Dom::sync: sticky error flag at 0, sweep blocks from here
 #define STRIP_ROWS 15                // sweep rows per strip workgroup (plus one chain wave)
+#define STRIP_ROWS_MIN 7             // fewest rows of a strip (strip_rows())
 
 __device__ __forceinline__ size_t c2(const DomG &d, int i, int j) { return (size_t)i * (size_t)d.nj2 + (size_t)j; }
 __device__ __forceinline__ size_t c3(const DomG &d, int i, int j) { return c2(d, i, j) * (size_t)d.nkp; }

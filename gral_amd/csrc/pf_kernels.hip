@@ -78,18 +78,20 @@ __global__ void k_fill_u32(unsigned *p, size_t n, unsigned v) {
     size_t g = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (g < n) p[g] = v;
 }
-// zero the pressure row scratch of every situation (PIMP/QIMP rows are fresh
-// arrays at the start of each pressure pass)
-// and the strip synchronisation blocks of the iteration's sweeps
-__global__ void k_zero_rows(const Dom *__restrict__ ds, int both) {
+// Clears the strip synchronisation blocks of the iteration's sweeps; for the
+// per-diagonal sweeps (diag) also the pressure row scratch of every situation
+// (PIMP/QIMP rows are fresh arrays at the start of each pressure pass; the
+// strips keep them in LDS).
+__global__ void k_zero_rows(const Dom *__restrict__ ds, int diag) {
     const DomG &d = reinterpret_cast<const DomG *>(ds)[blockIdx.z];
     size_t n = (size_t)d.nj2 * d.nkp;
     size_t g = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g < n) {
+    if (diag && g < n) {
         d.prow_q[g] = 0.0f;
-        if (both) d.prow_p[g] = 0.0f;
+        d.prow_p[g] = 0.0f;
     }
     if (d.sync && g < (size_t)5 * d.sync_stride) d.sync[SYNC_BLOCK0 + g] = 0;
+    if (d.sync && g == 0) d.sync[1] += 1;                     // the hand-off tags of this iteration's sweeps
 }
 
 // ------------------------------------------------------------------------
@@ -1435,6 +1437,9 @@ __global__ __launch_bounds__(4 * WAVE) void k_ml_coef(const Dom *__restrict__ ds
                 m = unpack_meta(ldg4i(d.meta + c2(d, i, j)));
             }
             if (m.adv) {
+                // U and V: the levels inside a building are neither updated nor
+                // read by the recurrence above them
+                if (COMP != 2) m.KSTART = m.KK + 1;
                 n = m.VI - m.KSTART + 1;
                 const ColInfo q = col_info(d, i, j);
                 int *sc = scol + c * SCOL;
@@ -1576,119 +1581,12 @@ __device__ __forceinline__ void chain_fwd(const float *__restrict__ D, const flo
     }
 }
 
-// relaxed back-substitution downwards: X[-t] += relax*(P[-t]*X[-t+1] + Q[-t] - X[-t]), t = 0..n-1
-__device__ __forceinline__ void chain_back(const float *__restrict__ P, const float *__restrict__ Q,
-                                           const float *__restrict__ X, float *__restrict__ Xn, float relax, int n,
-                                           int nmax, float *sink) {
-    float up = X[1];
-    float cp[CH], cq[CH], cx[CH];
-    // each chunk addresses its CH levels from the lowest one upwards, so that
-    // the accesses pair up with positive offsets (ds_read2/ds_write2 from one
-    // base) and few enough reads are in flight for a partial LDS wait
-    {
-        const float *Pb = P - (CH - 1), *Qb = Q - (CH - 1), *Xb = X - (CH - 1);
-#pragma unroll
-        for (int u = 0; u < CH; ++u) { cp[u] = Pb[CH - 1 - u]; cq[u] = Qb[CH - 1 - u]; cx[u] = Xb[CH - 1 - u]; }
-    }
-#pragma unroll
-    for (int h = 0; h < MAXCH; ++h) {
-        const int t = h * CH;
-        if (t >= nmax) break;
-        float np[CH], nq[CH], nx[CH];
-        const int o = (t + CH < n) ? t + CH : 0;
-        const float *Pb = P - (o + CH - 1), *Qb = Q - (o + CH - 1), *Xb = X - (o + CH - 1);
-#pragma unroll
-        for (int u = 0; u < CH; ++u) { np[u] = Pb[CH - 1 - u]; nq[u] = Qb[CH - 1 - u]; nx[u] = Xb[CH - 1 - u]; }
-        __builtin_amdgcn_sched_barrier(0);                // keep the next chunk's reads ahead of this chunk
-        float *Xw = (t < n) ? Xn - (t + CH - 1) : sink;   // a lane past its end stores to its sink
-#pragma unroll
-        for (int u = 0; u < CH; ++u) {
-            float x = cx[u] + relax * (cp[u] * up + cq[u] - cx[u]);
-            Xw[CH - 1 - u] = x;
-            up = x;
-        }
-#pragma unroll
-        for (int u = 0; u < CH; ++u) { cp[u] = np[u]; cq[u] = nq[u]; cx[u] = nx[u]; }
-    }
-}
-
-// pressure, downwards from the top: Q[-t] = (A[-t]*Q[-t+1] + D[-t]) * T[-t] with
-// A (= ATP) held in Q on entry and Q[1] = qtop, t = 0..n-1
-__device__ __forceinline__ void chain_pdown(const float *__restrict__ D, const float *__restrict__ T, float *__restrict__ Q,
-                                            float qtop, int n, int nmax, float *sink) {
-    float Qn = qtop;
-    float ca[CH], cd[CH], ct[CH];
-    // chunks addressed from their lowest level upwards, as in chain_back
-    {
-        const float *Qb = Q - (CH - 1), *Db = D - (CH - 1), *Tb = T - (CH - 1);
-#pragma unroll
-        for (int u = 0; u < CH; ++u) { ca[u] = Qb[CH - 1 - u]; cd[u] = Db[CH - 1 - u]; ct[u] = Tb[CH - 1 - u]; }
-    }
-#pragma unroll
-    for (int h = 0; h < MAXCH; ++h) {
-        const int t = h * CH;
-        if (t >= nmax) break;
-        float na[CH], nd[CH], nt[CH];
-        const int o = (t + CH < n) ? t + CH : 0;
-        const float *Qb = Q - (o + CH - 1), *Db = D - (o + CH - 1), *Tb = T - (o + CH - 1);
-#pragma unroll
-        for (int u = 0; u < CH; ++u) { na[u] = Qb[CH - 1 - u]; nd[u] = Db[CH - 1 - u]; nt[u] = Tb[CH - 1 - u]; }
-        __builtin_amdgcn_sched_barrier(0);                // keep the next chunk's reads ahead of this chunk
-        float *Qw = (t < n) ? Q - (t + CH - 1) : sink;
-#pragma unroll
-        for (int u = 0; u < CH; ++u) {
-            float q = (ca[u] * Qn + cd[u]) * ct[u];
-            Qw[CH - 1 - u] = q;
-            Qn = q;
-        }
-#pragma unroll
-        for (int u = 0; u < CH; ++u) { ca[u] = na[u]; cd[u] = nd[u]; ct[u] = nt[u]; }
-    }
-}
-
-// pressure, upwards: N[t] = P[t]*N[t-1] + Q[t], t = 0..n-1, N[-1] = bottom
-__device__ __forceinline__ void chain_pup(const float *__restrict__ P, const float *__restrict__ Q, float *__restrict__ N,
-                                          float bottom, int n, int nmax, float *sink) {
-    float dp = bottom;
-    float cp[CH], cq[CH];
-#pragma unroll
-    for (int u = 0; u < CH; ++u) { cp[u] = P[u]; cq[u] = Q[u]; }
-#pragma unroll
-    for (int h = 0; h < MAXCH; ++h) {
-        const int t = h * CH;
-        if (t >= nmax) break;
-        float np[CH], nq[CH];
-        const int o = (t + CH < n) ? t + CH : 0;
-#pragma unroll
-        for (int u = 0; u < CH; ++u) { np[u] = P[o + u]; nq[u] = Q[o + u]; }
-        __builtin_amdgcn_sched_barrier(0);                // keep the next chunk's reads ahead of this chunk
-        float *Nw = (t < n) ? N : sink - t;
-#pragma unroll
-        for (int u = 0; u < CH; ++u) {
-            float x = cp[u] * dp + cq[u];
-            Nw[t + u] = x;
-            dp = x;
-        }
-#pragma unroll
-        for (int u = 0; u < CH; ++u) { cp[u] = np[u]; cq[u] = nq[u]; }
-    }
-}
-
 // largest value of v over the lanes of the wave that pass `on` (0 if none)
 __device__ __forceinline__ int wave_max(int v, bool on) {
     int m = on ? v : 0;
     for (int off = WAVE / 2; off > 0; off >>= 1) m = max(m, __shfl_xor(m, off));
     return __builtin_amdgcn_readfirstlane(m);
 }
-
-// per-level values of one column that do not change during the sweep, loaded
-// one local step ahead
-struct MlPre {
-    float aw, as, ae, an, e, f, g, c0, x1, x2, x3, x4, c, t, p;
-    float x, xa, xb;      // own old value; old neighbours in the +IS (xa) and +JS (xb) directions
-    float ni, nj;         // -IS / -JS neighbours, prefetched only when another strip or the boundary holds them
-    float ap0;            // transient coefficient of the level (k-eps)
-};
 
 // p + byte_off with a 32-bit byte offset: with a uniform base the access can
 // take the scalar-base form (base in scalar registers, 32-bit lane offset), so
@@ -1697,46 +1595,6 @@ __device__ __forceinline__ const gf32 *at_bytes(const gf32 *base, unsigned byte_
     typedef const char __attribute__((address_space(1))) gc8;
     return (const gf32 *)((const gc8 *)base + byte_off);
 }
-template <int COMP, int KIND>
-__device__ __forceinline__ void ml_prefetch(const DomG &d, const gf32 *Pc, const gf32 *R3, const gf32 *Xc,
-                                            const gf32 *Xa, const gf32 *Xb, unsigned k, MlPre &r) {
-    // Pc, R3, Xc, Xa, Xb: the column's records and values and its +IS / +JS
-    // neighbours (uniform bases, so the level's byte offset is the only
-    // per-lane part of each address)
-    const gf32 *P = at_bytes(Pc, k * (unsigned)(4 * rec_floats<COMP>()));
-    float4 v0 = ldg4(P), v2 = ldg4(P + 4);
-    float3 v1 = ldg3(at_bytes(R3, k * 12u));
-    r.aw = v0.x; r.as = v0.y; r.ae = v0.z; r.an = v0.w;
-    r.c = v1.x; r.t = v1.y; r.p = v1.z;
-    r.f = v2.x; r.g = v2.y; r.e = v2.z;
-    if (COMP == 2) {
-        r.x1 = v2.w;
-        r.c0 = r.x2 = r.x3 = r.x4 = 0.0f;
-    } else {
-        float4 v3 = ldg4(P + 8);
-        r.c0 = v2.w;
-        r.x1 = v3.x; r.x2 = v3.y; r.x3 = v3.z; r.x4 = v3.w;
-    }
-    r.x = *at_bytes(Xc, 4u * k);
-    r.xa = *at_bytes(Xa, 4u * k);
-    r.xb = *at_bytes(Xb, 4u * k);
-    if (KIND != 0) r.ap0 = d.ap0[k];
-}
-
-__device__ __forceinline__ ColInfo meta_col(const Meta &m, int i, int j, int W) {
-    ColInfo q;
-    q.i = i; q.j = j; q.KK = m.KK; q.KSTART = m.KSTART; q.VI = m.VI; q.W = W; q.vegp = m.vegp;
-    q.as = q.an = q.aw = q.ae = false; q.cutk = q.cov = q.ht = q.ho = q.z0s = 0.0f;
-    return q;
-}
-
-// prefetched per-level values of one column of the pressure sweep
-struct PrPre {
-    float div, t, p, pa, pb;       // DIV / DTIME, TERMP, PIMP, old DPM in the +IS (i) and +JS (j) directions
-    float dn;                      // DPMNEW of the cell (read-modify-written one step later)
-    float ni, nj;                  // -IS / -JS neighbours when another strip or the boundary holds them
-};
-
 // ------------------------------------------------------------------------
 // Strip-pipelined sweeps.  Strip B reads the last row of strip B-1 (its new
 // values, and for the pressure sweep the QIMP row scratch) and nothing else
@@ -1772,13 +1630,6 @@ struct PrPre {
 #ifndef STRIP_PUBLISH
 #define STRIP_PUBLISH 1
 #endif
-#ifndef ML_PUBLISH_UV
-#define ML_PUBLISH_UV 1
-#endif
-#ifndef ML_PUBLISH_W
-#define ML_PUBLISH_W 1
-#endif
-template <int COMP> __device__ __forceinline__ constexpr int ml_publish() { return COMP == 2 ? ML_PUBLISH_W : ML_PUBLISH_UV; }
 #define STRIP_TIMEOUT_TICKS 200000000ull
 
 __device__ __forceinline__ int load_agent(const gi32 *p) {
@@ -1842,526 +1693,977 @@ __device__ __forceinline__ void strip_publish(gi32 *mine, int v, int lane) {
     if (lane == 0) store_agent(mine, v);
 }
 
-// KIND 0: mixing length; KIND 1: k-eps, KIND 2: no diffusion (sources by
-// ke_source, the TDMA divides by the denominators k_ml_coef<.., KIND> stored).
-template <int COMP, int KIND = 0>
-__global__ __launch_bounds__(STRIP_WAVES * WAVE) void k_ml_strip(const Dom *__restrict__ ds, int IS, int JS) {
-    const DomG &d = reinterpret_cast<const DomG *>(ds)[blockIdx.z];                   // situation of this launch slice
-    const gf32 *planes = d.planes;
-    extern __shared__ float sm[];
-    const int nkp = d.nkp, nkl = lds_slot(nkp);
-    const int oa = (COMP == 0) ? 3 : 2, ia = (COMP == 1) ? 3 : 2, ob = d.nii - 1, ib = d.njj - 1;
-    const int nstrip = (ib - ia + ROWS) / ROWS, nsteps = (ob - oa + 1) + ROWS - 1;
-    const int r = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
-    const bool chainw = r == ROWS;                            // the chain wave owns no row
-    gi32 *sync = d.sync + SYNC_BLOCK0 + (size_t)(1 + COMP) * d.sync_stride;
-    // per row: D, C, T, P, Q and the back-substitution results Xn of even and
-    // odd steps (a row stores its previous column while the next one is solved)
-    float *sD = sm + (size_t)r * 7 * nkl + SLOT_PAD, *sC = sD + nkl, *sT = sC + nkl, *sP = sT + nkl, *sQ = sP + nkl;
-    float *sXn0 = sQ + nkl;                                   // [2][nkl] by step parity
-    float *xbuf = sm + (size_t)ROWS * 7 * nkl + SLOT_PAD;      // [2][ROWS] slots of whole columns (old values)
-    float *sdzk = sm + (size_t)ROWS * 9 * nkl;                // [nkp]
-    int *sinfo = (int *)(sdzk + nkp);                         // [2][ROWS] per row: active, KSTART, KK, VI, KKm
-    int *sctl = sinfo + 10 * ROWS;                            // strip index of this workgroup
-    float *sdump = (float *)(sctl + 4);                       // [WAVE][CH] sinks of the chains
-    if (threadIdx.x == 0) sctl[0] = __hip_atomic_fetch_add(&sync[0], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    for (int k = threadIdx.x; k < nkp; k += STRIP_WAVES * WAVE) sdzk[k] = d.dzk[k];
-    __syncthreads();
-    const int B = sctl[0];
-    if (B >= nstrip) return;                                  // uniform over the workgroup
-    gi32 *mine = sync + SYNC_HDR + B;
-    gf32 *X = (COMP == 0 ? d.uk : COMP == 1 ? d.vk : d.wk);
-    if (chainw) {
-        // The chain wave runs its own loop with the same three barriers per
-        // step as the row waves (s_barrier counts waves, wherever they are in
-        // the code), so none of the row waves' loop-carried prefetch registers
-        // is live in the recurrences.  It issues ahead of the row waves on its
-        // SIMD (wave priority): the recurrences are the step's serial path,
-        // while the rows' look-ahead that overlaps them has slack.
-        __builtin_amdgcn_s_setprio(3);
-        // The rows publish the column data of step s one phase early (before
-        // the barrier that ends the recurrences of step s-1), so the chain wave
-        // reads them and takes its wave-wide maxima while the rows assemble.
-        const int cl = lane < ROWS ? lane : 0;
-        bool on = false;
-        int KK = 0, VI = 0, nf = 0, nb = 0, nfmax = 0, nbmax = 0;
-        auto info = [&](int s) {
-            const int *si = sinfo + (s & 1) * 5 * ROWS;
-            on = lane < ROWS && si[cl * 5];
-            const int KSTART = si[cl * 5 + 1], KKm = si[cl * 5 + 4];
-            KK = si[cl * 5 + 2]; VI = si[cl * 5 + 3];
-            // first level the back-substitution updates (U/V skip levels inside
-            // the building or its upstream neighbour; W updates every level)
-            const int kend = (COMP == 2) ? KSTART : max(KSTART, KKm + 1);
-            nf = VI - KK - 1; nb = VI - kend + 1;
-            nfmax = wave_max(nf, on); nbmax = wave_max(nb, on);
-        };
-        // The chain wave also stores the last row's results (the only column
-        // another strip reads) and publishes the strip's progress, while the
-        // rows assemble the next step: these stores are its only vector-memory
-        // operations, so the wait before a publish finds those of the step
-        // before complete, and the last row's own second phase is no longer
-        // than the others'.
-        const int blast = ia + B * ROWS + ROWS - 1;
-        auto store_last = [&](int s) {
-            const int l = s - (ROWS - 1);
-            if (__builtin_amdgcn_readlane((int)on, ROWS - 1) && blast <= ib && l >= 0 && oa + l <= ob) {
-                const int vil = __builtin_amdgcn_readlane(VI, ROWS - 1);
-                const int kendl = vil - __builtin_amdgcn_readlane(nb, ROWS - 1) + 1;
-                int i, j;
-                sweep_to_ij(d, 0, oa + l, blast, IS, JS, i, j);
-                gf32 *Xp = X + c3(d, i, j);
-                const float *xn = sm + (size_t)(ROWS - 1) * 7 * nkl + SLOT_PAD + (size_t)(5 + (s & 1)) * nkl;
-                for (int k = kendl + lane; k <= vil; k += WAVE) st_through(Xp + (unsigned)k, xn[k]);
-            }
-        };
-        for (int s = 0; s < nsteps; ++s) {
-            lds_barrier();                                    // the rows' sources are assembled
-            if (s == 0) info(0);
-            if (on) {
-                float *D = sm + (size_t)cl * 7 * nkl + SLOT_PAD;
-                float *Cc = D + nkl, *T = Cc + nkl, *P = T + nkl, *Q = P + nkl, *Xn = Q + nkl + (size_t)(s & 1) * nkl;
-                const float *Xs = xbuf + (size_t)((s & 1) * ROWS + cl) * nkl;
-                chain_fwd<KIND != 0>(D + KK + 2, Cc + KK + 2, T + KK + 2, Q + KK + 2, nf, nfmax, Q[KK + 1], sdump + lane * CH);
-                chain_back(P + VI, Q + VI, Xs + VI, Xn + VI, d.relax, nb, nbmax, sdump + lane * CH);
-            }
-            lds_barrier();                                    // the recurrences are done
-            // progress s: the last row's results of steps < s are stored (those
-            // of step s-1 one step ago)
-            if (s > 0 && s % ml_publish<COMP>() == 0) strip_publish(mine, s, lane);
-            store_last(s);
-            if (s + 1 < nsteps) info(s + 1);
-        }
-        strip_publish(mine, nsteps, lane);
-        return;
-    }
-    const int b = ia + B * ROWS + r;
-    const bool row_ok = b <= ib;
-    StripWait sw{B > 0 ? sync + SYNC_HDR + B - 1 : nullptr, d.sync, B > 0 ? 0 : 0x7fffffff, nsteps,
-                 wall_clock64() + STRIP_TIMEOUT_TICKS};
-    MlPre pre[2];
-    float xfull[2];
-    float wn = 0.0f;                                          // wall term of the located column (U, V)
-    Meta mn;
-    int in_ = 0, jn_ = 0;
-    bool inr_n = false;
-    // the metadata of a column is requested one step before its data (the data
-    // loads need it for their addresses)
-    auto meta_at = [&](int s) {
-        int l = s - r, i, j;
-        if (row_ok && l >= 0 && oa + l <= ob) {
-            sweep_to_ij(d, 0, oa + l, b, IS, JS, i, j);
-            return ldc4i(d.meta + c2(d, i, j));
-        }
-        return make_int4(0, -1, 0, 0);
-    };
-    int4 mq = meta_at(0);
-    auto locate = [&](int s) {
-        int l = s - r;                                        // column a = oa + l
-        inr_n = row_ok && l >= 0 && oa + l <= ob;
-        const int4 m4 = mq;
-        mq = meta_at(s + 1);
-        mn.adv = false;
-        if (inr_n) {
-            sweep_to_ij(d, 0, oa + l, b, IS, JS, in_, jn_);
-            in_ = __builtin_amdgcn_readfirstlane(in_);        // uniform: column bases in scalar registers
-            jn_ = __builtin_amdgcn_readfirstlane(jn_);
-            mn = unpack_meta(m4);
-            const gf32 *Xc = X + c3(d, in_, jn_);
-#pragma unroll
-            for (int m = 0; m < 2; ++m) {
-                const unsigned k = lane + WAVE * m;
-                if (k < (unsigned)nkp) xfull[m] = *at_bytes(Xc, 4u * k);
-            }
-        }
-        if (mn.adv) {
-            if (COMP != 2) wn = d.wcol[c2(d, in_, jn_)];
-            const size_t o = c3(d, in_, jn_);
-            const gf32 *Pc = planes + o * rec_floats<COMP>(), *R3 = d.rec3 + o * 3, *Xc = X + o;
-            const gf32 *Xa = X + c3(d, in_ + IS, jn_), *Xb = X + c3(d, in_, jn_ + JS), *Xi = X + c3(d, in_ - IS, jn_);
-#pragma unroll
-            for (int m = 0; m < 2; ++m) {
-                const int k = mn.KSTART + lane + WAVE * m;
-                if (k <= mn.VI) {
-                    ml_prefetch<COMP, KIND>(d, Pc, R3, Xc, Xa, Xb, (unsigned)k, pre[m]);
-                    if (l == 0) pre[m].ni = *at_bytes(Xi, 4u * (unsigned)k);
-                }
-            }
-        }
-    };
-    // row 0's -JS neighbours lie in the previous strip's last row: row 0 issues
-    // its other look-ahead loads first, then waits for that strip, then reads them
-    auto locate_prev = [&]() {
-        if (mn.adv) {
-#pragma unroll
-            for (int m = 0; m < 2; ++m) {
-                int k = mn.KSTART + lane + WAVE * m;
-                if (k <= mn.VI) pre[m].nj = ld_handoff(X + c3(d, in_, jn_ - JS) + (unsigned)k);
-            }
-        }
-    };
-    // the chain wave's data of the column located for step s (one lane writes)
-    auto put_info = [&](int s) {
-        if (lane == 0) {
-            int *si = sinfo + (s & 1) * 5 * ROWS;
-            si[r * 5] = mn.adv;
-            if (mn.adv) {
-                const int KKm = (COMP == 0) ? mn.KKmi : (COMP == 1) ? mn.KKmj : mn.KK;
-                si[r * 5 + 1] = mn.KSTART; si[r * 5 + 2] = mn.KK; si[r * 5 + 3] = mn.VI; si[r * 5 + 4] = KKm;
-            }
-        }
-    };
-    locate(0);
-    put_info(0);
-    if (r == 0) {
-        sw.wait(ROWS);
-        locate_prev();
-    }
-    // The results of a step are merged on use: level k of a row's previous
-    // column is the recurrence output (Xn of that step's parity) where the
-    // back-substitution updated it (kend..VI), else the old value in the column
-    // buffer.  Each row but the last (whose column the chain wave stores)
-    // stores the updated levels of its previous column in the next step's
-    // second phase, after issuing that phase's look-ahead loads: vector-memory
-    // waits count loads and stores in one ordered counter, so a store issued
-    // before those loads would make every wait for them (in the look-ahead
-    // itself and in the next assembly) wait for the write as well.
-    int pkend = 1 << 30, pvi = -1;                            // own previous column: updated levels
-    size_t po = 0;
-    auto store_prev = [&](const float *xn) {
-        gf32 *Xp = X + po;
-        for (int k = pkend + lane; k <= pvi; k += WAVE) st_through(Xp + (unsigned)k, xn[k]);
-    };
-    for (int s = 0; s < nsteps; ++s) {
-        const bool act = mn.adv, inr = inr_n;
-        const Meta mt = mn;
-        const int i = in_, j = jn_;
-        const float wcur = wn;
-        const ColInfo q = meta_col(mt, i, j, d.simd);
-        float *xcur = xbuf + (size_t)((s & 1) * ROWS + r) * nkl;
-        const float *xw_lds = xbuf + (size_t)(((s - 1) & 1) * ROWS + r) * nkl;
-        const float *xs_lds = xbuf + (size_t)(((s - 1) & 1) * ROWS + r - 1) * nkl;
-        const float *xprev = sXn0 + (size_t)((s - 1) & 1) * nkl;   // recurrence output of step s-1
-        const float *xs_new = xprev - (size_t)7 * nkl;       // row r-1's
-        const int *sp = sinfo + ((s - 1) & 1) * 5 * ROWS;
-        const bool w_in = (s - r >= 1), s_in = (r >= 1);
-        if (inr) {
-#pragma unroll
-            for (int m = 0; m < 2; ++m) {
-                int k = lane + WAVE * m;
-                if (k < nkp) xcur[k] = xfull[m];
-            }
-        }
-        if (act) {
-            const int KKP1 = q.KK + 1;
-            // updated levels of the southern neighbour's column (row r-1, previous step)
-            int skend = 1 << 30, svi = -1;
-            if (s_in && sp[(r - 1) * 5]) {
-                const int sks = sp[(r - 1) * 5 + 1], skm = sp[(r - 1) * 5 + 4];
-                skend = (COMP == 2) ? sks : max(sks, skm + 1);
-                svi = sp[(r - 1) * 5 + 3];
-            }
-#pragma unroll
-            for (int m = 0; m < 2; ++m) {
-                int k = q.KSTART + lane + WAVE * m;
-                if (k <= q.VI) {
-                    const MlPre &r_ = pre[m];
-                    float xnew_i = w_in ? ((k >= pkend && k <= pvi) ? xprev[k] : xw_lds[k]) : r_.ni;
-                    float xnew_j = s_in ? ((k >= skend && k <= svi) ? xs_new[k] : xs_lds[k]) : r_.nj;
-                    float xw = (IS == 1) ? xnew_i : r_.xa, xe = (IS == 1) ? r_.xa : xnew_i;
-                    float xs = (JS == 1) ? xnew_j : r_.xb, xn = (JS == 1) ? r_.xb : xnew_j;
-                    MlPieces pc;
-                    pc.AW1 = r_.aw; pc.AS1 = r_.as; pc.AE1 = r_.ae; pc.AN1 = r_.an; pc.e = r_.e; pc.f = r_.f;
-                    pc.g = r_.g; pc.w = wcur; pc.c0 = r_.c0; pc.X1 = r_.x1; pc.X2 = r_.x2; pc.X3 = r_.x3; pc.X4 = r_.x4;
-                    float D;
-                    if constexpr (KIND != 0) D = ke_source<COMP, KIND == 1>(d, q, k, sdzk[k], r_.ap0, pc, xw, xs, xe, xn, r_.x);
-                    else D = ml_source<COMP>(d, q, k, sdzk[k], pc, xw, xs, xe, xn, r_.x);
-                    sD[k] = D; sC[k] = r_.c; sT[k] = r_.t; sP[k] = r_.p;
-                    if (k <= KKP1) sQ[k] = (KIND != 0) ? D / r_.t : D * r_.t;
-                }
-            }
-        }
-        const int kend = (COMP == 2) ? q.KSTART : max(q.KSTART, ((COMP == 0) ? mt.KKmi : mt.KKmj) + 1);
-        lds_barrier();
-        // while the chain wave runs the recurrences every row prefetches its
-        // next column, then stores its previous one.  The look-ahead of row r
-        // reads columns that rows r and r+1 write two steps later at the
-        // earliest (for the last row, the next strip, which waits for this one);
-        // row 0 also reads the previous strip's last row, after its wait.
-        locate(s + 1);
-        if (s + 1 < nsteps) put_info(s + 1);
-        if (r == 0) {
-            sw.wait(s + 1 + ROWS);
-            locate_prev();
-        }
-        if (r != ROWS - 1) store_prev(xprev);
-        pkend = act ? kend : 1 << 30;
-        pvi = act ? q.VI : -1;
-        po = c3(d, i, j);
-        lds_barrier();                                        // the recurrence outputs are ready
-    }
-    if (r != ROWS - 1) store_prev(sXn0 + (size_t)((nsteps - 1) & 1) * nkl);
+// ------------------------------------------------------------------------
+// Strip rows in LDS.  A row's operands are stored by level relative to the
+// column's first free level, t = k - KKART - 1: the recurrences of all rows then
+// start at t = 0 on a 16-byte boundary whatever the columns' ground heights, and
+// walk chunks of CHK levels with ds_read_b128 / ds_write_b128 (a lone wave
+// issues an instruction every 4.5 cycles and a dependent one every 8.4, so with
+// 4-byte LDS accesses the recurrences were bound by their own instruction
+// stream: 46 and 55 cycles per level forward and back, 31 and 46 with 16-byte
+// accesses, against 25 and 42 for their 3 and 5 dependent operations).  An array
+// holds strip_low() levels below t = 0 (W inside buildings; the lowest chunk
+// is where lanes that are done store) and one spare chunk above the tallest
+// column (read ahead, or written by lanes past their own end).  The row stride
+// is 4 modulo 64 words: the 16-byte accesses of the chain wave's lanes fall into
+// different banks.
+// ------------------------------------------------------------------------
+#define CHK 8
+__host__ __device__ inline int strip_low(int nlow) { return ((nlow + CHK - 1) & ~(CHK - 1)) + CHK; }
+__host__ __device__ inline int strip_len(int nlow, int nact) { return strip_low(nlow) + ((nact + CHK - 1) & ~(CHK - 1)) + CHK; }
+__host__ __device__ inline int strip_stride(int arrays, int len) { return arrays * len + ((4 - arrays * len) & 63); }
+
+struct Chunk { float v[CHK]; };
+__device__ __forceinline__ Chunk ld_chunk(const float *p) {
+    const float4 a = *(const float4 *)p, b = *(const float4 *)(p + 4);
+    return Chunk{{a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w}};
+}
+__device__ __forceinline__ void st_chunk(float *p, const Chunk &c) {
+    *(float4 *)p = make_float4(c.v[0], c.v[1], c.v[2], c.v[3]);
+    *(float4 *)(p + 4) = make_float4(c.v[4], c.v[5], c.v[6], c.v[7]);
+}
+// largest value over the 16 lanes of each row of the wave (lanes 0-15, 16-31,
+// ...): rotations within the row instead of LDS permutes
+__device__ __forceinline__ int row_max(int v) {
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x128, 0xf, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x124, 0xf, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x122, 0xf, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x121, 0xf, 0xf, false));
+    return v;
 }
 
-// Pressure sweep on strips.  The QIMP row scratch of sweep row a travels
-// with the wavefront through LDS (ring slot (a - oa) mod RING; the ROWS rows of
-// a step hold ROWS consecutive sweep rows): row 0 loads it from global memory
-// (as strip B-1 left it), each row updates it with its column, and the last
-// row stores it back for strip B+1.
-#define RING 16
-__global__ __launch_bounds__(STRIP_WAVES * WAVE) void k_pressure_strip(const Dom *__restrict__ ds, int IS, int JS, int slot) {
-    const DomG &d = reinterpret_cast<const DomG *>(ds)[blockIdx.z];
-    const gf32 *ptab = d.ptab[IS == 1 ? 0 : 1], *ttab = d.ttab[IS == 1 ? 0 : 1];
-    extern __shared__ float sm[];
-    const int nkp = d.nkp, nkl = lds_slot(nkp);
-    const int oa = 2, ia = 2, ob = d.njj - 1, ib = d.nii - 1;
-    const int nstrip = (ib - ia + ROWS) / ROWS, nsteps = (ob - oa + 1) + ROWS - 1;
+// The chunk loops are straight-line blocks of CHK_BLOCK chunks: within a block
+// the compiler waits for exactly the reads a chunk needs, while a loop's back
+// edge makes it wait for every LDS access in flight.  Each chunk issues the
+// next chunk's reads before its own operations, in one group: an LDS access
+// between two dependent operations costs more than its issue.  Measured on one
+// wave, 40 levels, in cycles per level: forward 29.6, back 39.7, pressure up
+// 24.6; with two chunks per loop round 34.7, 49.8, 29.3; with the reads between
+// the operations 37.6, 44.7, 25.4.
+#define CHK_BLOCK 8
+
+// forward: Q[t] = (D[t] + C[t]*Q[t-1]) * T[t] for nch chunks from t = 0, where
+// Q[0] = D[0]*T[0]; Q replaces D
+template <bool DIV>
+__device__ __forceinline__ void strip_fwd(float *DQ, const float *C, const float *T, int nch) {
+    float q = 0.0f;
+    Chunk d[2], c[2], t[2];
+    d[0] = ld_chunk(DQ); c[0] = ld_chunk(C); t[0] = ld_chunk(T);
+    c[0].v[0] = -0.0f;                                        // -0*0 added to D[0] leaves it as it is
+    for (int b = 0; b < nch; b += CHK_BLOCK) {
+#pragma unroll
+        for (int h = 0; h < CHK_BLOCK; ++h) {
+            if (b + h >= nch) return;
+            const int k = h & 1, n = k ^ 1;
+            d[n] = ld_chunk(DQ + (h + 1) * CHK); c[n] = ld_chunk(C + (h + 1) * CHK); t[n] = ld_chunk(T + (h + 1) * CHK);
+            __builtin_amdgcn_sched_barrier(0);                // the next chunk's reads stay ahead of this chunk
+#pragma unroll
+            for (int u = 0; u < CHK; ++u) {
+                const float s = d[k].v[u] + c[k].v[u] * q;
+                q = DIV ? s / t[k].v[u] : s * t[k].v[u];
+                d[k].v[u] = q;
+            }
+            st_chunk(DQ + h * CHK, d[k]);
+        }
+        DQ += CHK_BLOCK * CHK; C += CHK_BLOCK * CHK; T += CHK_BLOCK * CHK;
+    }
+}
+
+// relaxed back-substitution from t = n-1 down, nch chunks starting with the one
+// that holds t = n-1: X[t] += relax*(P[t]*X[t+1] + Q[t] - X[t]).  part: some lane's
+// column ends inside its first chunk.  Lanes that are done go on in the chunk
+// at low (the arrays' start).
+__device__ __forceinline__ void strip_back(const float *P, const float *Q, float *X, float relax, int n, int nch, bool part,
+                                           int low) {
+    int o = (n - 1) & ~(CHK - 1);
+    const int top = n - o;
+    float up = X[n];
+    Chunk p[2], q[2], x[2];
+    p[0] = ld_chunk(P + o); q[0] = ld_chunk(Q + o); x[0] = ld_chunk(X + o);
+    for (int b = 0; b < nch; b += CHK_BLOCK) {
+#pragma unroll
+        for (int h = 0; h < CHK_BLOCK; ++h) {
+            if (b + h >= nch) return;
+            const int k = h & 1, m = k ^ 1, on = max(o - CHK, -low);
+            p[m] = ld_chunk(P + on); q[m] = ld_chunk(Q + on); x[m] = ld_chunk(X + on);
+            __builtin_amdgcn_sched_barrier(0);
+            if (h == 0 && part && b == 0) {
+#pragma unroll
+                for (int u = CHK - 1; u >= 0; --u) {
+                    const float r = x[k].v[u] + relax * (p[k].v[u] * up + q[k].v[u] - x[k].v[u]);
+                    up = (u >= top) ? up : r;
+                    x[k].v[u] = r;
+                }
+            } else {
+#pragma unroll
+                for (int u = CHK - 1; u >= 0; --u) {
+                    up = x[k].v[u] + relax * (p[k].v[u] * up + q[k].v[u] - x[k].v[u]);
+                    x[k].v[u] = up;
+                }
+            }
+            st_chunk(X + o, x[k]);
+            o = on;
+        }
+    }
+}
+
+// Hand-off between strips: the last row's new values go to the next strip as
+// 8-byte {value, tag} words, each one store, so the reader needs no progress
+// counter: a word whose tag is this sweep's holds this sweep's value.  The tag
+// counts the situation's iterations (sync[1], advanced by k_zero_rows) and
+// names the sweep, so no word of an earlier sweep matches.  Against a progress
+// counter the writer need not wait for its stores and the reader not for a poll
+// before its loads.
+typedef unsigned long long __attribute__((address_space(1))) gu64;
+__device__ __forceinline__ unsigned hand_tag(const DomG &d, int kind) { return 8u * (unsigned)d.sync[1] + (unsigned)kind; }
+__device__ __forceinline__ void hand_put(gu64 *p, float v, unsigned tag) {
+    __hip_atomic_store(p, ((unsigned long long)tag << 32) | __float_as_uint(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ unsigned long long hand_get(const gu64 *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// bounded wait of a whole wave for the words of the lanes that need one
+struct HandWait {
+    gi32 *error;
+    unsigned long long deadline;
+    bool dead;
+    __device__ __forceinline__ void wait(const gu64 *p, bool need, unsigned tag, unsigned long long &w) {
+        for (int spins = 0; __any(need && (unsigned)(w >> 32) != tag) && !dead; ++spins) {
+            if (wall_clock64() > deadline || spins > (1 << 22)) {
+                store_agent(error, 1);
+                dead = true;
+                break;
+            }
+            __builtin_amdgcn_s_sleep(1);
+            if (need) w = hand_get(p);
+        }
+    }
+};
+
+// LDS positions as byte offsets from the workgroup's dynamic LDS, and columns of
+// a field as a uniform byte address plus a 32-bit lane offset: with the offset
+// opaque to the compiler at every use the access takes the scalar-base form,
+// otherwise it widens the offset once and adds 64-bit addresses per access.
+__device__ __forceinline__ float &lds_at(float *sm, int byte_off) { return *(float *)((char *)sm + byte_off); }
+typedef const char __attribute__((address_space(1))) gc8;
+__device__ __forceinline__ const gf32 *lane_at(const gf32 *base, unsigned byte_off) {
+    asm volatile("" : "+v"(byte_off));
+    return (const gf32 *)((gc8 *)base + byte_off);
+}
+
+// Metadata of a sweep position as the strips' rows keep it (uniform); a column
+// outside the sub-domains or the sweep has VI = -1.
+struct StripCol { int KK, VI, ks, kend, veg; };   // ks: KSTART, kend: first level the sweep updates
+template <int COMP>
+__device__ __forceinline__ StripCol strip_col(int4 m) {
+    StripCol c;
+    c.KK = m.x;
+    c.VI = (m.z & 0x10000) ? m.y : -1;
+    c.ks = m.z & 0xffff;
+    // U and V skip the levels inside the building or its upstream neighbour; W
+    // updates every level from KSTART
+    c.kend = (COMP == 2) ? c.ks : (COMP == 0) ? (m.w & 0xffff) + 1 : ((m.w >> 16) & 0xffff) + 1;
+    c.veg = m.z & 0x20000;
+    return c;
+}
+
+// Raw operands of one column, as loaded one step before they are worked up:
+// records, own and old neighbour values, the -IS / -JS neighbours' values as
+// memory holds them (used where this sweep does not update them) and, for row 0
+// of a strip, the hand-off words of the previous strip's last row.
+struct MlRaw {
+    float4 v0, v2, v3;
+    float3 v1;
+    float x, xa, xb, ni, nj;
+    unsigned long long hw;
+};
+// What a column's assembly needs beside the two new neighbour values
+struct MlIn {
+    float ai, aj, pa, pb;      // coefficients of the new neighbours, products of the old ones
+    float ao, xo;              // coefficient and value of the old i neighbour (512-bit solvers fuse their product)
+    float e, f, g, w, x, dd, eo, y1, y2, y3, y4, c0, t;
+    double t5, fd, gd;
+    float ni, nj;
+    int li, lj;                // LDS positions of the new neighbours' values
+    bool si, sj, cross;        // they hold this level; the cross terms apply
+};
+
+// One strip of a momentum sweep.  R row waves own a sweep row each, the chain
+// wave runs the recurrences of all rows (lane = row), the control wave prepares
+// the chain wave's column data and hands the last row's results to the next
+// strip.  A local step s has two phases between barriers:
+//   1. every row reads the two new neighbour values of its column (a = oa+s-r)
+//      from LDS and finishes the source term D; everything else in D was worked
+//      up before;
+//   2. the chain wave runs the forward recurrence and the back-substitution,
+//      while the rows work up the column of step s+1 (loaded a whole step
+//      before: coefficients to LDS, products of the old neighbours and the
+//      cross terms' fixed parts to registers), issue the loads of step s+2 and
+//      store the column of step s-1.
+// Bound by the recurrences (40 levels: about 31 + 46 cycles per level) plus phase
+// 1.  M: 64-level groups a column of this sweep can span.  WFIX: the solver
+// width when every situation of the launch has it, else 0.
+// KIND 0: mixing length; KIND 1: k-eps, KIND 2: no diffusion (sources by
+// ke_source's arithmetic, the TDMA divides by the denominators k_ml_coef stored).
+template <int COMP, int WFIX, int KIND, int M>
+__global__ __launch_bounds__(STRIP_WAVES * WAVE) void k_ml_strip(const Dom *__restrict__ ds, int IS, int JS) {
+    const DomG &d = reinterpret_cast<const DomG *>(ds)[blockIdx.z];                   // situation of this launch slice
+    extern __shared__ __align__(16) float sm[];
+    // the fields the steps use, read once: a scalar load inside a step would
+    // wait for its latency and, sharing its counter, for the LDS accesses
+    const int nkp = d.nkp, nii = d.nii, njj = d.njj, nj2 = d.nj2, hcols = d.hand_cols;
+    const int low = strip_low((COMP == 2) ? d.nlow : 0), len = strip_len((COMP == 2) ? d.nlow : 0, d.nact);
+    const int rs = strip_stride(9, len);
+    const int oa = (COMP == 0) ? 3 : 2, ia = (COMP == 1) ? 3 : 2, ob = nii - 1, ib = njj - 1, na = ob - oa + 1;
+    const int R = blockDim.x / WAVE - 2;                      // rows of a strip (strip_rows())
+    const int nstrip = (ib - ia + R) / R, nsteps = na + R - 1;
     const int r = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
-    const bool chainw = r == ROWS;                            // the chain wave owns no row
-    gi32 *sync = d.sync + SYNC_BLOCK0;
-    // per row: D, Q, T, P and the recurrence output N (the new DPM) of even and
-    // odd steps (a row stores its previous column while the next one is solved)
-    float *sD = sm + (size_t)r * 6 * nkl + SLOT_PAD, *sQ = sD + nkl, *sT = sQ + nkl, *sP = sT + nkl, *sN0 = sP + nkl;
-    float *xbuf = sm + (size_t)ROWS * 6 * nkl + SLOT_PAD;      // [2][ROWS] slots of whole DPM columns (old values)
-    float *ring = sm + (size_t)ROWS * 8 * nkl + SLOT_PAD;      // [RING] QIMP row scratch slots
-    float *sdzk = sm + (size_t)(ROWS * 8 + RING) * nkl, *satp = sdzk + nkp;
-    int *sinfo = (int *)(satp + nkp);                         // [2][ROWS] per row: active, KK, VI, ring slot
-    int *sctl = sinfo + 8 * ROWS;
-    float *sdump = (float *)(sctl + 4);                       // [WAVE][CH] sinks of the chains
+    gi32 *sync = d.sync + SYNC_BLOCK0 + (size_t)(1 + COMP) * d.sync_stride;
+    // per row: D (replaced by Q), then per step parity C, T, P and X (the old
+    // column, replaced by the new one)
+    float *sdzk = sm + (size_t)R * rs, *sap0 = sdzk + nkp;         // [nkp] each
+    int4 *sinfo = (int4 *)(sap0 + nkp);                       // [2][16] per row by step parity, for the chain wave
+    int *sctl = (int *)(sinfo + 32);
     if (threadIdx.x == 0) sctl[0] = __hip_atomic_fetch_add(&sync[0], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    for (int k = threadIdx.x; k < nkp; k += STRIP_WAVES * WAVE) { sdzk[k] = d.dzk[k]; satp[k] = d.atp[k]; }
+    for (int k = threadIdx.x; k < nkp; k += blockDim.x) { sdzk[k] = d.dzk[k]; sap0[k] = d.ap0[k]; }
     __syncthreads();
-    const int B = sctl[0];
-    if (B >= nstrip) return;
-    if (chainw) {                                             // own loop, as in k_ml_strip
-        __builtin_amdgcn_s_setprio(3);                        // ahead of the row waves, as in k_ml_strip
-        // column data of step s published by the rows one phase early, read
-        // while they assemble (as in k_ml_strip)
-        const int cl = lane < ROWS ? lane : 0;
-        bool on = false;
-        int KK2 = 0, VI2 = 0, rs2 = 0, nmax = 0;
-        auto info = [&](int s) {
-            const int *si = sinfo + (s & 1) * 4 * ROWS;
-            on = lane < ROWS && si[cl * 4];
-            KK2 = si[cl * 4 + 1]; VI2 = si[cl * 4 + 2]; rs2 = si[cl * 4 + 3];
-            nmax = wave_max(VI2 - KK2, on);
-        };
+    const int B = __builtin_amdgcn_readfirstlane(sctl[0]);
+    if (B >= nstrip) return;                                  // uniform over the workgroup
+    const unsigned tag = hand_tag(d, 1 + COMP);
+    gu64 *hand = (gu64 *)d.hand;                              // [strip][hand_cols][nkp] words
+    const int4 *meta = (const int4 *)d.meta;
+    // The chain and the control wave run loops of their own with the same
+    // barriers per step as the row waves (s_barrier counts waves, wherever they
+    // are in the code), so none of the row waves' registers is live in the
+    // recurrences.  They issue ahead of the row waves on their SIMDs (wave
+    // priority): the recurrences are the step's serial path.
+    if (r == R) {
+        __builtin_amdgcn_s_setprio(3);
+        const float relax = d.relax;
+        float *L = sm + (size_t)(lane < R ? lane : 0) * rs + low;
+        lds_barrier();                                        // the control wave's data of step 0
         for (int s = 0; s < nsteps; ++s) {
+            // lane's levels (0: no column), the longest chains in chunks
+            const int4 si = sinfo[(s & 1) * 16 + (lane & 15)];
+            const int n = lane < R ? si.x : 0;
+            const int fmax = __builtin_amdgcn_readfirstlane(si.y), bmax = __builtin_amdgcn_readfirstlane(si.z);
+            const bool part = __builtin_amdgcn_readfirstlane(si.w) != 0;
             lds_barrier();                                    // the rows' sources are assembled
-            if (s == 0) info(0);
-            if (on) {
-                float *Dd = sm + (size_t)cl * 6 * nkl + SLOT_PAD;
-                float *Q = Dd + nkl, *T = Q + nkl, *P = T + nkl, *N = P + nkl + (size_t)(s & 1) * nkl;
-                const float *O = xbuf + (size_t)((s & 1) * ROWS + cl) * nkl;
-                // Q[k] holds ATP[k] on entry; the new DPM goes to N
-                chain_pdown(Dd + VI2, T + VI2, Q + VI2, ring[(size_t)rs2 * nkl + VI2 + 1], VI2 - KK2, nmax, sdump + lane * CH);
-                chain_pup(P + KK2 + 1, Q + KK2 + 1, N + KK2 + 1, O[KK2], VI2 - KK2, nmax, sdump + lane * CH);
+            if (n > 0) {
+                float *Lp = L + (1 + 4 * (s & 1)) * len;
+                strip_fwd<KIND != 0>(L, Lp, Lp + len, fmax);
+                strip_back(Lp + 2 * len, L, Lp + 3 * len, relax, n, bmax, part, low);
             }
             lds_barrier();                                    // the recurrences are done
-            if (s + 1 < nsteps) info(s + 1);
         }
         return;
     }
-    const int b = ia + B * ROWS + r;
-    const bool row_ok = b <= ib;
-    StripWait sw{B > 0 ? sync + SYNC_HDR + B - 1 : nullptr, d.sync, B > 0 ? 0 : 0x7fffffff, nsteps,
-                 wall_clock64() + STRIP_TIMEOUT_TICKS};
-    gi32 *mine = sync + SYNC_HDR + B;
-    const float DXK = d.dxk, DYK = d.dyk;
-    float rmax = 0.0f;
-    PrPre pre[2];
-    float xfull[2], qfull[2];
-    int in_ = 0, jn_ = 0, KKn = 0, VIn = 0;
-    bool inr_n = false, actn = false;
-    auto meta_at = [&](int s) {
-        int l = s - r, i, j;
-        if (row_ok && l >= 0 && oa + l <= ob) {
-            sweep_to_ij(d, 1, oa + l, b, IS, JS, i, j);
-            return ldc4i(d.meta + c2(d, i, j));
-        }
-        return make_int4(0, -1, 0, 0);
-    };
-    int4 mq = meta_at(0);
-    auto locate = [&](int s) {
-        int l = s - r;                                        // sweep row a = oa + l
-        inr_n = row_ok && l >= 0 && oa + l <= ob;
-        actn = false;
-        const int4 m4 = mq;
-        mq = meta_at(s + 1);
-        if (inr_n) {
-            sweep_to_ij(d, 1, oa + l, b, IS, JS, in_, jn_);
-            Meta m = unpack_meta(m4);
-            actn = m.adv;
-            KKn = m.KK; VIn = m.VI;
-            const size_t o = c3(d, in_, jn_);
-#pragma unroll
-            for (int m2 = 0; m2 < 2; ++m2) {
-                int k = lane + WAVE * m2;
-                if (k < nkp) xfull[m2] = d.dpm[o + k];
-            }
-        }
-        if (actn) {
-            size_t o = c3(d, in_, jn_);
-#pragma unroll
-            for (int m2 = 0; m2 < 2; ++m2) {
-                int k = KKn + 1 + lane + WAVE * m2;
-                if (k <= VIn) {
-                    pre[m2].div = d.div[o + k];
-                    pre[m2].t = ttab[o + k];
-                    pre[m2].p = ptab[o + k];
-                    pre[m2].pa = d.dpm[c3(d, in_ + IS, jn_) + k];
-                    pre[m2].pb = d.dpm[c3(d, in_, jn_ + JS) + k];
-                    pre[m2].dn = d.dpmnew[o + k];
-                    if (l == 0) pre[m2].nj = d.dpm[c3(d, in_, jn_ - JS) + k];
-                }
-            }
-        }
-    };
-    // row 0 reads the previous strip's last row (-IS neighbours) and the row
-    // scratch as that strip left it: after its other look-ahead loads and its wait
-    auto locate_prev = [&]() {
-        if (inr_n) {
-#pragma unroll
-            for (int m2 = 0; m2 < 2; ++m2) {
-                int k = lane + WAVE * m2;
-                if (k < nkp) qfull[m2] = ld_handoff(d.prow_q + (size_t)jn_ * nkp + k);
-            }
-        }
-        if (actn) {
-            size_t o = c3(d, in_ - IS, jn_);
-#pragma unroll
-            for (int m2 = 0; m2 < 2; ++m2) {
-                int k = KKn + 1 + lane + WAVE * m2;
-                if (k <= VIn) pre[m2].ni = ld_handoff(d.dpm + o + k);
-            }
-        }
-    };
-    // the chain wave's data of the column located for step s (one lane writes)
-    auto put_info = [&](int s) {
-        if (lane == 0) {
-            int *si = sinfo + (s & 1) * 4 * ROWS;
-            si[r * 4] = actn;
-            if (actn) { si[r * 4 + 1] = KKn; si[r * 4 + 2] = VIn; si[r * 4 + 3] = (s - r) & (RING - 1); }
-        }
-    };
-    locate(0);
-    put_info(0);
-    if (r == 0) {
-        sw.wait(ROWS);
-        locate_prev();
-    }
-    // The results of a step are merged on use, as in k_ml_strip: level k of a
-    // row's previous column is the new DPM (N of that step's parity) in
-    // KK+1..VI, else the old value.  Each row finishes its previous column in
-    // the next step: the row scratch update before the new sources replace sQ;
-    // then, after issuing the look-ahead loads of the second phase (whose waits
-    // would otherwise include these stores, as in k_ml_strip), the last row's
-    // hand-off of the row scratch to strip B+1, the residual and the DPM/DPMNEW
-    // stores (DPMNEW prefetched one step ahead).  The stores of step s-1 are
-    // issued in step s, so the progress a strip publishes in step s is s-1.
-    int pkk = 0, pvi = -1, prs = 0, pj = 0;                  // own previous column (pvi < 0: none)
-    bool pinr = false;
-    size_t po = 0;
-    float dnp[2] = {0.0f, 0.0f};
-    auto finish_ring = [&]() {
-        float *qring = ring + (size_t)prs * nkl;
-        for (int k = pkk + 1 + lane; k <= pvi; k += WAVE) qring[k] = sQ[k];
-    };
-    auto hand_off = [&]() {
-        if (r == ROWS - 1 && pinr) {                          // hand the row scratch to strip B+1
-            const float *qring = ring + (size_t)prs * nkl;
-            gf32 *qrow = d.prow_q + (size_t)pj * nkp;
-            for (int k = lane; k < nkp; k += WAVE) st_through(qrow + k, qring[k]);
-        }
-    };
-    auto finish_store = [&](const float *xold, const float *sN) {
-#pragma unroll
-        for (int m = 0; m < 2; ++m) {
-            int k = pkk + 1 + lane + WAVE * m;
-            if (k <= pvi) {
-                float temp = sN[k];
-                double qv = (double)conv_to_int((double)temp * d.frund) / d.frund;
-                float rr = (float)fabs((double)xold[k] - qv);
-                rmax = rr > rmax ? rr : rmax;
-                st_through(d.dpm + po + k, temp);
-                st_through(d.dpmnew + po + k, dnp[m] + d.relaxp * temp);
-            }
-        }
-    };
-    for (int s = 0; s < nsteps; ++s) {
-        const bool act = actn, inr = inr_n;
-        const int i = in_, j = jn_, KK = KKn, VI = VIn;
-        const int rs = (s - r) & (RING - 1);                  // ring slot of this wave's sweep row
-        float *xcur = xbuf + (size_t)((s & 1) * ROWS + r) * nkl;
-        const float *xw_lds = xbuf + (size_t)(((s - 1) & 1) * ROWS + r) * nkl;
-        const float *xs_lds = xbuf + (size_t)(((s - 1) & 1) * ROWS + r - 1) * nkl;
-        const float *snprev = sN0 + (size_t)((s - 1) & 1) * nkl;  // new DPM of the previous step
-        const float *xs_new = snprev - (size_t)6 * nkl;      // row r-1's
-        const int *sp = sinfo + ((s - 1) & 1) * 4 * ROWS;
-        const bool w_in = (s - r >= 1), s_in = (r >= 1);
-        finish_ring();
-        if (inr) {
-#pragma unroll
-            for (int m = 0; m < 2; ++m) {
-                int k = lane + WAVE * m;
-                if (k < nkp) {
-                    xcur[k] = xfull[m];
-                    if (r == 0) ring[(size_t)rs * nkl + k] = qfull[m];
-                }
-            }
-        }
-        if (act) {
-            // updated levels of the neighbouring row's column (row r-1, previous step)
-            int slo = 1 << 30, shi = -1;
-            if (s_in && sp[(r - 1) * 4]) {
-                slo = sp[(r - 1) * 4 + 1] + 1;
-                shi = sp[(r - 1) * 4 + 2];
-            }
-#pragma unroll
-            for (int m = 0; m < 2; ++m) {
-                int k = KK + 1 + lane + WAVE * m;
-                if (k <= VI) {
-                    const PrPre &r_ = pre[m];
-                    float newj = w_in ? ((k > pkk && k <= pvi) ? snprev[k] : xw_lds[k]) : r_.nj;
-                    float newi = s_in ? ((k >= slo && k <= shi) ? xs_new[k] : xs_lds[k]) : r_.ni;
-                    float dim_ = (IS == 1) ? newi : r_.pa, dip = (IS == 1) ? r_.pa : newi;
-                    float djm = (JS == 1) ? newj : r_.pb, djp = (JS == 1) ? r_.pb : newj;
-                    float dz = sdzk[k];
-                    sD[k] = r_.div + (dim_ + dip) / DXK * DYK * dz + (djm - djp) / DYK * DXK * dz;
-                    sT[k] = r_.t;
-                    sP[k] = r_.p;
-                    sQ[k] = satp[k];                  // consumed and replaced by QIMP in phase 2
-                }
-            }
-        }
-        const float dn0 = pre[0].dn, dn1 = pre[1].dn;         // this column's DPMNEW, before the look-ahead
+    if (r == R + 1) {
+        __builtin_amdgcn_s_setprio(2);
+        // lane r's column at step s is a = oa + s - r of row b; its metadata is
+        // requested a step ahead
+        const int b = ia + B * R + lane;
+        const bool lane_ok = lane < R && b <= ib;
+        int cidx = ((IS == -1) ? nii - oa + 1 : oa) * nj2 + ((JS == -1) ? njj - b + 1 : b) - lane * IS * nj2;
+        auto meta_at = [&](int s) {
+            const int l = s - lane;
+            int4 m = make_int4(0, -1, 0, 0);
+            if (lane_ok && l >= 0 && l < na) m = ldg4i((const DomG::P<const int4>)meta + cidx);
+            cidx += IS * nj2;
+            return m;
+        };
+        int4 mq = meta_at(0);
+        StripCol c{0, -1, 0, 0, 0};                           // the column of step s
+        auto info = [&](int s) {                              // ... of step s, into LDS
+            const StripCol cn = strip_col<COMP>(mq);
+            mq = meta_at(s + 1);
+            const int n = cn.VI < 0 ? 0 : cn.VI - cn.KK;
+            const int nb = n > 0 ? ((n - 1) >> 3) - ((cn.kend - cn.KK - 1) >> 3) + 1 : 0;
+            const int part = __any((n & (CHK - 1)) != 0);
+            const int fm = row_max((n + CHK - 1) >> 3), bm = row_max(nb);
+            if (lane < 16) sinfo[(s & 1) * 16 + lane] = make_int4(n, fm, bm, part);
+            return cn;
+        };
+        const bool send = B + 1 < nstrip;
+        gu64 *h = hand + ((size_t)B * hcols - (R - 1)) * nkp; // the last row's column at step s: + s*nkp
+        c = info(0);
         lds_barrier();
-        // while the chain wave runs the recurrences: publish and prefetch as in
-        // k_ml_strip; row 0 reads the previous strip's row scratch and last row
-        // after its wait; then the previous column's stores
-        if (r == ROWS - 1 && s > 1 && (s - 1) % STRIP_PUBLISH == 0) strip_publish(mine, s - 1, lane);
-        locate(s + 1);
-        if (s + 1 < nsteps) put_info(s + 1);
-        if (r == 0) {
-            sw.wait(s + 1 + ROWS);
-            locate_prev();
+        for (int s = 0; s < nsteps; ++s) {
+            lds_barrier();
+            const StripCol cn = info(s + 1);
+            lds_barrier();                                    // the recurrences are done
+            const int vil = __builtin_amdgcn_readlane(c.VI, R - 1);
+            if (send && vil >= 0) {
+                // the last row's results, the only column another strip reads, go
+                // out while the rows assemble the next step
+                const int kel = __builtin_amdgcn_readlane(c.kend, R - 1), kkl = __builtin_amdgcn_readlane(c.KK, R - 1);
+                const float *xn = sm + (size_t)(R - 1) * rs + (4 + 4 * (s & 1)) * len + low - (kkl + 1);
+                for (int k = kel + lane; k <= vil; k += WAVE) hand_put(h + (size_t)s * nkp + k, xn[k], tag);
+            }
+            c = cn;
         }
-        hand_off();
-        finish_store(xw_lds, snprev);
-        pkk = KK; pvi = act ? VI : -1; prs = rs; pj = j; pinr = inr; po = c3(d, i, j);
-        dnp[0] = dn0; dnp[1] = dn1;
+        return;
+    }
+    const int b = ia + B * R + r;
+    const bool row_ok = b <= ib, from_prev = r == 0 && B > 0;
+    const bool ip = IS == 1, jp = JS == 1, v512 = KIND == 0 && (WFIX ? WFIX : d.simd) == 16;
+    const int wlev = v512 ? 16 : 8;                           // levels of a vector block
+    HandWait hwait{d.sync, wall_clock64() + STRIP_TIMEOUT_TICKS, false};
+    // neighbour levels the sweep updates: the same row's previous column always
+    // lies in the sweep, the previous row's only if there is one
+    const bool has_j = r > 0 || B > 0;
+    const float ddf = (COMP == 0) ? d.dyk : d.dxk;
+    const int rowb = 4 * r * rs;                              // the row's LDS, in bytes
+    const gf32 *X = (COMP == 0 ? d.uk : COMP == 1 ? d.vk : d.wk), *planes = d.planes, *rec3 = d.rec3, *wcol = d.wcol;
+    // the row's column at l = s - r: column index cidx, one sweep step apart dcol
+    const int dcol = IS * nj2;
+    int l2 = -r;                                              // l of the step whose metadata is requested
+    int cidx2 = ((IS == -1) ? nii - oa + 1 : oa) * nj2 + ((JS == -1) ? njj - b + 1 : b) - r * dcol;
+    int4 m2, m2j;                                             // requested a step before their use
+    auto request = [&]() {                                    // metadata of the next column and its -JS neighbour
+        m2 = m2j = make_int4(0, -1, 0, 0);
+        if (row_ok && l2 >= 0 && l2 < na) {
+            m2 = ldc4i(meta + cidx2);
+            if (has_j) m2j = ldc4i(meta + (cidx2 - JS));
+        }
+        ++l2;
+        cidx2 += dcol;
+    };
+    // byte offsets of a lane in the columns it loads, from the lowest of them
+    const unsigned fi = 4u * (unsigned)nj2 * (unsigned)nkp, fj = 4u * (unsigned)nkp, base = fi + fj;
+    const unsigned off_c = base + 4u * lane, off_a = ip ? off_c + fi : off_c - fi, off_b = jp ? off_c + fj : off_c - fj;
+    const unsigned off_i = ip ? off_c - fi : off_c + fi, off_j = jp ? off_c - fj : off_c + fj;
+    const unsigned off_p = (unsigned)(4 * rec_floats<COMP>()) * lane, off_r = 12u * lane, off_h = 8u * lane;
+    const StripCol none{0, -1, 0, 0, 0};
+    StripCol c0 = none, c1 = none, c1j = none, c2m = none;    // columns of step s, s+1 (and its -JS neighbour), s-1
+    unsigned o0 = 0, o1 = 0, op = 0;                          // their first cells
+    MlRaw raw[M];
+    MlIn in[M];
+    float wraw = 0.0f;
+    // requests the operands of the row's next column; p: the one before it
+    auto issue = [&](const StripCol &p, const StripCol &cn, const StripCol &cnj) {
+        c1 = cn;
+        c1j = cnj;
+        const int ci = cidx2 - 2 * dcol, l = l2 - 2;          // request() is one column ahead
+        if (c1.VI < 0) return;
+        o1 = (unsigned)ci * (unsigned)nkp;
+        const int kb = (COMP == 2) ? c1.ks : c1.KK + 1;       // first level with a source
+        const size_t o = (size_t)o1 + kb;
+        const gf32 *Pc = planes + o * rec_floats<COMP>(), *R3 = rec3 + o * 3;
+        const gf32 *Xl = X + o - (base >> 2);
+        const gf32 *H = (const gf32 *)(hand + ((size_t)(B - 1) * hcols + l) * nkp + kb);
+        const bool old_i = p.kend > kb || p.VI < c1.VI, old_j = c1j.kend > kb || c1j.VI < c1.VI;
+        const int top = c1.VI + 1 - kb;
+        if (COMP != 2) wraw = wcol[ci];
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+            if (lane + WAVE * m <= top) {
+                MlRaw &q = raw[m];
+                const gf32 *P = lane_at(Pc + m * WAVE * rec_floats<COMP>(), off_p);
+                q.v0 = ldg4(P); q.v2 = ldg4(P + 4);
+                if (COMP != 2) q.v3 = ldg4(P + 8);
+                q.v1 = ldg3(lane_at(R3 + m * WAVE * 3, off_r));
+                const gf32 *Xm = Xl + m * WAVE;
+                q.x = *lane_at(Xm, off_c);
+                q.xa = *lane_at(Xm, off_a);
+                q.xb = *lane_at(Xm, off_b);
+                if (old_i) q.ni = *lane_at(Xm, off_i);
+                if (old_j) q.nj = *lane_at(Xm, off_j);
+                if (from_prev) q.hw = hand_get((const gu64 *)lane_at(H + m * WAVE * 2, off_h));
+            }
+        }
+    };
+    // works up the operands of step s: recurrence operands to LDS, the rest to in[]
+    auto work_up = [&](int s, const StripCol &p) {
+        const StripCol &c = c1;
+        if (c.VI < 0) return;
+        const int kb = (COMP == 2) ? c.ks : c.KK + 1;
+        // LDS of level k: at(k) + 4*lane, X of this and the other parity
+        const int sc = rowb + 4 * ((1 + 4 * (s & 1)) * len + low + kb - (c.KK + 1)), l4 = 4 * len;
+        const int sx = rowb + 4 * ((8 - 4 * (s & 1)) * len + low + kb - (p.KK + 1));
+        const int sj = rowb - 4 * rs + 4 * ((8 - 4 * (s & 1)) * len + low + kb - (c1j.KK + 1));
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+            const int t4 = 4 * (lane + WAVE * m), k = kb + lane + WAVE * m;
+            MlRaw &q = raw[m];
+            MlIn &a = in[m];
+            if (k <= c.VI + 1) lds_at(sm, sc + 3 * l4 + t4) = q.x;
+            if (k <= c.VI) {
+                lds_at(sm, sc + t4) = q.v1.x;
+                lds_at(sm, sc + l4 + t4) = q.v1.y;
+                lds_at(sm, sc + 2 * l4 + t4) = q.v1.z;
+                const float aw = q.v0.x, as = q.v0.y, ae = q.v0.z, an = q.v0.w;
+                a.ai = ip ? aw : ae; a.aj = jp ? as : an;
+                a.ao = ip ? ae : aw; a.xo = q.xa;
+                a.pa = a.ao * q.xa; a.pb = (jp ? an : as) * q.xb;
+                a.e = q.v2.z; a.f = q.v2.x; a.g = q.v2.y;
+                a.x = q.x; a.t = q.v1.y;
+                bool cross = KIND != 2 && k > c.KK + 1;
+                if (KIND == 0) cross = min(c.ks + ((k - c.ks) & -wlev), c.VI + 1 - wlev) > c.KK + 1;   // block_base()
+                a.cross = cross;
+                if (COMP == 2) {
+                    a.y1 = cross ? q.v2.w : -0.0f;            // -0: adding it changes nothing
+                } else {
+                    a.c0 = q.v2.w;
+                    a.w = (lane + WAVE * m == 0) ? wraw : 0.0f;
+                    a.dd = ddf * sdzk[k];
+                    a.y1 = q.v3.x; a.y2 = q.v3.y; a.y3 = q.v3.z; a.y4 = q.v3.w;
+                    const bool fwd = (COMP == 0) ? ip : jp;   // the new value is the lower neighbour's
+                    const float xold = (COMP == 0) ? q.xa : q.xb;
+                    a.eo = (fwd ? xold - q.x : q.x - xold) * a.dd;
+                    if (COMP == 1) {
+                        a.y1 = a.y1 - a.y2;
+                        if (fwd) a.y1 = a.y1 + a.eo;
+                    }
+                    if (COMP == 0 && v512 && !c.veg) a.g = -0.0f;
+                }
+                if (KIND != 0) {
+                    a.t5 = (double)sap0[k] * 0.5 * (double)a.e;
+                    a.fd = (double)a.f; a.gd = (double)a.g;
+                }
+                a.ni = q.ni; a.nj = q.nj;
+                a.si = k >= p.kend && k <= p.VI;
+                a.sj = k >= c1j.kend && k <= c1j.VI;
+                // a safe position where the neighbour does not hold the level
+                a.li = a.si ? sx + t4 : 0;
+                a.lj = a.sj ? sj + t4 : 0;
+            }
+        }
+        if (from_prev) {
+            const gu64 *h = hand + ((size_t)(B - 1) * hcols + (s - r)) * nkp;
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+                const int k = kb + lane + WAVE * m;
+                const bool need = k <= c.VI && k >= c1j.kend && k <= c1j.VI;
+                hwait.wait(h + k, need, tag, raw[m].hw);
+                if (need) in[m].nj = __uint_as_float((unsigned)raw[m].hw);
+                in[m].sj = false;                             // the value is in nj
+                in[m].lj = 0;
+            }
+        }
+    };
+    StripCol c2, c2j;                                         // column of step s+2
+    auto located = [&]() {
+        c2 = strip_col<COMP>(m2);
+        c2j = strip_col<COMP>(m2j);
+        request();
+    };
+    request();
+    located();
+    issue(none, c2, c2j);
+    located();
+    work_up(0, none);
+    c0 = c1; o0 = o1;
+    issue(c0, c2, c2j);
+    lds_barrier();                                            // the control wave's data of step 0
+    for (int s = 0; s < nsteps; ++s) {
+        // phase 1: the new neighbours enter the source terms of step s
+        if (c0.VI >= 0) {
+            const int kb = (COMP == 2) ? c0.ks : c0.KK + 1;
+            const int sd = rowb + 4 * (low + kb - (c0.KK + 1));
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+                const int k = kb + lane + WAVE * m;
+                if (k <= c0.VI) {
+                    const MlIn &a = in[m];
+                    float vi = lds_at(sm, a.li), vj = lds_at(sm, a.lj);
+                    vi = a.si ? vi : a.ni;
+                    vj = a.sj ? vj : a.nj;
+                    const float mi = a.ai * vi, mj = a.aj * vj;
+                    float D;
+                    if (v512 && (COMP != 1 || c0.veg)) {
+                        // FMA(AW, X_W, AS*X_S) + FMA(AE, X_E, AN*X_N)
+                        const float ts = jp ? mj : a.pb, tn = jp ? a.pb : mj;
+                        const float xw = ip ? vi : a.xo, xe = ip ? a.xo : vi, aw = ip ? a.ai : a.ao, ae = ip ? a.ao : a.ai;
+                        D = fmaf(aw, xw, ts) + fmaf(ae, xe, tn);
+                    } else {                                  // AW*X_W + AS*X_S + AE*X_E + AN*X_N; selects, no branches
+                        D = (ip ? mi : a.pa) + (jp ? mj : a.pb) + (ip ? a.pa : mi) + (jp ? a.pb : mj);
+                    }
+                    if (KIND != 0) {
+                        if (COMP == 2) D = (float)((double)D + a.t5 + a.fd);
+                        else D = (float)((double)D + a.t5 + a.fd + a.gd);
+                    } else {
+                        D = D + a.e + a.f;
+                        D = (COMP == 2) ? D - a.g : D + a.g;
+                    }
+                    if (COMP != 2) {
+                        D -= a.w;
+                        if (KIND != 2) {
+                            float z;
+                            if (COMP == 0) {
+                                const float en = (ip ? a.x - vi : vi - a.x) * a.dd;
+                                z = (ip ? a.eo - en : en - a.eo) + a.y1 - a.y2 + a.y3 - a.y4;
+                            } else {
+                                const float en = (jp ? a.x - vj : vj - a.x) * a.dd;
+                                z = (jp ? a.y1 - en : a.y1 + en - a.eo) + a.y3 - a.y4;
+                            }
+                            D += a.cross ? a.c0 * z : -0.0f;
+                        }
+                    } else if (KIND != 2) {
+                        D += a.y1;
+                    }
+                    // below KKART+1 (W inside buildings) Q is D over the diagonal;
+                    // the chain forms the one at KKART+1 itself
+                    if (COMP == 2 && k <= c0.KK) D = (KIND != 0) ? D / a.t : D * a.t;
+                    lds_at(sm, sd + 4 * (lane + WAVE * m)) = D;
+                }
+            }
+        }
+        lds_barrier();
+        // phase 2, beside the recurrences
+        float xst[M];
+        const StripCol done = c2m;                            // the column of step s-1, before its buffer is reused
+        const unsigned od = op;
+        if (done.VI >= 0) {
+            const int sn = rowb + 4 * ((8 - 4 * (s & 1)) * len + low + done.kend - (done.KK + 1) + lane);
+#pragma unroll
+            for (int m = 0; m < M; ++m)
+                if (done.kend + lane + WAVE * m <= done.VI) xst[m] = lds_at(sm, sn + 4 * WAVE * m);
+        }
+        located();                                            // ahead of the work: the barrier waits for scalar loads
+        if (s + 1 < nsteps) work_up(s + 1, c0);
+        c2m = c0; op = o0;
+        c0 = c1; o0 = o1;
+        if (s + 1 < nsteps) issue(c0, c2, c2j);
+        else c0 = none;
+        if (done.VI >= 0) {
+            gf32 *Xp = (gf32 *)X + (size_t)od + done.kend;
+#pragma unroll
+            for (int m = 0; m < M; ++m)
+                if (done.kend + lane + WAVE * m <= done.VI) *(gf32 *)lane_at(Xp + WAVE * m, off_c - base) = xst[m];
+        }
         lds_barrier();                                        // the recurrence outputs are ready
     }
-    finish_ring();
-    hand_off();
-    finish_store(xbuf + (size_t)(((nsteps - 1) & 1) * ROWS + r) * nkl, sN0 + (size_t)((nsteps - 1) & 1) * nkl);
-    if (r == ROWS - 1) strip_publish(mine, nsteps, lane);
+    if (c2m.VI >= 0) {
+        const float *xn = sm + (size_t)r * rs + (4 + 4 * ((nsteps - 1) & 1)) * len + low - (c2m.KK + 1);
+        gf32 *Xp = (gf32 *)X + (size_t)op;
+        for (int k = c2m.kend + lane; k <= c2m.VI; k += WAVE) Xp[(unsigned)k] = xn[k];
+    }
+}
+
+// Pressure sweep on strips (a = j1 outer, b = i1 inner), laid out as
+// k_ml_strip.  The QIMP row scratch of a sweep row, which every column of the
+// row starts its elimination from and leaves its values in, travels with the
+// wavefront through LDS (ring slot (a - oa) mod RING; the rows of a step
+// hold consecutive sweep rows): the control wave puts the row the previous strip
+// handed over into row 0's slot, each row merges its column's Q, and the control
+// wave hands the row on after the last row's merge.
+// Chains per column: Q[t] = (A[t]*Q[t+1] + D[t])*T[t] from the top (A = ATP; 3
+// dependent operations a level), then N[t] = P[t]*N[t-1] + Q[t] from the bottom (2).
+#define RING 16
+__device__ __forceinline__ void strip_pdown(float *DQ, const float *A, const float *T, float qtop, int n, int nch, bool part,
+                                            int low) {
+    int o = (n - 1) & ~(CHK - 1);
+    const int top = n - o;
+    float qn = qtop;
+    Chunk d[2], a[2], t[2];
+    d[0] = ld_chunk(DQ + o); a[0] = ld_chunk(A + o); t[0] = ld_chunk(T + o);
+    for (int b = 0; b < nch; b += CHK_BLOCK) {
+#pragma unroll
+        for (int h = 0; h < CHK_BLOCK; ++h) {
+            if (b + h >= nch) return;
+            const int k = h & 1, m = k ^ 1, on = max(o - CHK, -low);
+            d[m] = ld_chunk(DQ + on); a[m] = ld_chunk(A + on); t[m] = ld_chunk(T + on);
+            __builtin_amdgcn_sched_barrier(0);
+            if (h == 0 && part && b == 0) {
+#pragma unroll
+                for (int u = CHK - 1; u >= 0; --u) {
+                    const float q = (a[k].v[u] * qn + d[k].v[u]) * t[k].v[u];
+                    qn = (u >= top) ? qn : q;
+                    d[k].v[u] = q;
+                }
+            } else {
+#pragma unroll
+                for (int u = CHK - 1; u >= 0; --u) {
+                    qn = (a[k].v[u] * qn + d[k].v[u]) * t[k].v[u];
+                    d[k].v[u] = qn;
+                }
+            }
+            st_chunk(DQ + o, d[k]);
+            o = on;
+        }
+    }
+}
+__device__ __forceinline__ void strip_pup(const float *P, const float *Q, float *N, float bottom, int nch) {
+    float x = bottom;
+    Chunk p[2], q[2];
+    p[0] = ld_chunk(P); q[0] = ld_chunk(Q);
+    for (int b = 0; b < nch; b += CHK_BLOCK) {
+#pragma unroll
+        for (int h = 0; h < CHK_BLOCK; ++h) {
+            if (b + h >= nch) return;
+            const int k = h & 1, m = k ^ 1;
+            p[m] = ld_chunk(P + (h + 1) * CHK); q[m] = ld_chunk(Q + (h + 1) * CHK);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < CHK; ++u) {
+                x = p[k].v[u] * x + q[k].v[u];
+                q[k].v[u] = x;
+            }
+            st_chunk(N + h * CHK, q[k]);
+        }
+        P += CHK_BLOCK * CHK; Q += CHK_BLOCK * CHK; N += CHK_BLOCK * CHK;
+    }
+}
+
+// raw operands of one column, loaded a step before they are worked up
+struct PrRaw {
+    float div, t, p, pa, pb;       // DIV / DTIME, TERMP, PIMP, old DPM in the +IS (i) and +JS (j) directions
+    float ni, nj;                  // -IS / -JS neighbours as memory holds them
+    unsigned long long hw;
+};
+struct PrIn {
+    float div, pa, pb, dz, ni, nj;
+    int li, lj;
+    bool si, sj;
+};
+
+template <int M>
+__global__ __launch_bounds__(STRIP_WAVES * WAVE) void k_pressure_strip(const Dom *__restrict__ ds, int IS, int JS, int slot) {
+    const DomG &d = reinterpret_cast<const DomG *>(ds)[blockIdx.z];
+    extern __shared__ __align__(16) float sm[];
+    const int nkp = d.nkp, nii = d.nii, njj = d.njj, nj2 = d.nj2, hcols = d.hand_cols;
+    const int low = strip_low(0), len = strip_len(0, d.nact), rs = strip_stride(9, len);
+    const int oa = 2, ia = 2, ob = njj - 1, ib = nii - 1, na = ob - oa + 1;
+    const int R = blockDim.x / WAVE - 2;                      // rows of a strip (strip_rows())
+    const int nstrip = (ib - ia + R) / R, nsteps = na + R - 1;
+    const int r = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
+    gi32 *sync = d.sync + SYNC_BLOCK0;
+    // per row: D (replaced by Q), then per step parity A, T, P and the new DPM
+    float *ring = sm + (size_t)R * rs;                        // [RING][nkp] QIMP row scratch
+    float *sdzk = ring + RING * nkp, *satp = sdzk + nkp;      // [nkp] each
+    int4 *sinfo = (int4 *)(satp + nkp);                       // [2][16] per row by step parity, for the chain wave
+    int *sctl = (int *)(sinfo + 32);
+    if (threadIdx.x == 0) sctl[0] = __hip_atomic_fetch_add(&sync[0], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int k = threadIdx.x; k < nkp; k += blockDim.x) { sdzk[k] = d.dzk[k]; satp[k] = d.atp[k]; }
+    __syncthreads();
+    const int B = __builtin_amdgcn_readfirstlane(sctl[0]);
+    if (B >= nstrip) return;                                  // uniform over the workgroup
+    const unsigned tag = hand_tag(d, 0);
+    gu64 *hand = (gu64 *)d.hand, *handq = hand + d.hand_words;        // new DPM, row scratch: [strip][hand_cols][nkp]
+    const int4 *meta = (const int4 *)d.meta;
+    HandWait hwait{d.sync, wall_clock64() + STRIP_TIMEOUT_TICKS, false};
+    const bool send = B + 1 < nstrip;
+    if (r == R) {                                             // chain wave, as in k_ml_strip
+        __builtin_amdgcn_s_setprio(3);
+        float *L = sm + (size_t)(lane < R ? lane : 0) * rs + low;
+        // The last row's new values, which the next strip waits for, go out while
+        // the rows assemble the next step: this wave waits for no load, so the
+        // stores cost it their issue only.
+        const float *xl = sm + (size_t)(R - 1) * rs + 4 * len + low;
+        gu64 *h = hand + ((size_t)B * hcols - R) * nkp;       // + s*nkp: the last row's column of step s - 1
+        int n = 0, top = 0;
+        auto send_last = [&](int s) {
+            const int nl = __builtin_amdgcn_readlane(n, R - 1), kl = __builtin_amdgcn_readlane(top, R - 1) - nl;
+            if (send)
+                for (int t = lane; t < nl; t += WAVE) hand_put(h + (size_t)s * nkp + kl + t, xl[4 * ((s - 1) & 1) * len + t], tag);
+        };
+        lds_barrier();                                        // the control wave's data of step 0
+        for (int s = 0; s < nsteps; ++s) {
+            // levels (0: no column), chunks | partial chunk << 16, VI + 1, DPM below the column
+            const int4 si = sinfo[(s & 1) * 16 + (lane & 15)];
+            send_last(s);
+            n = lane < R ? si.x : 0;
+            top = si.z;
+            const int fm = __builtin_amdgcn_readfirstlane(si.y);
+            const float *rq = ring + (size_t)((s - lane) & (RING - 1)) * nkp + top;
+            lds_barrier();                                    // the rows' sources are assembled
+            if (n > 0) {
+                float *Lp = L + (1 + 4 * (s & 1)) * len;
+                strip_pdown(L, Lp, Lp + len, *rq, n, fm & 0xffff, (fm >> 16) != 0, low);
+                strip_pup(Lp + 2 * len, L, Lp + 3 * len, __int_as_float(si.w), fm & 0xffff);
+            }
+            lds_barrier();                                    // the recurrences are done
+        }
+        send_last(nsteps);
+        lds_barrier();                                        // the last columns are merged into the ring
+        return;
+    }
+    if (r == R + 1) {                                         // control wave
+        __builtin_amdgcn_s_setprio(2);
+        const int b = ia + B * R + lane;
+        const bool lane_ok = lane < R && b <= ib;
+        int cidx = ((IS == -1) ? nii - b + 1 : b) * nj2 + ((JS == -1) ? njj - oa + 1 : oa) - lane * JS;
+        // lane r's column: its metadata is requested two steps ahead, the DPM below
+        // it one step ahead
+        auto meta_at = [&](int s) {
+            const int l = s - lane;
+            int4 m = make_int4(0, -1, 0, 0);
+            if (lane_ok && l >= 0 && l < na) m = ldg4i((const DomG::P<const int4>)meta + cidx);
+            cidx += JS;
+            return m;
+        };
+        int4 mq = meta_at(0), mb = make_int4(0, -1, 0, 0);
+        float bot = 0.0f;
+        auto advance = [&](int s) {                           // metadata of step s arrives, its DPM is requested
+            const int c = cidx - JS;
+            mb = mq;
+            mq = meta_at(s + 1);
+            bot = 0.0f;
+            if (mb.z & 0x10000) bot = d.dpm[(size_t)c * nkp + mb.x];
+        };
+        auto info = [&](int s) {
+            const int n = (mb.z & 0x10000) ? mb.y - mb.x : 0;
+            const int part = __any((n & (CHK - 1)) != 0) ? 0x10000 : 0;
+            const int fm = row_max((n + CHK - 1) >> 3);
+            if (lane < 16) sinfo[(s & 1) * 16 + lane] = make_int4(n, fm | part, n > 0 ? mb.y + 1 : 0, __float_as_int(bot));
+        };
+        // row 0's row scratch, as the previous strip hands it over: the words of a
+        // step are requested a step ahead, two groups of 64 levels at once
+        unsigned long long qw[2] = {0, 0}, qn[2];
+        auto qrequest = [&](int s) {
+#pragma unroll
+            for (int m = 0; m < 2; ++m)
+                if (B > 0 && s < na && lane + WAVE * m < nkp)
+                    qw[m] = hand_get(handq + ((size_t)(B - 1) * hcols + s) * nkp + lane + WAVE * m);
+        };
+        auto qstore = [&](int s) {
+            if (s >= na) return;
+            float *rq = ring + (size_t)(s & (RING - 1)) * nkp;
+            const gu64 *hq = handq + ((size_t)(B - 1) * hcols + s) * nkp;
+#pragma unroll
+            for (int m = 0; m < 2; ++m) {
+                const int k = lane + WAVE * m;
+                if (B > 0) hwait.wait(hq + k, k < nkp, tag, qn[m]);
+                if (k < nkp) rq[k] = B > 0 ? __uint_as_float((unsigned)qn[m]) : 0.0f;
+            }
+            for (int k = lane + 2 * WAVE; k - lane < nkp; k += WAVE) {
+                unsigned long long w = 0;
+                if (B > 0) hwait.wait(hq + k, k < nkp, tag, w);
+                if (k < nkp) rq[k] = __uint_as_float((unsigned)w);
+            }
+        };
+        advance(0);
+        qrequest(0);
+        info(0);
+        qn[0] = qw[0]; qn[1] = qw[1];
+        qstore(0);
+        advance(1);
+        qrequest(1);
+        gu64 *h = handq + ((size_t)B * hcols - R) * nkp;      // + s*nkp: the last row's row scratch of step s - 1
+        auto send_ring = [&](int s) {
+            const int l = s - R;
+            if (send && l >= 0 && l < na) {
+                const float *rq = ring + (size_t)(l & (RING - 1)) * nkp;
+                for (int k = lane; k < nkp; k += WAVE) hand_put(h + (size_t)s * nkp + k, rq[k], tag);
+            }
+        };
+        lds_barrier();
+        for (int s = 0; s < nsteps; ++s) {
+            // the loads of the step before arrive and the next are issued ahead of
+            // this step's stores: a wait for a load covers the stores before it
+            info(s + 1);
+            qn[0] = qw[0]; qn[1] = qw[1];
+            advance(s + 2);
+            qrequest(s + 2);
+            lds_barrier();
+            qstore(s + 1);
+            send_ring(s);
+            lds_barrier();
+        }
+        lds_barrier();
+        send_ring(nsteps);
+        return;
+    }
+    const int b = ia + B * R + r;
+    const bool row_ok = b <= ib, from_prev = r == 0 && B > 0, has_i = r > 0 || B > 0, jp = JS == 1;
+    const float DXK = d.dxk, DYK = d.dyk, relaxp = d.relaxp;
+    // a division by a power of two is a multiplication by its reciprocal, bit for bit
+    const float rx = 1.0f / DXK, ry = 1.0f / DYK;
+    const bool p2 = (((__float_as_uint(DXK) | __float_as_uint(DYK)) & 0x7fffffu) == 0) && fabsf(log2f(DXK)) < 100.0f &&
+                    fabsf(log2f(DYK)) < 100.0f;
+    const int rowb = 4 * r * rs;
+    const gf32 *DPM = d.dpm, *DIV = d.div, *PT = d.ptab[IS == 1 ? 0 : 1], *TT = d.ttab[IS == 1 ? 0 : 1];
+    gf32 *DPMNEW = d.dpmnew;
+    int l2 = -r;
+    int cidx2 = ((IS == -1) ? nii - b + 1 : b) * nj2 + ((JS == -1) ? njj - oa + 1 : oa) - r * JS;
+    int4 m2, m2i;
+    auto request = [&]() {                                    // metadata of the next column and its -IS neighbour
+        m2 = m2i = make_int4(0, -1, 0, 0);
+        if (row_ok && l2 >= 0 && l2 < na) {
+            m2 = ldc4i(meta + cidx2);
+            if (has_i) m2i = ldc4i(meta + (cidx2 - IS * nj2));
+        }
+        ++l2;
+        cidx2 += JS;
+    };
+    const unsigned fi = 4u * (unsigned)nj2 * (unsigned)nkp, fj = 4u * (unsigned)nkp, base = fi + fj;
+    const unsigned off_l = 4u * lane, off_c = base + off_l, off_a = IS == 1 ? off_c + fi : off_c - fi;
+    const unsigned off_b = jp ? off_c + fj : off_c - fj, off_i = IS == 1 ? off_c - fi : off_c + fi;
+    const unsigned off_j = jp ? off_c - fj : off_c + fj, off_h = 8u * lane;
+    const StripCol none{0, -1, 0, 0, 0};
+    StripCol c0 = none, c1 = none, c1i = none, c2m = none, c2, c2i;   // steps s, s+1 (and its -IS neighbour), s-1, s+2
+    unsigned o0 = 0, o1 = 0, op = 0;
+    PrRaw raw[M];
+    PrIn in[M];
+    float dn[M] = {}, pmax = 0.0f, pmin = 0.0f;
+    auto located = [&]() {
+        c2 = strip_col<0>(m2);                                // kend unused
+        c2i = strip_col<0>(m2i);
+        request();
+    };
+    auto issue = [&](const StripCol &p, const StripCol &cn, const StripCol &cni) {
+        c1 = cn;
+        c1i = cni;
+        const int ci = cidx2 - 2 * JS, l = l2 - 2;
+        if (c1.VI < 0) return;
+        o1 = (unsigned)ci * (unsigned)nkp;
+        const size_t o = (size_t)o1 + c1.KK + 1;
+        const gf32 *Xl = DPM + o - (base >> 2);
+        const gf32 *H = (const gf32 *)(hand + ((size_t)(B - 1) * hcols + l) * nkp + c1.KK + 1);
+        const bool old_j = p.KK > c1.KK || p.VI < c1.VI, old_i = c1i.KK > c1.KK || c1i.VI < c1.VI;
+        const int n = c1.VI - c1.KK;
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+            if (lane + WAVE * m < n) {
+                PrRaw &q = raw[m];
+                q.div = *lane_at(DIV + o + m * WAVE, off_l);
+                q.t = *lane_at(TT + o + m * WAVE, off_l);
+                q.p = *lane_at(PT + o + m * WAVE, off_l);
+                const gf32 *Xm = Xl + m * WAVE;
+                q.pa = *lane_at(Xm, off_a);
+                q.pb = *lane_at(Xm, off_b);
+                if (old_i) q.ni = *lane_at(Xm, off_i);
+                if (old_j) q.nj = *lane_at(Xm, off_j);
+                if (from_prev) q.hw = hand_get((const gu64 *)lane_at(H + m * WAVE * 2, off_h));
+            }
+        }
+    };
+    auto work_up = [&](int s, const StripCol &p) {
+        const StripCol &c = c1;
+        if (c.VI < 0) return;
+        const int sc = rowb + 4 * ((1 + 4 * (s & 1)) * len + low), l4 = 4 * len;
+        const int sj = rowb + 4 * ((8 - 4 * (s & 1)) * len + low + c.KK - p.KK);
+        const int si = rowb - 4 * rs + 4 * ((8 - 4 * (s & 1)) * len + low + c.KK - c1i.KK);
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+            const int t4 = 4 * (lane + WAVE * m), k = c.KK + 1 + lane + WAVE * m;
+            PrRaw &q = raw[m];
+            PrIn &a = in[m];
+            if (k <= c.VI) {
+                lds_at(sm, sc + t4) = satp[k];
+                lds_at(sm, sc + l4 + t4) = q.t;
+                lds_at(sm, sc + 2 * l4 + t4) = q.p;
+                a.dz = sdzk[k];
+                a.div = q.div; a.pa = q.pa; a.pb = q.pb; a.ni = q.ni; a.nj = q.nj;
+                a.sj = k > p.KK && k <= p.VI;
+                a.si = k > c1i.KK && k <= c1i.VI;
+                a.lj = a.sj ? sj + t4 : 0;
+                a.li = a.si ? si + t4 : 0;
+            }
+        }
+        if (from_prev) {
+            const gu64 *h = hand + ((size_t)(B - 1) * hcols + (s - r)) * nkp;
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+                const int k = c.KK + 1 + lane + WAVE * m;
+                const bool need = k <= c.VI && k > c1i.KK && k <= c1i.VI;
+                hwait.wait(h + k, need, tag, raw[m].hw);
+                if (need) in[m].ni = __uint_as_float((unsigned)raw[m].hw);
+                in[m].si = false;                             // the value is in ni
+                in[m].li = 0;
+            }
+        }
+    };
+    // merges the Q of the column of step s into its ring slot
+    auto merge = [&](int s, const StripCol &c) {
+        if (c.VI < 0) return;
+        float *rq = ring + (size_t)((s - r) & (RING - 1)) * nkp + c.KK + 1;
+#pragma unroll
+        for (int m = 0; m < M; ++m)
+            if (lane + WAVE * m < c.VI - c.KK) rq[lane + WAVE * m] = lds_at(sm, rowb + 4 * (low + lane + WAVE * m));
+    };
+    request();
+    located();
+    issue(none, c2, c2i);
+    located();
+    work_up(0, none);
+    c0 = c1; o0 = o1;
+    issue(c0, c2, c2i);
+    lds_barrier();                                            // the control wave's data of step 0
+    for (int s = 0; s < nsteps; ++s) {
+        // phase 1: the previous column's Q to the ring, the sources of step s over it
+        merge(s - 1, c2m);
+        if (c0.VI >= 0) {
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+                if (lane + WAVE * m < c0.VI - c0.KK) {
+                    const PrIn &a = in[m];
+                    float vi = lds_at(sm, a.li), vj = lds_at(sm, a.lj);
+                    vi = a.si ? vi : a.ni;
+                    vj = a.sj ? vj : a.nj;
+                    const float sx = vi + a.pa, sy = (jp ? vj : a.pb) - (jp ? a.pb : vj);
+                    float qx, qy;
+                    if (p2) { qx = sx * rx; qy = sy * ry; }
+                    else { qx = sx / DXK; qy = sy / DYK; }
+                    lds_at(sm, rowb + 4 * (low + lane + WAVE * m)) = a.div + qx * DYK * a.dz + qy * DXK * a.dz;
+                }
+            }
+        }
+        lds_barrier();
+        // phase 2, beside the recurrences
+        float xst[M], dnst[M];
+        const StripCol done = c2m;                            // the column of step s-1, before its buffer is reused
+        const unsigned od = op;
+        if (done.VI >= 0) {
+            const int sn = rowb + 4 * ((8 - 4 * (s & 1)) * len + low + lane);
+#pragma unroll
+            for (int m = 0; m < M; ++m)
+                if (lane + WAVE * m < done.VI - done.KK) {
+                    xst[m] = lds_at(sm, sn + 4 * WAVE * m);
+                    dnst[m] = dn[m];
+                }
+        }
+        located();
+        if (s + 1 < nsteps) work_up(s + 1, c0);
+        c2m = c0; op = o0;
+        c0 = c1; o0 = o1;
+        if (s + 1 < nsteps) issue(c0, c2, c2i);
+        else c0 = none;
+        if (c2m.VI >= 0) {                                    // DPMNEW of the column of step s, for its store
+#pragma unroll
+            for (int m = 0; m < M; ++m)
+                if (lane + WAVE * m < c2m.VI - c2m.KK) dn[m] = *lane_at(DPMNEW + (size_t)op + c2m.KK + 1 + m * WAVE, off_l);
+        }
+        if (done.VI >= 0) {
+            const size_t o = (size_t)od + done.KK + 1;
+#pragma unroll
+            for (int m = 0; m < M; ++m)
+                if (lane + WAVE * m < done.VI - done.KK) {
+                    pmax = xst[m] > pmax ? xst[m] : pmax;
+                    pmin = xst[m] < pmin ? xst[m] : pmin;
+                    *(gf32 *)lane_at(DPM + o + m * WAVE, off_l) = xst[m];
+                    *(gf32 *)lane_at(DPMNEW + o + m * WAVE, off_l) = dnst[m] + relaxp * xst[m];
+                }
+        }
+        lds_barrier();                                        // the recurrence outputs are ready
+    }
+    merge(nsteps - 1, c2m);
+    lds_barrier();
+    if (c2m.VI >= 0) {
+        const size_t o = (size_t)op + c2m.KK + 1;
+#pragma unroll
+        for (int m = 0; m < M; ++m)
+            if (lane + WAVE * m < c2m.VI - c2m.KK) {
+                const float x = sm[(size_t)r * rs + (4 + 4 * ((nsteps - 1) & 1)) * len + low + lane + WAVE * m];
+                pmax = x > pmax ? x : pmax;
+                pmin = x < pmin ? x : pmin;
+                ((gf32 *)DPM)[o + lane + WAVE * m] = x;
+                DPMNEW[o + lane + WAVE * m] = dn[m] + relaxp * x;
+            }
+    }
+    // residual: the largest |old DPM - quantised new DPM|.  The divergence pass has
+    // zeroed the old DPM of every cell, and the quantisation is monotonic, so it
+    // is taken from the extreme new values, once per lane instead of per cell.
+    const float ra = (float)fabs((double)conv_to_int((double)pmax * d.frund) / d.frund);
+    const float rb = (float)fabs((double)conv_to_int((double)pmin * d.frund) / d.frund);
+    float rmax = ra > rb ? ra : rb;
     for (int off = WAVE / 2; off > 0; off >>= 1) {
         float other = __shfl_xor(rmax, off);
         rmax = other > rmax ? other : rmax;
     }
-    const int rs = slot - d.iter_off;                 // this situation's residual slot
-    if (lane == 0 && rmax > 0.0f && slot >= 0 && rs >= 0 && rs < d.resid_cap) atomicMax((unsigned *)&d.resid[rs], __float_as_uint(rmax));
+    const int rsl = slot - d.iter_off;                // this situation's residual slot
+    if (lane == 0 && rmax > 0.0f && slot >= 0 && rsl >= 0 && rsl < d.resid_cap) atomicMax((unsigned *)&d.resid[rsl], __float_as_uint(rmax));
 }
 
 static inline int ndiag(int oa, int ob, int ia, int ib) { return (ob - oa) + (ib - ia) + 1; }
@@ -2943,6 +3245,62 @@ static inline int lds_limit(const void *kern, size_t bytes) {
     if (q == n) ++n;
     return 0;
 }
+// Rows of a strip.  A strip is a workgroup of rows + 2 waves; fewer rows mean
+// less work per step and CU, more strips and (a sweep's path is its column
+// range plus rows per strip) about the same number of steps.  Ten rows while
+// all strips of the launch find a CU of their own (400 x 400 city, one
+// situation: pressure, U and V sweeps 1.33, 1.41 and 1.38 ms against 1.42, 1.48
+// and 1.48 with 14), else 14 (eight situations: 1.62, 2.04 and 1.71 ms against
+// 1.80, 2.16 and 1.91 with ten).  Short sweeps, whose path is mostly the fill of
+// their first strips, take seven (25 rows: 60 against 65 us).  swap: the
+// pressure sweep, whose rows run along i.
+static int strip_rows(const Dom *hd, int nsit, bool swap) {
+    long n = 0, longest = 0;
+    for (int q = 0; q < nsit; ++q) {
+        const int nb = (swap ? hd[q].nii : hd[q].njj) - 2;
+        n += (nb + 9) / 10;
+        longest = max(longest, (long)nb);
+    }
+    return n > 256 ? 14 : longest > 40 ? 10 : 7;
+}
+typedef void (*PressureKernel)(const Dom *, int, int, int);
+static PressureKernel pressure_strip(const Dom *hd, int nsit) {
+    int n = 0;
+    for (int q = 0; q < nsit; ++q) n = max(n, hd[q].nact);
+    return n <= WAVE ? k_pressure_strip<1> : k_pressure_strip<2>;
+}
+static size_t pressure_strip_lds(const Dom *hd, int nsit, int rows) {
+    size_t m = 0;
+    for (int q = 0; q < nsit; ++q)
+        m = max(m, sizeof(float) * ((size_t)rows * strip_stride(9, strip_len(0, hd[q].nact)) + (RING + 2) * hd[q].nkp) +
+                       32 * sizeof(int4) + 16);
+    return m;
+}
+// LDS of the momentum strips of a launch (w: the W sweep, whose columns go down
+// into the buildings) and the 64-level groups its tallest column spans
+static inline size_t ml_strip_lds(const Dom *hd, int nsit, bool w, int rows) {
+    size_t m = 0;
+    for (int q = 0; q < nsit; ++q) {
+        const int len = strip_len(w ? hd[q].nlow : 0, hd[q].nact);
+        m = max(m, sizeof(float) * ((size_t)rows * strip_stride(9, len) + 2 * hd[q].nkp) + 32 * sizeof(int4) + 16);
+    }
+    return m;
+}
+typedef void (*StripKernel)(const Dom *, int, int);
+template <int COMP, int WFIX, int KIND>
+static StripKernel ml_strip(const Dom *hd, int nsit) {
+    int n = 0;
+    for (int q = 0; q < nsit; ++q) n = max(n, (COMP == 2 ? hd[q].nlow : 0) + hd[q].nact + 1);
+    return n <= WAVE ? k_ml_strip<COMP, WFIX, KIND, 1> : k_ml_strip<COMP, WFIX, KIND, 2>;
+}
+template <int COMP>
+static int ml_strip_limit(int model, const Dom *hd, int nsit) {
+    bool w8 = true;
+    for (int q = 0; q < nsit; ++q) w8 = w8 && hd[q].simd == 8;
+    const StripKernel k = model == 2 ? ml_strip<COMP, 0, 1>(hd, nsit) : model == 0 ? ml_strip<COMP, 0, 2>(hd, nsit) :
+                          w8 ? ml_strip<COMP, 8, 0>(hd, nsit) : ml_strip<COMP, 0, 0>(hd, nsit);
+    return lds_limit((const void *)k, ml_strip_lds(hd, nsit, COMP == 2, strip_rows(hd, nsit, false)));
+}
 // longest diagonal t over the situations; the pressure sweep runs a over j
 // (outer) and b over i, the momentum sweeps a over i and b over j
 static inline int diag_len_max(const Dom *hd, int nsit, int t, int oa, int ia, bool pressure) {
@@ -3005,6 +3363,7 @@ static int launch_iteration(const Dom *hd, int nsit, const Dom *dd, int iter, in
         nkp = max(nkp, hd[q].nkp); nj2 = max(nj2, hd[q].nj2);
     }
     const unsigned Z = (unsigned)nsit;
+    const int rows_p = strip_rows(hd, nsit, true), rows = strip_rows(hd, nsit, false);
     int kb = (nk + 63) / 64;
     int IS = 1, JS = 1;
     switch (iter % 4) {
@@ -3016,24 +3375,13 @@ static int launch_iteration(const Dom *hd, int nsit, const Dom *dd, int iter, in
     // every strip kernel this iteration launches gets its dynamic-LDS limit
     // before the first launch, so a refusal leaves the fields untouched
     if (d0.tiled == 2) {
-        const size_t shm_p = sizeof(float) * ((size_t)(8 * ROWS + RING) * lds_slot_h(nkp) + 2 * nkp + 8 + WAVE * CH) +
-                             sizeof(int) * (9 * ROWS + 4);
-        const size_t shm_m = sizeof(float) * ((size_t)9 * lds_slot_h(nkp) * ROWS + nkp + 8 + WAVE * CH) +
-                             sizeof(int) * (10 * ROWS + 4);
-        int bad = lds_limit((const void *)k_pressure_strip, shm_p);
-        if (d0.model == 1) {
-            bad |= lds_limit((const void *)k_ml_strip<0>, shm_m) | lds_limit((const void *)k_ml_strip<1>, shm_m) |
-                   lds_limit((const void *)k_ml_strip<2>, shm_m);
-        } else if (d0.model == 2) {
-            bad |= lds_limit((const void *)k_ml_strip<0, 1>, shm_m) | lds_limit((const void *)k_ml_strip<1, 1>, shm_m) |
-                   lds_limit((const void *)k_ml_strip<2, 1>, shm_m);
+        int bad = lds_limit((const void *)pressure_strip(hd, nsit), pressure_strip_lds(hd, nsit, rows_p));
+        bad |= ml_strip_limit<0>(d0.model, hd, nsit) | ml_strip_limit<1>(d0.model, hd, nsit) | ml_strip_limit<2>(d0.model, hd, nsit);
+        if (d0.model == 2) {
             bad |= lds_limit((const void *)k_tke_coef,
                              sizeof(float) * 5 * (nkp | 1) * COEF_COLS + sizeof(int) * (TKE_SCOL * COEF_COLS + 4));
             bad |= lds_limit((const void *)k_tke_strip, sizeof(float) * ((size_t)TKE_SLOTS * ROWS * lds_slot_h(nkp) + WAVE * CH) +
                                                             sizeof(int) * (10 * ROWS + 4));
-        } else {
-            bad |= lds_limit((const void *)k_ml_strip<0, 2>, shm_m) | lds_limit((const void *)k_ml_strip<1, 2>, shm_m) |
-                   lds_limit((const void *)k_ml_strip<2, 2>, shm_m);
         }
         if (bad) return (int)hipErrorInvalidValue;
     }
@@ -3046,19 +3394,17 @@ static int launch_iteration(const Dom *hd, int nsit, const Dom *dd, int iter, in
     }
     const int nrow8 = (nii - 2 + NXCD - 1) / NXCD * NXCD;                 // x extent of the cell kernels (rows)
     L.go(FAM_STENCIL, [&] { hipLaunchKernelGGL(k_divergence, dim3(nrow8, 1, Z), dim3(CELL_THREADS), 0, s, dd); });
-    size_t nrow = (size_t)nj2 * nkp;
+    size_t nrow = d0.tiled ? 0 : (size_t)nj2 * nkp;
     for (int q = 0; q < nsit; ++q) nrow = max(nrow, (size_t)5 * hd[q].sync_stride);
     L.go(FAM_STENCIL, [&] {
         hipLaunchKernelGGL(k_zero_rows, dim3((unsigned)((nrow + 255) / 256), 1, Z), dim3(256), 0, s, dd, d0.tiled ? 0 : 1);
     });
     if (d0.tiled == 2) {
         int nst = 0;
-        for (int q = 0; q < nsit; ++q) nst = max(nst, (hd[q].nii - 1 - 2 + ROWS) / ROWS);
-        size_t shm = sizeof(float) * ((size_t)(8 * ROWS + RING) * lds_slot_h(nkp) + 2 * nkp + 8 + WAVE * CH) +
-                     sizeof(int) * (9 * ROWS + 4);
-        if (lds_limit((const void *)k_pressure_strip, shm)) return (int)hipErrorInvalidValue;
+        for (int q = 0; q < nsit; ++q) nst = max(nst, (hd[q].nii - 3 + rows_p) / rows_p);
+        const size_t shm = pressure_strip_lds(hd, nsit, rows_p);
         L.go(FAM_PRESSURE, [&] {
-            hipLaunchKernelGGL(k_pressure_strip, dim3(nst, 1, Z), dim3(STRIP_WAVES * WAVE), shm, s, dd, IS, JS, slot);
+            hipLaunchKernelGGL(pressure_strip(hd, nsit), dim3(nst, 1, Z), dim3((rows_p + 2) * WAVE), shm, s, dd, IS, JS, slot);
         });
     } else {
         int oa = 2, ob = njj - 1, ia = 2, ib = nii - 1;
@@ -3088,31 +3434,29 @@ static int launch_iteration(const Dom *hd, int nsit, const Dom *dd, int iter, in
                 L.go(fam, [&] { hipLaunchKernelGGL(kern, dim3(len, 1, Z), dim3(WAVE), shm, s, dd, t, is, js); });
         }
     };
-    int lds_err = 0;
     auto strip_sweep = [&](int fam, auto coef, auto strip, int oa, int ia, int is, int js) {
         int nblk = 0, nst = 0;
         for (int q = 0; q < nsit; ++q) {
             int ob = hd[q].nii - 1, ib = hd[q].njj - 1;
             int na = ob - oa + 1, nb = ib - ia + 1;
             nblk = max(nblk, ((na * nb + COEF_COLS - 1) / COEF_COLS + NXCD - 1) / NXCD * NXCD);
-            nst = max(nst, (ib - ia + ROWS) / ROWS);
+            nst = max(nst, (ib - ia + rows) / rows);
         }
         size_t shm_c = sizeof(float) * 3 * (nkp | 1) * COEF_COLS + sizeof(int) * (SCOL * COEF_COLS + 4);
         L.go(FAM_COEF, [&] { hipLaunchKernelGGL(coef, dim3(nblk, 1, Z), dim3(4 * WAVE), shm_c, s, dd, is, js); });
-        size_t shm_t = sizeof(float) * ((size_t)9 * lds_slot_h(nkp) * ROWS + nkp + 8 + WAVE * CH) + sizeof(int) * (10 * ROWS + 4);
-        if (lds_limit((const void *)strip, shm_t)) { lds_err = 1; return; }
-        L.go(fam, [&] { hipLaunchKernelGGL(strip, dim3(nst, 1, Z), dim3(STRIP_WAVES * WAVE), shm_t, s, dd, is, js); });
+        const size_t shm_t = ml_strip_lds(hd, nsit, oa == 2 && ia == 2, rows);
+        L.go(fam, [&] { hipLaunchKernelGGL(strip, dim3(nst, 1, Z), dim3((rows + 2) * WAVE), shm_t, s, dd, is, js); });
     };
     bool all_w8 = true;
     for (int q = 0; q < nsit; ++q) all_w8 = all_w8 && hd[q].simd == 8;
     if (d0.model == 1 && d0.tiled == 2 && all_w8) {
-        strip_sweep(FAM_U, k_ml_coef<0, 8>, k_ml_strip<0>, 3, 2, IS, JS);
-        strip_sweep(FAM_V, k_ml_coef<1, 8>, k_ml_strip<1>, 2, 3, -IS, -JS);
-        strip_sweep(FAM_W, k_ml_coef<2, 8>, k_ml_strip<2>, 2, 2, IS, JS);
+        strip_sweep(FAM_U, k_ml_coef<0, 8>, ml_strip<0, 8, 0>(hd, nsit), 3, 2, IS, JS);
+        strip_sweep(FAM_V, k_ml_coef<1, 8>, ml_strip<1, 8, 0>(hd, nsit), 2, 3, -IS, -JS);
+        strip_sweep(FAM_W, k_ml_coef<2, 8>, ml_strip<2, 8, 0>(hd, nsit), 2, 2, IS, JS);
     } else if (d0.model == 1 && d0.tiled == 2) {
-        strip_sweep(FAM_U, k_ml_coef<0, 0>, k_ml_strip<0>, 3, 2, IS, JS);
-        strip_sweep(FAM_V, k_ml_coef<1, 0>, k_ml_strip<1>, 2, 3, -IS, -JS);
-        strip_sweep(FAM_W, k_ml_coef<2, 0>, k_ml_strip<2>, 2, 2, IS, JS);
+        strip_sweep(FAM_U, k_ml_coef<0, 0>, ml_strip<0, 0, 0>(hd, nsit), 3, 2, IS, JS);
+        strip_sweep(FAM_V, k_ml_coef<1, 0>, ml_strip<1, 0, 0>(hd, nsit), 2, 3, -IS, -JS);
+        strip_sweep(FAM_W, k_ml_coef<2, 0>, ml_strip<2, 0, 0>(hd, nsit), 2, 2, IS, JS);
     } else if (d0.model == 1) {
         sweep(FAM_U, k_momentum<0, 0>, 3, 2, IS, JS);
         sweep(FAM_V, k_momentum<1, 0>, 2, 3, -IS, -JS);
@@ -3120,9 +3464,9 @@ static int launch_iteration(const Dom *hd, int nsit, const Dom *dd, int iter, in
     } else if (d0.model == 2) {
         if (d0.tiled == 2) {
             // the k-eps V solver sweeps in the same directions as U and W
-            strip_sweep(FAM_U, k_ml_coef<0, 0, 1>, k_ml_strip<0, 1>, 3, 2, IS, JS);
-            strip_sweep(FAM_V, k_ml_coef<1, 0, 1>, k_ml_strip<1, 1>, 2, 3, IS, JS);
-            strip_sweep(FAM_W, k_ml_coef<2, 0, 1>, k_ml_strip<2, 1>, 2, 2, IS, JS);
+            strip_sweep(FAM_U, k_ml_coef<0, 0, 1>, ml_strip<0, 0, 1>(hd, nsit), 3, 2, IS, JS);
+            strip_sweep(FAM_V, k_ml_coef<1, 0, 1>, ml_strip<1, 0, 1>(hd, nsit), 2, 3, IS, JS);
+            strip_sweep(FAM_W, k_ml_coef<2, 0, 1>, ml_strip<2, 0, 1>(hd, nsit), 2, 2, IS, JS);
         } else {
             sweep(FAM_U, k_momentum<0, 1>, 3, 2, IS, JS);
             sweep(FAM_V, k_momentum<1, 1>, 2, 3, IS, JS);
@@ -3153,16 +3497,15 @@ static int launch_iteration(const Dom *hd, int nsit, const Dom *dd, int iter, in
             }
         }
     } else if (d0.tiled == 2) {
-        strip_sweep(FAM_U, k_ml_coef<0, 0, 2>, k_ml_strip<0, 2>, 3, 2, IS, JS);
-        strip_sweep(FAM_V, k_ml_coef<1, 0, 2>, k_ml_strip<1, 2>, 2, 3, IS, JS);
-        strip_sweep(FAM_W, k_ml_coef<2, 0, 2>, k_ml_strip<2, 2>, 2, 2, IS, JS);
+        strip_sweep(FAM_U, k_ml_coef<0, 0, 2>, ml_strip<0, 0, 2>(hd, nsit), 3, 2, IS, JS);
+        strip_sweep(FAM_V, k_ml_coef<1, 0, 2>, ml_strip<1, 0, 2>(hd, nsit), 2, 3, IS, JS);
+        strip_sweep(FAM_W, k_ml_coef<2, 0, 2>, ml_strip<2, 0, 2>(hd, nsit), 2, 2, IS, JS);
     } else {
         sweep(FAM_U, k_momentum<0, 2>, 3, 2, IS, JS);
         sweep(FAM_V, k_momentum<1, 2>, 2, 3, IS, JS);
         sweep(FAM_W, k_momentum<2, 2>, 2, 2, IS, JS);
     }
     if (launches) *launches += L.n;
-    if (lds_err) return (int)hipErrorInvalidValue;
     return (int)hipGetLastError();
 }
 
