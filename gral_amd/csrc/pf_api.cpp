@@ -699,10 +699,8 @@ extern "C" int gral_pf_prepare(gral_pf_handle *h, const gral_pf_params *p) {
     if (sw && std::strcmp(sw, "diag") == 0) d.tiled = 0;
     if (h->kadvmax + 2 > 128) d.tiled = 0;   // the strip kernels hold at most 128 levels per column
     {
-        // strip synchronisation: header + one block per sweep kind (pressure, U, V, W)
-        const int rows = STRIP_ROWS;
-        int nstrip = (std::max(h->nii, h->njj) + rows - 1) / rows + 1;
-        d.sync_stride = ((2 + nstrip) + 63) & ~63;
+        // strip synchronisation: header + one block per sweep kind (pressure, U, V, W, TKE)
+        d.sync_stride = 64;
         int *fs;
         if ((rc = dalloc(h, &fs, (size_t)SYNC_BLOCK0 + 5 * (size_t)d.sync_stride))) return rc;
         HIPCHK(h, hipMemsetAsync(fs, 0, sizeof(int) * ((size_t)SYNC_BLOCK0 + 5 * (size_t)d.sync_stride), h->stream));

@@ -43,8 +43,8 @@ struct DomT {
     int resid_cap;                   // entries in resid
     // sweep kernels
     int tiled;                       // 2: strip-pipelined sweeps, 0: one launch per anti-diagonal
-    P<int> sync;                     // strip sweeps: [64] header (sticky error flag at 0), then 4 blocks
-    int sync_stride;                 //   of sync_stride ints (ticket, unused, progress per strip)
+    P<int> sync;                     // strip sweeps: [64] header (sticky error flag, iteration count), then per
+    int sync_stride;                 //   sweep kind sync_stride ints (the ticket, alone in its cache lines)
     P<unsigned long long> hand;      // values handed from strip to strip: {value, tag} words [2][strip][hand_cols][nkp]
     size_t hand_words;               // words of one of the two
     int hand_cols;
@@ -178,8 +178,7 @@ struct MomAdj {
     float *gres;        // dL/dX before, complete
 };
 
-#define SYNC_BLOCK0 64               // Dom::sync: sticky error flag at 0, sweep blocks from here
-#define STRIP_ROWS 15                // sweep rows per strip workgroup (plus one chain wave)
+#define SYNC_BLOCK0 64               // Dom::sync: sweep blocks from here
 #define STRIP_ROWS_MIN 7             // fewest rows of a strip (strip_rows())
 
 __device__ __forceinline__ size_t c2(const DomG &d, int i, int j) { return (size_t)i * (size_t)d.nj2 + (size_t)j; }

@@ -1350,8 +1350,8 @@ __global__ __launch_bounds__(WAVE) void k_tke(const Dom *__restrict__ ds, int t,
 // ------------------------------------------------------------------------
 // Strip wavefront path (mixing-length model and pressure)
 // ------------------------------------------------------------------------
-// A workgroup owns ROWS consecutive sweep rows (b) with one wave per row plus
-// a chain wave.  Row wave r owns row b0 + r and at local step s handles column
+// A workgroup owns consecutive sweep rows (b) with one wave per row, a chain
+// wave and a control wave.  Row wave r owns row b0 + r and at local step s handles column
 // a = oa + s - r, so every local step is one anti-diagonal of the strip.  Each
 // step is three phases separated by workgroup barriers: (1) every active row
 // wave assembles its column's source terms (lanes over k) into LDS, (2) the
@@ -1359,8 +1359,7 @@ __global__ __launch_bounds__(WAVE) void k_tke(const Dom *__restrict__ ds, int t,
 // (lane = row) while the row waves prefetch their next columns, (3) the row
 // waves write their columns back.  Neighbours updated in the previous step are
 // exchanged through LDS column buffers.
-#define ROWS STRIP_ROWS
-#define STRIP_WAVES (STRIP_ROWS + 1)
+#define STRIP_WAVES 16            // waves of a strip at most: 14 rows, the chain and the control wave
 
 // coefficient records written by k_ml_coef and read by the strip sweeps; per
 // cell, two records, each written whole, in one pass:
@@ -1529,168 +1528,25 @@ __global__ __launch_bounds__(4 * WAVE) void k_ml_coef(const Dom *__restrict__ ds
 }
 
 
-// Serial Thomas recurrences of one column (one lane), software-pipelined: the
-// operands of the next CH levels are read from LDS while the current CH levels
-// are computed.  Pointers are relative to the first level of the recurrence and
-// the loops run over n levels; the LDS slots carry 2*CH floats of padding on
-// both sides, so the look-ahead reads need no clamping (their values are unused).
-#define CH 8
-#define SLOT_PAD (2 * CH)
-__device__ __forceinline__ int lds_slot(int nkp) { return (nkp + 2 * SLOT_PAD) | 1; }
-
-// The chunk loops below are unrolled over the largest column the strip
-// kernels hold (MAXCH chunks of CH levels) and leave early at the
-// wave-wide longest chain (nmax): straight-line code lets the compiler wait
-// for exactly the LDS reads a chunk needs, while the reads of the next chunk
-// are in flight.  Reads stay within CH levels past a lane's own range (the
-// slot padding); a lane that is done re-reads its first chunk.  A lane's
-// last chunk stores up to CH-1 levels past its range (into the slot padding or
-// levels nobody reads), and chunks after its end go to a per-lane sink of CH
-// words, so the chunks are branch-free.  The back-substitution writes its
-// result to a separate slot (the old column stays readable and untouched below
-// the range).
-#define MAXCH (128 / CH)
-
-// forward: Q[t] = (D[t] + C[t]*Q[t-1]) * T[t], t = 0..n-1, Q[-1] = q0
-template <bool DIV>
-__device__ __forceinline__ void chain_fwd(const float *__restrict__ D, const float *__restrict__ C,
-                                          const float *__restrict__ T, float *__restrict__ Q, int n, int nmax, float q0,
-                                          float *sink) {
-    float Qp = q0;
-    float cd[CH], cc[CH], ct[CH];
-#pragma unroll
-    for (int u = 0; u < CH; ++u) { cd[u] = D[u]; cc[u] = C[u]; ct[u] = T[u]; }
-#pragma unroll
-    for (int h = 0; h < MAXCH; ++h) {
-        const int t = h * CH;
-        if (t >= nmax) break;
-        float nd[CH], nc[CH], nt[CH];
-        const int o = (t + CH < n) ? t + CH : 0;          // lanes already past their end re-read level 0
-#pragma unroll
-        for (int u = 0; u < CH; ++u) { nd[u] = D[o + u]; nc[u] = C[o + u]; nt[u] = T[o + u]; }
-        __builtin_amdgcn_sched_barrier(0);                // keep the next chunk's reads ahead of this chunk
-        float *Qw = (t < n) ? Q : sink - t;              // a lane past its end stores to its sink
-#pragma unroll
-        for (int u = 0; u < CH; ++u) {
-            float q = DIV ? (cd[u] + cc[u] * Qp) / ct[u] : (cd[u] + cc[u] * Qp) * ct[u];
-            Qw[t + u] = q;
-            Qp = q;
-        }
-#pragma unroll
-        for (int u = 0; u < CH; ++u) { cd[u] = nd[u]; cc[u] = nc[u]; ct[u] = nt[u]; }
-    }
-}
-
-// largest value of v over the lanes of the wave that pass `on` (0 if none)
-__device__ __forceinline__ int wave_max(int v, bool on) {
-    int m = on ? v : 0;
-    for (int off = WAVE / 2; off > 0; off >>= 1) m = max(m, __shfl_xor(m, off));
-    return __builtin_amdgcn_readfirstlane(m);
-}
-
-// p + byte_off with a 32-bit byte offset: with a uniform base the access can
-// take the scalar-base form (base in scalar registers, 32-bit lane offset), so
-// no 64-bit address arithmetic per lane
-__device__ __forceinline__ const gf32 *at_bytes(const gf32 *base, unsigned byte_off) {
-    typedef const char __attribute__((address_space(1))) gc8;
-    return (const gf32 *)((const gc8 *)base + byte_off);
-}
 // ------------------------------------------------------------------------
 // Strip-pipelined sweeps.  Strip B reads the last row of strip B-1 (its new
 // values, and for the pressure sweep the QIMP row scratch) and nothing else
-// from other strips, so it only has to stay ROWS steps behind strip B-1: one
-// launch holds the whole sweep, whose serial path is about (a range) +
-// ROWS * (number of strips) local steps.
+// from other strips, so it only has to stay a strip's rows behind strip B-1: one
+// launch holds the whole sweep, whose serial path is about (a range) + rows *
+// (number of strips) local steps.
 //
-// Synchronisation, per situation and sweep kind, in int sync[...]:
-//   [0] ticket counter: strips are numbered in the order their workgroups
-//       start, so the strip a workgroup waits for is held by a workgroup
-//       that is already running (no dependence on dispatch order);
-//   [2 + B] steps of strip B whose hand-off stores are complete;
-// the blocks are cleared at the start of every iteration.  d.sync[0] is the
-// situation's sticky error flag: set when a wait exceeded the time limit.
-// The wave that stores the last row's results (the chain wave in the momentum
-// strips, the last row wave otherwise) publishes the strip's progress after
-// waiting for those write-through stores; row 0 of the next strip polls it and
-// then reads the handed-over values with agent-scope loads.  Every
-// wait is bounded (STRIP_TIMEOUT_TICKS of the constant 100 MHz clock): on
-// timeout the strip sets the error flag and goes on without waiting, so the
+// Strips are numbered by a ticket per sweep kind (sync[SYNC_BLOCK0 + kind *
+// sync_stride], cleared at the start of every iteration) in the order their
+// workgroups start, so the strip a workgroup waits for is held by a workgroup
+// that is already running, whatever the dispatch order.  Every wait is bounded
+// (STRIP_TIMEOUT_TICKS of the constant 100 MHz clock): on timeout the strip sets
+// the situation's sticky error flag (sync[0]) and goes on without waiting, so the
 // kernel always ends; the host reports the error.
 // ------------------------------------------------------------------------
-#define SYNC_HDR 2
-// a strip publishes its progress every STRIP_PUBLISH steps (and at its end); a
-// longer interval adds up to STRIP_PUBLISH-1 steps of lag per strip.  The
-// publish is a wait for the strip's own write-through stores, and the reader
-// takes the hand-off values with agent-scope loads, so neither side writes back
-// or invalidates an L2.  Measured on the 8-direction city batch (ms per launch,
-// publishing every 1 / 2 / 3 / 4 steps): U and V sweeps 2.8 / 2.9 / 2.95 / 3.0,
-// W 2.77 / 2.84 / 2.96 / 3.06, pressure 2.62 / 2.78 / 2.81 / 2.95.  (With an
-// agent-scope release fence, which writes back the whole L2 of the XCD, every
-// publish cost about 4 us: 7.6-8.2 ms for U and V at every step, 4.1 at every 6th.)
-#ifndef STRIP_PUBLISH
-#define STRIP_PUBLISH 1
-#endif
 #define STRIP_TIMEOUT_TICKS 200000000ull
 
-__device__ __forceinline__ int load_agent(const gi32 *p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 __device__ __forceinline__ void store_agent(gi32 *p, int v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-// The values a strip hands to the next one (the new last row, the pressure row
-// scratch) are read with agent-scope loads: they are served coherently across
-// the XCDs' L2 caches, so the reader needs no L2 invalidation (an agent-scope
-// acquire fence, which would also drop every other workgroup's cached lines on
-// that XCD) - only the order after its progress poll, which the poll's
-// control dependency and a compiler fence give.
-__device__ __forceinline__ float ld_handoff(const gf32 *p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-struct StripWait {
-    const gi32 *prev;              // progress of the previous strip (null for strip 0)
-    gi32 *error;
-    int seen;                      // progress of the previous strip known so far
-    int cap;                       // steps of a strip
-    unsigned long long deadline;
-    // called by every lane of one wave; returns once the previous strip has
-    // completed min(target, cap) steps (or the time limit passed)
-    __device__ __forceinline__ void wait(int target) {
-        target = min(target, cap);
-        if (seen >= target) return;
-        for (int spins = 0;; ++spins) {
-            int p = __builtin_amdgcn_readfirstlane(load_agent(prev));
-            if (p >= target) { seen = p; break; }
-            if (wall_clock64() > deadline || spins > (1 << 22)) {
-                store_agent(error, 1);
-                seen = 0x7fffffff;
-                break;
-            }
-            __builtin_amdgcn_s_sleep(2);
-        }
-        // the hand-off loads that follow are agent-scope loads (ld_handoff):
-        // keep the compiler from moving them above the poll
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    }
-};
-
-// The sweeps' own stores are agent-scope (sc1) stores, which the L2 writes
-// through, so the L2 of the XCD holds no dirty lines from them when a strip
-// publishes (an agent-scope release writes back every dirty line of the L2).
-__device__ __forceinline__ void st_through(gf32 *p, float v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// called by every lane of the publishing wave: progress v (steps whose
-// stores this wave issued) becomes visible with the stores before it.  Those
-// stores are agent-scope write-through stores: once complete they are visible
-// to the agent-scope loads of every XCD, so the release is a wait for them
-// (no write-back of the whole L2, as an agent-scope release fence would do)
-// followed by the progress store.
-__device__ __forceinline__ void strip_publish(gi32 *mine, int v, int lane) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    if (lane == 0) store_agent(mine, v);
 }
 
 // ------------------------------------------------------------------------
@@ -2967,265 +2823,342 @@ __global__ __launch_bounds__(4 * WAVE) void k_tke_coef(const Dom *__restrict__ d
     }
 }
 
-// Relaxation-free back-substitution of the TKE sweep, downwards from level
-// VI (pointers at VI): X[-t] = max(P*X[-t+1] + Q, floor), or the wall value
-// where the wall flag is set, t = 0..n-1, X[1] = top (the old value above VI).
-// The clamp is the reference's double-precision Math.Max.
-__device__ __forceinline__ void chain_tke_back(const float *__restrict__ P, const float *__restrict__ Q,
-                                               const float *__restrict__ WF, const float *__restrict__ WV,
-                                               float *__restrict__ X, float top, double floor_, int n, int nmax,
-                                               float *sink) {
+// Relaxation-free back-substitution of the TKE sweep from t = n-1 down, chunks
+// as in strip_back: X[t] = max(P[t]*X[t+1] + Q[t], floor), or the wall value V[t]
+// (already floored) where there is one (V != -1; wall values are not negative),
+// X[n] = top; X replaces V.  The reference floors with the double-precision
+// Math.Max(x, floor_): floor is floor_ rounded to float, which lies above floor_
+// for both of its values, so x is replaced exactly where x < floor, and a NaN
+// stays.
+#define TKE_NO_WALL (-1.0f)
+__device__ __forceinline__ void strip_tke_back(const float *P, const float *Q, float *V, float top, float floor, int n, int nch,
+                                               bool part, int low) {
+    int o = (n - 1) & ~(CHK - 1);
+    const int tl = n - o;
     float up = top;
-    float cp[CH], cq[CH], cf[CH], cv[CH];
-    // chunks addressed from their lowest level upwards, as in chain_back
-    {
-        const float *Pb = P - (CH - 1), *Qb = Q - (CH - 1), *Fb = WF - (CH - 1), *Vb = WV - (CH - 1);
+    Chunk p[2], q[2], v[2];
+    p[0] = ld_chunk(P + o); q[0] = ld_chunk(Q + o); v[0] = ld_chunk(V + o);
+    for (int b = 0; b < nch; b += CHK_BLOCK) {
 #pragma unroll
-        for (int u = 0; u < CH; ++u) {
-            cp[u] = Pb[CH - 1 - u]; cq[u] = Qb[CH - 1 - u]; cf[u] = Fb[CH - 1 - u]; cv[u] = Vb[CH - 1 - u];
+        for (int h = 0; h < CHK_BLOCK; ++h) {
+            if (b + h >= nch) return;
+            const int k = h & 1, m = k ^ 1, on = max(o - CHK, -low);
+            p[m] = ld_chunk(P + on); q[m] = ld_chunk(Q + on); v[m] = ld_chunk(V + on);
+            __builtin_amdgcn_sched_barrier(0);
+            const bool sel = h == 0 && part && b == 0;
+#pragma unroll
+            for (int u = CHK - 1; u >= 0; --u) {
+                float x = p[k].v[u] * up + q[k].v[u];
+                x = x < floor ? floor : x;
+                x = v[k].v[u] != TKE_NO_WALL ? v[k].v[u] : x;
+                if (h == 0) up = (sel && u >= tl) ? up : x;
+                else up = x;
+                v[k].v[u] = x;
+            }
+            st_chunk(V + o, v[k]);
+            o = on;
         }
-    }
-#pragma unroll
-    for (int h = 0; h < MAXCH; ++h) {
-        const int t = h * CH;
-        if (t >= nmax) break;
-        float np[CH], nq[CH], nf[CH], nv[CH];
-        const int o = (t + CH < n) ? t + CH : 0;
-        const float *Pb = P - (o + CH - 1), *Qb = Q - (o + CH - 1), *Fb = WF - (o + CH - 1), *Vb = WV - (o + CH - 1);
-#pragma unroll
-        for (int u = 0; u < CH; ++u) {
-            np[u] = Pb[CH - 1 - u]; nq[u] = Qb[CH - 1 - u]; nf[u] = Fb[CH - 1 - u]; nv[u] = Vb[CH - 1 - u];
-        }
-        __builtin_amdgcn_sched_barrier(0);                // keep the next chunk's reads ahead of this chunk
-        float *Xw = (t < n) ? X - (t + CH - 1) : sink;
-#pragma unroll
-        for (int u = 0; u < CH; ++u) {
-            float x = (cf[u] != 0.0f) ? cv[u] : cp[u] * up + cq[u];
-            x = (float)mmaxd((double)x, floor_);
-            Xw[CH - 1 - u] = x;
-            up = x;
-        }
-#pragma unroll
-        for (int u = 0; u < CH; ++u) { cp[u] = np[u]; cq[u] = nq[u]; cf[u] = nf[u]; cv[u] = nv[u]; }
     }
 }
 
-// per-level values of one column of the TKE sweep, loaded one local step ahead
-struct TkePre {
+// raw operands of one column of the TKE sweep, loaded a step before they are worked up
+struct TkeRaw {
     float4 c0, c1, c2;              // record words 0..11
     float4 c3;                      // den1, P1, den2, P2
     float2 c4;                      // wall TURB, wall TDISS
     float ta, ea, tb, eb;           // old TURB/TDISS in the +IS (a) and +JS (b) directions
     float nit, nie, njt, nje;       // -IS / -JS neighbours as memory holds them
+    unsigned long long ht, he;      // row 0: the previous strip's last row
+};
+struct TkeIn {
+    float ai, aj, at, bt, ae, be;   // coefficients of the new neighbours, products of the old ones
+    float w1, pro, pbo, w2, eps;
+    float nit, nie, njt, nje;
+    int li, lj;
+    bool si, sj;
 };
 
-// Strip sweep of TURB and TDISS, laid out as k_ml_strip: ROWS row waves and a
-// chain wave.  Row wave r owns sweep row b0 + r (j direction) and at step s
-// handles column a = 2 + s - r: it assembles the column's two sources from the
-// record (k_tke_coef) and the four neighbours (lanes over levels) and lays the
-// recurrence operands out in LDS; the chain wave then runs the Q recurrences and
-// the back-substitution of every row at once (lane r: TURB of row r, lane
-// ROWS + r: TDISS of row r), while the row waves load the next column.  The
-// neighbours updated earlier in the sweep (the previous column of the same
-// row, the previous row's column of the previous step) are merged on use from
-// the recurrence outputs in LDS over the levels they updated; their other
-// levels, and row 0's neighbours in the previous strip, come from memory.
-// LDS per row: D1, D2, C1, den1, P1, C2, den2, P2, wall flag, wall TURB,
-// wall TDISS, Q1, Q2, new TURB, new TDISS.
-#define TKE_SLOTS 15
+// Strip sweep of TURB and TDISS, laid out as k_ml_strip (row, chain and control
+// waves, two phases a step).  The chain wave runs both recurrences of every row
+// at once: lane r TURB of row r, lane 16 + r TDISS of row r.
+#define TKE_ARRAYS 18
+template <int M>
 __global__ __launch_bounds__(STRIP_WAVES * WAVE) void k_tke_strip(const Dom *__restrict__ ds, int IS, int JS) {
     const DomG &d = reinterpret_cast<const DomG *>(ds)[blockIdx.z];                   // situation of this launch slice
-    extern __shared__ float sm[];
-    const int nkp = d.nkp, nkl = lds_slot(nkp);
-    const int oa = 2, ia = 2, ob = d.nii - 1, ib = d.njj - 1;
-    const int nstrip = (ib - ia + ROWS) / ROWS, nsteps = (ob - oa + 1) + ROWS - 1;
+    extern __shared__ __align__(16) float sm[];
+    const int nkp = d.nkp, nii = d.nii, njj = d.njj, nj2 = d.nj2, hcols = d.hand_cols;
+    const int low = strip_low(0), len = strip_len(0, d.nact), rs = strip_stride(TKE_ARRAYS, len), fs = 9 * len;
+    const int oa = 2, ia = 2, ob = nii - 1, ib = njj - 1, na = ob - oa + 1;
+    const int R = blockDim.x / WAVE - 2;
+    const int nstrip = (ib - ia + R) / R, nsteps = na + R - 1;
     const int r = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
-    const bool chainw = r == ROWS;
     gi32 *sync = d.sync + SYNC_BLOCK0 + (size_t)4 * d.sync_stride;
-    float *rowb = sm + (size_t)r * TKE_SLOTS * nkl + SLOT_PAD;
-    float *sD1 = rowb, *sD2 = rowb + nkl, *sC1 = rowb + 2 * nkl, *sN1 = rowb + 3 * nkl, *sP1 = rowb + 4 * nkl;
-    float *sC2 = rowb + 5 * nkl, *sN2 = rowb + 6 * nkl, *sP2 = rowb + 7 * nkl, *sWF = rowb + 8 * nkl;
-    float *sWT = rowb + 9 * nkl, *sWE = rowb + 10 * nkl, *sQ1 = rowb + 11 * nkl, *sQ2 = rowb + 12 * nkl;
-    float *sOT = rowb + 13 * nkl, *sOE = rowb + 14 * nkl;
-    float *sdump = sm + (size_t)ROWS * TKE_SLOTS * nkl;          // [WAVE][CH] sinks of the chains
-    int *sinfo = (int *)(sdump + WAVE * CH);                    // [2][ROWS] per row: active, lo, VI, top TURB, top TDISS
-    int *sctl = sinfo + 10 * ROWS;
+    // per row, for TURB and (fs further) TDISS: D (replaced by Q), then per step
+    // parity C, the denominator, P and the wall value (replaced by the new value)
+    int4 *sinfo = (int4 *)(sm + (size_t)R * rs);              // [2][32] per chain lane by step parity
+    int *sctl = (int *)(sinfo + 64);
     if (threadIdx.x == 0) sctl[0] = __hip_atomic_fetch_add(&sync[0], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
-    const int B = sctl[0];
+    const int B = __builtin_amdgcn_readfirstlane(sctl[0]);
     if (B >= nstrip) return;                                  // uniform over the workgroup
-    if (chainw) {
-        __builtin_amdgcn_s_setprio(3);                        // ahead of the row waves, as in k_ml_strip
-        // the rows publish the levels of step s one phase early (as in
-        // k_ml_strip) and the values above the top with their sources
-        const int f = lane >= ROWS ? 1 : 0, cl = lane < 2 * ROWS ? lane - f * ROWS : 0;
-        bool on = false;
-        int lo = 0, VI = 0, nfmax = 0, nbmax = 0;
-        auto info = [&](int s) {
-            const int *si = sinfo + (s & 1) * 5 * ROWS;
-            on = lane < 2 * ROWS && si[cl * 5];
-            lo = si[cl * 5 + 1]; VI = si[cl * 5 + 2];
-            nfmax = wave_max(VI - lo, on); nbmax = wave_max(VI - lo + 1, on);
+    const unsigned tag = hand_tag(d, 4);
+    gu64 *handt = (gu64 *)d.hand, *hande = handt + d.hand_words;      // TURB, TDISS: [strip][hand_cols][nkp]
+    const int4 *meta = (const int4 *)d.meta;
+    const bool send = B + 1 < nstrip;
+    if (r == R) {                                             // chain wave
+        __builtin_amdgcn_s_setprio(3);
+        const int f = (lane >> 4) & 1, cl = (lane & 15) < R ? lane & 15 : 0;
+        float *L = sm + (size_t)cl * rs + f * fs + low;
+        const float floor = f ? 0.0000001f : 0.001f;
+        // the last row's new values go out while the rows assemble the next step
+        const float *xl = sm + (size_t)(R - 1) * rs + 4 * len + low;
+        const size_t hb = ((size_t)B * hcols - R) * nkp;      // + s*nkp: the last row's column of step s - 1
+        int n = 0, vi = 0;
+        auto send_last = [&](int s) {
+            const int nl = __builtin_amdgcn_readlane(n, R - 1), kl = __builtin_amdgcn_readlane(vi, R - 1) - nl + 1;
+            if (send)
+                for (int t = lane; t < nl; t += WAVE) {
+                    const float *x = xl + 4 * ((s - 1) & 1) * len + t;
+                    hand_put(handt + hb + (size_t)s * nkp + kl + t, x[0], tag);
+                    hand_put(hande + hb + (size_t)s * nkp + kl + t, x[fs], tag);
+                }
         };
+        lds_barrier();                                        // the control wave's data of step 0
         for (int s = 0; s < nsteps; ++s) {
+            // levels (0: no column), chunks | partial chunk << 16, VI, value above the column
+            const int4 si = sinfo[(s & 1) * 32 + (lane & 31)];
+            send_last(s);
+            n = (lane < 32 && (lane & 15) < R) ? si.x : 0;
+            vi = si.z;
+            const int fm = __builtin_amdgcn_readfirstlane(si.y);
             lds_barrier();                                    // the rows' sources are assembled
-            if (s == 0) info(0);
-            const int *si = sinfo + (s & 1) * 5 * ROWS;
-            const float top = __int_as_float(si[cl * 5 + 3 + f]);
-            if (on) {
-                float *R = sm + (size_t)cl * TKE_SLOTS * nkl + SLOT_PAD;
-                float *Dv = R + (size_t)f * nkl, *Cv = R + (size_t)(2 + 3 * f) * nkl, *Nv = R + (size_t)(3 + 3 * f) * nkl;
-                float *Pv = R + (size_t)(4 + 3 * f) * nkl, *WF = R + 8 * (size_t)nkl, *WV = R + (size_t)(9 + f) * nkl;
-                float *Qv = R + (size_t)(11 + f) * nkl, *Ov = R + (size_t)(13 + f) * nkl;
-                chain_fwd<true>(Dv + lo + 1, Cv + lo + 1, Nv + lo + 1, Qv + lo + 1, VI - lo, nfmax, Qv[lo], sdump + lane * CH);
-                chain_tke_back(Pv + VI, Qv + VI, WF + VI, WV + VI, Ov + VI, top, f ? 0.0000001 : 0.001, VI - lo + 1,
-                               nbmax, sdump + lane * CH);
+            if (n > 0) {
+                float *Lp = L + (1 + 4 * (s & 1)) * len;
+                strip_fwd<true>(L, Lp, Lp + len, fm & 0xffff);
+                strip_tke_back(Lp + 2 * len, L, Lp + 3 * len, __int_as_float(si.w), floor, n, fm & 0xffff, (fm >> 16) != 0, low);
             }
             lds_barrier();                                    // the recurrences are done
-            if (s + 1 < nsteps) info(s + 1);
+        }
+        send_last(nsteps);
+        return;
+    }
+    if (r == R + 1) {                                         // control wave
+        __builtin_amdgcn_s_setprio(2);
+        const int row = lane & 15, b = ia + B * R + row;
+        const bool lane_ok = lane < 32 && row < R && b <= ib;
+        const gf32 *F = lane < 16 ? d.turb : d.tdiss;
+        int cidx = ((IS == -1) ? nii - oa + 1 : oa) * nj2 + ((JS == -1) ? njj - b + 1 : b) - row * IS * nj2;
+        // a column's metadata is requested two steps ahead, the value above it one
+        auto meta_at = [&](int s) {
+            const int l = s - row;
+            int4 m = make_int4(0, -1, 0, 0);
+            if (lane_ok && l >= 0 && l < na) m = ldg4i((const DomG::P<const int4>)meta + cidx);
+            cidx += IS * nj2;
+            return m;
+        };
+        int4 mq = meta_at(0), mb = make_int4(0, -1, 0, 0);
+        float top = 0.0f;
+        auto advance = [&](int s) {                           // metadata of step s arrives, its top value is requested
+            const int c = cidx - IS * nj2;
+            mb = mq;
+            mq = meta_at(s + 1);
+            top = 0.0f;
+            if (mb.z & 0x10000) top = F[(size_t)c * nkp + mb.y + 1];
+        };
+        auto info = [&](int s) {
+            const int n = (mb.z & 0x10000) ? mb.y - mb.x : 0;
+            const int part = __any((n & (CHK - 1)) != 0) ? 0x10000 : 0;
+            const int fm = row_max((n + CHK - 1) >> 3);
+            if (lane < 32) sinfo[(s & 1) * 32 + lane] = make_int4(n, fm | part, mb.y, __float_as_int(top));
+        };
+        advance(0);
+        info(0);
+        advance(1);
+        lds_barrier();
+        for (int s = 0; s < nsteps; ++s) {
+            info(s + 1);
+            advance(s + 2);
+            lds_barrier();
+            lds_barrier();
         }
         return;
     }
-    const int b = ia + B * ROWS + r;
-    const bool row_ok = b <= ib;
-    StripWait sw{B > 0 ? sync + SYNC_HDR + B - 1 : nullptr, d.sync, B > 0 ? 0 : 0x7fffffff, nsteps,
-                 wall_clock64() + STRIP_TIMEOUT_TICKS};
-    gi32 *mine = sync + SYNC_HDR + B;
-    TkePre pre[2];
-    Meta mn;
-    int in_ = 0, jn_ = 0;
-    bool inr_n = false;
-    float topt = 0.0f, tope = 0.0f;
-    auto meta_at = [&](int s) {
-        int l = s - r, i, j;
-        if (row_ok && l >= 0 && oa + l <= ob) {
-            sweep_to_ij(d, 0, oa + l, b, IS, JS, i, j);
-            return ldc4i(d.meta + c2(d, i, j));
+    const int b = ia + B * R + r;
+    const bool row_ok = b <= ib, from_prev = r == 0 && B > 0, has_j = r > 0 || B > 0, ip = IS == 1, jp = JS == 1;
+    HandWait hwait{d.sync, wall_clock64() + STRIP_TIMEOUT_TICKS, false};
+    const int rowb = 4 * r * rs, dcol = IS * nj2;
+    gf32 *TW = d.turb, *EW = d.tdiss;
+    const gf32 *planes = d.planes, *rec4 = d.planes + tke_rec4(d);
+    int l2 = -r;
+    int cidx2 = ((IS == -1) ? nii - oa + 1 : oa) * nj2 + ((JS == -1) ? njj - b + 1 : b) - r * dcol;
+    int4 m2, m2j;
+    auto request = [&]() {                                    // metadata of the next column and its -JS neighbour
+        m2 = m2j = make_int4(0, -1, 0, 0);
+        if (row_ok && l2 >= 0 && l2 < na) {
+            m2 = ldc4i(meta + cidx2);
+            if (has_j) m2j = ldc4i(meta + (cidx2 - JS));
         }
-        return make_int4(0, -1, 0, 0);
+        ++l2;
+        cidx2 += dcol;
     };
-    int4 mq = meta_at(0);
-    auto locate = [&](int s) {
-        int l = s - r;
-        inr_n = row_ok && l >= 0 && oa + l <= ob;
-        const int4 m4 = mq;
-        mq = meta_at(s + 1);
-        mn.adv = false;
-        if (inr_n) {
-            sweep_to_ij(d, 0, oa + l, b, IS, JS, in_, jn_);
-            mn = unpack_meta(m4);
-        }
-        if (mn.adv) {
-            const size_t o = c3(d, in_, jn_);
-            topt = d.turb[o + mn.VI + 1];
-            tope = d.tdiss[o + mn.VI + 1];
-            const size_t oa_ = c3(d, in_ + IS, jn_), ob_ = c3(d, in_, jn_ + JS), oi = c3(d, in_ - IS, jn_);
-            const size_t oj = c3(d, in_, jn_ - JS);
+    const unsigned fi = 4u * (unsigned)nj2 * (unsigned)nkp, fj = 4u * (unsigned)nkp, base = fi + fj;
+    const unsigned off_l = 4u * lane, off_c = base + off_l, off_a = ip ? off_c + fi : off_c - fi, off_b = jp ? off_c + fj : off_c - fj;
+    const unsigned off_i = ip ? off_c - fi : off_c + fi, off_j = jp ? off_c - fj : off_c + fj;
+    const unsigned off_p = 4u * TKE_REC * lane, off_q = 16u * lane, off_h = 8u * lane;
+    const StripCol none{0, -1, 0, 0, 0};
+    StripCol c0 = none, c1 = none, c1j = none, c2m = none, c2, c2j;   // steps s, s+1 (and its -JS neighbour), s-1, s+2
+    unsigned o0 = 0, o1 = 0, op = 0;
+    TkeRaw raw[M];
+    TkeIn in[M];
+    auto located = [&]() {
+        c2 = strip_col<2>(m2);                                // kend unused
+        c2j = strip_col<2>(m2j);
+        request();
+    };
+    auto issue = [&](const StripCol &p, const StripCol &cn, const StripCol &cnj) {
+        c1 = cn;
+        c1j = cnj;
+        const int ci = cidx2 - 2 * dcol, l = l2 - 2;
+        if (c1.VI < 0) return;
+        o1 = (unsigned)ci * (unsigned)nkp;
+        const size_t o = (size_t)o1 + c1.KK + 1;
+        const gf32 *Tl = TW + o - (base >> 2), *El = EW + o - (base >> 2);
+        const size_t ho = ((size_t)(B - 1) * hcols + l) * nkp + c1.KK + 1;
+        const gf32 *Ht = (const gf32 *)(handt + ho), *He = (const gf32 *)(hande + ho);
+        const bool old_i = p.KK > c1.KK || p.VI < c1.VI, old_j = c1j.KK > c1.KK || c1j.VI < c1.VI;
+        const int n = c1.VI - c1.KK;
 #pragma unroll
-            for (int m = 0; m < 2; ++m) {
-                int k = mn.KK + 1 + lane + WAVE * m;
-                if (k <= mn.VI) {
-                    TkePre &p = pre[m];
-                    const gf32 *rr = d.planes + (o + k) * TKE_REC;
-                    p.c0 = ldg4(rr); p.c1 = ldg4(rr + 4); p.c2 = ldg4(rr + 8); p.c4 = ldg2(rr + 12);
-                    p.c3 = ldg4(d.planes + tke_rec4(d) + (o + k) * 4);
-                    p.ta = d.turb[oa_ + k]; p.ea = d.tdiss[oa_ + k];
-                    p.tb = d.turb[ob_ + k]; p.eb = d.tdiss[ob_ + k];
-                    p.nit = d.turb[oi + k]; p.nie = d.tdiss[oi + k];
-                    if (r > 0) { p.njt = d.turb[oj + k]; p.nje = d.tdiss[oj + k]; }
+        for (int m = 0; m < M; ++m) {
+            if (lane + WAVE * m < n) {
+                TkeRaw &q = raw[m];
+                const gf32 *P = lane_at(planes + (o + m * WAVE) * TKE_REC, off_p);
+                q.c0 = ldg4(P); q.c1 = ldg4(P + 4); q.c2 = ldg4(P + 8); q.c4 = ldg2(P + 12);
+                q.c3 = ldg4(lane_at(rec4 + (o + m * WAVE) * 4, off_q));
+                const gf32 *Tm = Tl + m * WAVE, *Em = El + m * WAVE;
+                q.ta = *lane_at(Tm, off_a); q.ea = *lane_at(Em, off_a);
+                q.tb = *lane_at(Tm, off_b); q.eb = *lane_at(Em, off_b);
+                if (old_i) { q.nit = *lane_at(Tm, off_i); q.nie = *lane_at(Em, off_i); }
+                if (old_j) { q.njt = *lane_at(Tm, off_j); q.nje = *lane_at(Em, off_j); }
+                if (from_prev) {
+                    q.ht = hand_get((const gu64 *)lane_at(Ht + m * WAVE * 2, off_h));
+                    q.he = hand_get((const gu64 *)lane_at(He + m * WAVE * 2, off_h));
                 }
             }
         }
     };
-    // row 0's -JS neighbours lie in the previous strip's last row: read after the wait
-    auto locate_prev = [&]() {
-        if (mn.adv) {
-            const size_t oj = c3(d, in_, jn_ - JS);
+    auto work_up = [&](int s, const StripCol &p) {
+        const StripCol &c = c1;
+        if (c.VI < 0) return;
+        const int sc = rowb + 4 * ((1 + 4 * (s & 1)) * len + low), l4 = 4 * len, f4 = 4 * fs;
+        const int si = rowb + 4 * ((8 - 4 * (s & 1)) * len + low + c.KK - p.KK);
+        const int sj = rowb - 4 * rs + 4 * ((8 - 4 * (s & 1)) * len + low + c.KK - c1j.KK);
 #pragma unroll
-            for (int m = 0; m < 2; ++m) {
-                int k = mn.KK + 1 + lane + WAVE * m;
-                if (k <= mn.VI) { pre[m].njt = ld_handoff(d.turb + oj + k); pre[m].nje = ld_handoff(d.tdiss + oj + k); }
+        for (int m = 0; m < M; ++m) {
+            const int t4 = 4 * (lane + WAVE * m), k = c.KK + 1 + lane + WAVE * m;
+            TkeRaw &q = raw[m];
+            TkeIn &a = in[m];
+            if (k <= c.VI) {
+                const bool wall = q.c2.w != 0.0f;
+                const float wt = q.c4.x < 0.001f ? 0.001f : q.c4.x, we = q.c4.y < 0.0000001f ? 0.0000001f : q.c4.y;
+                lds_at(sm, sc + t4) = q.c2.y;
+                lds_at(sm, sc + l4 + t4) = q.c3.x;
+                lds_at(sm, sc + 2 * l4 + t4) = q.c3.y;
+                lds_at(sm, sc + 3 * l4 + t4) = wall ? wt : TKE_NO_WALL;
+                lds_at(sm, sc + f4 + t4) = q.c2.z;
+                lds_at(sm, sc + f4 + l4 + t4) = q.c3.z;
+                lds_at(sm, sc + f4 + 2 * l4 + t4) = q.c3.w;
+                lds_at(sm, sc + f4 + 3 * l4 + t4) = wall ? we : TKE_NO_WALL;
+                const float aw = q.c0.x, as = q.c0.y, ae = q.c0.z, an = q.c0.w;
+                const float oi = ip ? ae : aw, oj = jp ? an : as;
+                a.ai = ip ? aw : ae; a.aj = jp ? as : an;
+                a.at = oi * q.ta; a.ae = oi * q.ea; a.bt = oj * q.tb; a.be = oj * q.eb;
+                a.w1 = q.c1.x; a.pro = q.c1.y; a.pbo = q.c1.z; a.w2 = q.c1.w; a.eps = q.c2.x;
+                a.nit = q.nit; a.nie = q.nie; a.njt = q.njt; a.nje = q.nje;
+                a.si = k > p.KK && k <= p.VI;
+                a.sj = k > c1j.KK && k <= c1j.VI;
+                a.li = a.si ? si + t4 : 0;
+                a.lj = a.sj ? sj + t4 : 0;
+            }
+        }
+        if (from_prev) {
+            const size_t ho = ((size_t)(B - 1) * hcols + (s - r)) * nkp;
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+                const int k = c.KK + 1 + lane + WAVE * m;
+                const bool need = k <= c.VI && k > c1j.KK && k <= c1j.VI;
+                hwait.wait(handt + ho + k, need, tag, raw[m].ht);
+                hwait.wait(hande + ho + k, need, tag, raw[m].he);
+                if (need) {
+                    in[m].njt = __uint_as_float((unsigned)raw[m].ht);
+                    in[m].nje = __uint_as_float((unsigned)raw[m].he);
+                }
+                in[m].sj = false;                             // the values are in njt, nje
+                in[m].lj = 0;
             }
         }
     };
-    // the chain wave's levels of the column located for step s (one lane writes)
-    auto put_info = [&](int s) {
-        if (lane == 0) {
-            int *si = sinfo + (s & 1) * 5 * ROWS;
-            si[r * 5] = mn.adv;
-            if (mn.adv) { si[r * 5 + 1] = mn.KK + 1; si[r * 5 + 2] = mn.VI; }
-        }
-    };
-    locate(0);
-    put_info(0);
-    if (r == 0) {
-        sw.wait(ROWS);
-        locate_prev();
-    }
-    // the outputs of a row's previous column (levels plo..pvi) are stored during
-    // the next step's assembly, before that step's publish
-    int plo = 1 << 30, pvi = -1;
-    size_t po = 0;
-    auto store_prev = [&]() {
-        gf32 *TW = d.turb + po, *EW = d.tdiss + po;
-        for (int k = plo + lane; k <= pvi; k += WAVE) { st_through(TW + k, sOT[k]); st_through(EW + k, sOE[k]); }
-    };
+    request();
+    located();
+    issue(none, c2, c2j);
+    located();
+    work_up(0, none);
+    c0 = c1; o0 = o1;
+    issue(c0, c2, c2j);
+    lds_barrier();                                            // the control wave's data of step 0
     for (int s = 0; s < nsteps; ++s) {
-        const bool act = mn.adv;
-        const Meta mt = mn;
-        const int i = in_, j = jn_;
-        int *si = sinfo + (s & 1) * 5 * ROWS;
-        const int *sp = sinfo + ((s - 1) & 1) * 5 * ROWS;
-        if (act) {
-            const int lo = mt.KK + 1, VI = mt.VI;
-            // levels of the two new neighbours that hold this sweep's values
-            const bool w_in = s - r >= 1;
-            int slo = 1 << 30, svi = -1;
-            if (r >= 1 && sp[(r - 1) * 5]) { slo = sp[(r - 1) * 5 + 1]; svi = sp[(r - 1) * 5 + 2]; }
-            const float *sOTs = sOT - (size_t)TKE_SLOTS * nkl, *sOEs = sOE - (size_t)TKE_SLOTS * nkl;
+        // phase 1: the new neighbours enter the sources of step s
+        if (c0.VI >= 0) {
 #pragma unroll
-            for (int m = 0; m < 2; ++m) {
-                int k = lo + lane + WAVE * m;
-                if (k <= VI) {
-                    const TkePre &p = pre[m];
-                    float tA = p.nit, eA = p.nie, tB = p.njt, eB = p.nje;
-                    if (w_in && k >= plo && k <= pvi) { tA = sOT[k]; eA = sOE[k]; }
-                    if (k >= slo && k <= svi) { tB = sOTs[k]; eB = sOEs[k]; }
-                    const float tW = (IS == 1) ? tA : p.ta, tE = (IS == 1) ? p.ta : tA;
-                    const float tS = (JS == 1) ? tB : p.tb, tN = (JS == 1) ? p.tb : tB;
-                    const float eW = (IS == 1) ? eA : p.ea, eE = (IS == 1) ? p.ea : eA;
-                    const float eS = (JS == 1) ? eB : p.eb, eN = (JS == 1) ? p.eb : eB;
-                    const float4 c0 = p.c0, c1 = p.c1, c2v = p.c2, c3v = p.c3;
-                    const float D1 = c0.x * tW + c0.y * tS + c0.z * tE + c0.w * tN + c1.x + c1.y + c1.z;
-                    const float D2 = c0.x * eW + c0.y * eS + c0.z * eE + c0.w * eN + c1.w + c2v.x;
-                    sD1[k] = D1; sD2[k] = D2;
-                    sC1[k] = c2v.y; sN1[k] = c3v.x; sP1[k] = c3v.y;
-                    sC2[k] = c2v.z; sN2[k] = c3v.z; sP2[k] = c3v.w; sWF[k] = c2v.w;
-                    sWT[k] = p.c4.x; sWE[k] = p.c4.y;
-                    if (k == lo) { sQ1[k] = D1 / c3v.x; sQ2[k] = D2 / c3v.z; }
+            for (int m = 0; m < M; ++m) {
+                if (lane + WAVE * m < c0.VI - c0.KK) {
+                    const TkeIn &a = in[m];
+                    float ti = lds_at(sm, a.li), ei = lds_at(sm, a.li + 4 * fs), tj = lds_at(sm, a.lj), ej = lds_at(sm, a.lj + 4 * fs);
+                    ti = a.si ? ti : a.nit; ei = a.si ? ei : a.nie;
+                    tj = a.sj ? tj : a.njt; ej = a.sj ? ej : a.nje;
+                    const float mti = a.ai * ti, mtj = a.aj * tj, mei = a.ai * ei, mej = a.aj * ej;
+                    const float D1 = (ip ? mti : a.at) + (jp ? mtj : a.bt) + (ip ? a.at : mti) + (jp ? a.bt : mtj) + a.w1 + a.pro + a.pbo;
+                    const float D2 = (ip ? mei : a.ae) + (jp ? mej : a.be) + (ip ? a.ae : mei) + (jp ? a.be : mej) + a.w2 + a.eps;
+                    const int q = rowb + 4 * (low + lane + WAVE * m);
+                    lds_at(sm, q) = D1;
+                    lds_at(sm, q + 4 * fs) = D2;
                 }
             }
-            if (lane == 0) { si[r * 5 + 3] = __float_as_int(topt); si[r * 5 + 4] = __float_as_int(tope); }
         }
-        store_prev();
-        plo = act ? mt.KK + 1 : 1 << 30;
-        pvi = act ? mt.VI : -1;
-        po = c3(d, i, j);
         lds_barrier();
-        if (r == ROWS - 1 && s > 0 && s % STRIP_PUBLISH == 0) strip_publish(mine, s, lane);
-        locate(s + 1);
-        if (s + 1 < nsteps) put_info(s + 1);
-        if (r == 0) {
-            sw.wait(s + 1 + ROWS);
-            locate_prev();
+        // phase 2, beside the recurrences
+        float xt[M], xe[M];
+        const StripCol done = c2m;                            // the column of step s-1, before its buffer is reused
+        const unsigned od = op;
+        if (done.VI >= 0) {
+            const int sn = rowb + 4 * ((8 - 4 * (s & 1)) * len + low + lane);
+#pragma unroll
+            for (int m = 0; m < M; ++m)
+                if (lane + WAVE * m < done.VI - done.KK) { xt[m] = lds_at(sm, sn + 4 * WAVE * m); xe[m] = lds_at(sm, sn + 4 * fs + 4 * WAVE * m); }
+        }
+        located();
+        if (s + 1 < nsteps) work_up(s + 1, c0);
+        c2m = c0; op = o0;
+        c0 = c1; o0 = o1;
+        if (s + 1 < nsteps) issue(c0, c2, c2j);
+        else c0 = none;
+        if (done.VI >= 0) {
+            const size_t o = (size_t)od + done.KK + 1;
+#pragma unroll
+            for (int m = 0; m < M; ++m)
+                if (lane + WAVE * m < done.VI - done.KK) {
+                    *(gf32 *)lane_at(TW + o + m * WAVE, off_l) = xt[m];
+                    *(gf32 *)lane_at(EW + o + m * WAVE, off_l) = xe[m];
+                }
         }
         lds_barrier();                                        // the recurrence outputs are ready
     }
-    store_prev();
-    if (r == ROWS - 1) strip_publish(mine, nsteps, lane);
+    if (c2m.VI >= 0) {
+        const size_t o = (size_t)op + c2m.KK + 1;
+        const float *x = sm + (size_t)r * rs + (4 + 4 * ((nsteps - 1) & 1)) * len + low;
+        for (int t = lane; t < c2m.VI - c2m.KK; t += WAVE) { TW[o + t] = x[t]; EW[o + t] = x[fs + t]; }
+    }
 }
 
-static inline int lds_slot_h(int nkp) { return (nkp + 2 * SLOT_PAD) | 1; }
 // raises a kernel's dynamic LDS limit to bytes (above the default 64 KB; the
 // device's is 160 KB) the first time a launch needs it; 1 on failure
 static inline int lds_limit(const void *kern, size_t bytes) {
@@ -3244,24 +3177,6 @@ static inline int lds_limit(const void *kern, size_t bytes) {
     set[q] = bytes;
     if (q == n) ++n;
     return 0;
-}
-// Rows of a strip.  A strip is a workgroup of rows + 2 waves; fewer rows mean
-// less work per step and CU, more strips and (a sweep's path is its column
-// range plus rows per strip) about the same number of steps.  Ten rows while
-// all strips of the launch find a CU of their own (400 x 400 city, one
-// situation: pressure, U and V sweeps 1.33, 1.41 and 1.38 ms against 1.42, 1.48
-// and 1.48 with 14), else 14 (eight situations: 1.62, 2.04 and 1.71 ms against
-// 1.80, 2.16 and 1.91 with ten).  Short sweeps, whose path is mostly the fill of
-// their first strips, take seven (25 rows: 60 against 65 us).  swap: the
-// pressure sweep, whose rows run along i.
-static int strip_rows(const Dom *hd, int nsit, bool swap) {
-    long n = 0, longest = 0;
-    for (int q = 0; q < nsit; ++q) {
-        const int nb = (swap ? hd[q].nii : hd[q].njj) - 2;
-        n += (nb + 9) / 10;
-        longest = max(longest, (long)nb);
-    }
-    return n > 256 ? 14 : longest > 40 ? 10 : 7;
 }
 typedef void (*PressureKernel)(const Dom *, int, int, int);
 static PressureKernel pressure_strip(const Dom *hd, int nsit) {
@@ -3286,7 +3201,41 @@ static inline size_t ml_strip_lds(const Dom *hd, int nsit, bool w, int rows) {
     }
     return m;
 }
+static size_t ml_strip_lds_w(const Dom *hd, int nsit, int rows) { return ml_strip_lds(hd, nsit, true, rows); }
+static size_t tke_strip_lds(const Dom *hd, int nsit, int rows) {
+    size_t m = 0;
+    for (int q = 0; q < nsit; ++q)
+        m = max(m, sizeof(float) * (size_t)rows * strip_stride(TKE_ARRAYS, strip_len(0, hd[q].nact)) + 64 * sizeof(int4) + 16);
+    return m;
+}
 typedef void (*StripKernel)(const Dom *, int, int);
+static StripKernel tke_strip(const Dom *hd, int nsit) {
+    int n = 0;
+    for (int q = 0; q < nsit; ++q) n = max(n, hd[q].nact);
+    return n <= WAVE ? k_tke_strip<1> : k_tke_strip<2>;
+}
+// Rows of a strip.  A strip is a workgroup of rows + 2 waves; fewer rows mean
+// less work per step and CU, more strips and (a sweep's path is its column
+// range plus rows per strip) about the same number of steps.  Ten rows while
+// all strips of the launch find a CU of their own (400 x 400 city, one
+// situation: pressure, U and V sweeps 1.33, 1.41 and 1.38 ms against 1.42, 1.48
+// and 1.48 with 14), else 14 (eight situations: 1.62, 2.04 and 1.71 ms against
+// 1.80, 2.16 and 1.91 with ten).  Short sweeps, whose path is mostly the fill of
+// their first strips, take seven (25 rows: 60 against 65 us).  swap: the
+// pressure sweep, whose rows run along i; lds: the kernel's LDS at a row count
+// (tall columns take fewer rows).
+#define LDS_BYTES (160 * 1024)
+static int strip_rows(const Dom *hd, int nsit, bool swap, size_t (*lds)(const Dom *, int, int)) {
+    long n = 0, longest = 0;
+    for (int q = 0; q < nsit; ++q) {
+        const int nb = (swap ? hd[q].nii : hd[q].njj) - 2;
+        n += (nb + 9) / 10;
+        longest = max(longest, (long)nb);
+    }
+    int rows = n > 256 ? 14 : longest > 40 ? 10 : STRIP_ROWS_MIN;
+    while (rows > STRIP_ROWS_MIN && lds(hd, nsit, rows) > LDS_BYTES) rows = rows > 10 ? 10 : STRIP_ROWS_MIN;
+    return rows;
+}
 template <int COMP, int WFIX, int KIND>
 static StripKernel ml_strip(const Dom *hd, int nsit) {
     int n = 0;
@@ -3299,7 +3248,7 @@ static int ml_strip_limit(int model, const Dom *hd, int nsit) {
     for (int q = 0; q < nsit; ++q) w8 = w8 && hd[q].simd == 8;
     const StripKernel k = model == 2 ? ml_strip<COMP, 0, 1>(hd, nsit) : model == 0 ? ml_strip<COMP, 0, 2>(hd, nsit) :
                           w8 ? ml_strip<COMP, 8, 0>(hd, nsit) : ml_strip<COMP, 0, 0>(hd, nsit);
-    return lds_limit((const void *)k, ml_strip_lds(hd, nsit, COMP == 2, strip_rows(hd, nsit, false)));
+    return lds_limit((const void *)k, ml_strip_lds(hd, nsit, COMP == 2, strip_rows(hd, nsit, false, ml_strip_lds_w)));
 }
 // longest diagonal t over the situations; the pressure sweep runs a over j
 // (outer) and b over i, the momentum sweeps a over i and b over j
@@ -3363,7 +3312,8 @@ static int launch_iteration(const Dom *hd, int nsit, const Dom *dd, int iter, in
         nkp = max(nkp, hd[q].nkp); nj2 = max(nj2, hd[q].nj2);
     }
     const unsigned Z = (unsigned)nsit;
-    const int rows_p = strip_rows(hd, nsit, true), rows = strip_rows(hd, nsit, false);
+    const int rows_p = strip_rows(hd, nsit, true, pressure_strip_lds);
+    const int rows = strip_rows(hd, nsit, false, ml_strip_lds_w), rows_t = strip_rows(hd, nsit, false, tke_strip_lds);
     int kb = (nk + 63) / 64;
     int IS = 1, JS = 1;
     switch (iter % 4) {
@@ -3380,8 +3330,7 @@ static int launch_iteration(const Dom *hd, int nsit, const Dom *dd, int iter, in
         if (d0.model == 2) {
             bad |= lds_limit((const void *)k_tke_coef,
                              sizeof(float) * 5 * (nkp | 1) * COEF_COLS + sizeof(int) * (TKE_SCOL * COEF_COLS + 4));
-            bad |= lds_limit((const void *)k_tke_strip, sizeof(float) * ((size_t)TKE_SLOTS * ROWS * lds_slot_h(nkp) + WAVE * CH) +
-                                                            sizeof(int) * (10 * ROWS + 4));
+            bad |= lds_limit((const void *)tke_strip(hd, nsit), tke_strip_lds(hd, nsit, rows_t));
         }
         if (bad) return (int)hipErrorInvalidValue;
     }
@@ -3481,11 +3430,10 @@ static int launch_iteration(const Dom *hd, int nsit, const Dom *dd, int iter, in
             if (lds_limit((const void *)k_tke_coef, shm_c)) return (int)hipErrorInvalidValue;
             L.go(FAM_COEF, [&] { hipLaunchKernelGGL(k_tke_coef, dim3(nblk_t, 1, Z), dim3(4 * WAVE), shm_c, s, dd); });
             int nst = 0;
-            for (int q = 0; q < nsit; ++q) nst = max(nst, (hd[q].njj - 1 - 2 + ROWS) / ROWS);
-            const size_t shm_k = sizeof(float) * ((size_t)TKE_SLOTS * ROWS * lds_slot_h(nkp) + WAVE * CH) + sizeof(int) * (10 * ROWS + 4);
-            if (lds_limit((const void *)k_tke_strip, shm_k)) return (int)hipErrorInvalidValue;
+            for (int q = 0; q < nsit; ++q) nst = max(nst, (hd[q].njj - 3 + rows_t) / rows_t);
+            const size_t shm_k = tke_strip_lds(hd, nsit, rows_t);
             L.go(FAM_TKE, [&] {
-                hipLaunchKernelGGL(k_tke_strip, dim3(nst, 1, Z), dim3(STRIP_WAVES * WAVE), shm_k, s, dd, IS, JS);
+                hipLaunchKernelGGL(tke_strip(hd, nsit), dim3(nst, 1, Z), dim3((rows_t + 2) * WAVE), shm_k, s, dd, IS, JS);
             });
         } else {
             size_t shm_t = sizeof(float) * 12 * nkp;
