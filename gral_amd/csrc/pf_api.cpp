@@ -616,6 +616,10 @@ static int put_vec(gral_pf_handle *h, T *dptr, const std::vector<T> &v) {
     return 0;
 }
 
+// columns of more than 126 levels: a batch holds situations of one kind (see
+// gral_pf_batch_create), since such a situation may run per-diagonal
+static bool tall(const gral_pf_handle *h) { return h->kadvmax + 2 > 128; }
+
 extern "C" int gral_pf_prepare(gral_pf_handle *h, const gral_pf_params *p) {
     if (!h) return GRAL_PF_EINVAL;
     // a failed prepare leaves the handle unprepared: the device state of an
@@ -697,7 +701,6 @@ extern "C" int gral_pf_prepare(gral_pf_handle *h, const gral_pf_params *p) {
     const char *sw = std::getenv("GRAL_PF_SWEEP");
     d.tiled = 2;
     if (sw && std::strcmp(sw, "diag") == 0) d.tiled = 0;
-    if (h->kadvmax + 2 > 128) d.tiled = 0;   // the strip kernels hold at most 128 levels per column
     {
         // strip synchronisation: header + one block per sweep kind (pressure, U, V, W, TKE)
         d.sync_stride = 64;
@@ -715,34 +718,52 @@ extern "C" int gral_pf_prepare(gral_pf_handle *h, const gral_pf_params *p) {
                 if (h->cutk[c] != 0) d.nlow = std::max(d.nlow, (int)h->kk[c]);
             }
         d.hand_cols = std::max(h->nii, h->njj);
-        if (d.tiled) {
-            d.hand_words = (size_t)(std::max(h->nii, h->njj) / STRIP_ROWS_MIN + 1) * d.hand_cols * d.nkp;
-            if ((rc = dalloc(h, &d.hand, 2 * d.hand_words))) return rc;
-            HIPCHK(h, hipMemsetAsync(d.hand, 0, 2 * d.hand_words * sizeof(unsigned long long), h->stream));
-        }
+        d.hand_words = (size_t)(d.hand_cols / STRIP_ROWS_MIN + 1) * d.hand_cols * d.nkp;
     }
+    // The strips hold 256 levels a column, 127 of them above the ground: the W
+    // sweep deals a column to at most 4 groups of 64 lanes, the others to 2
+    if (h->kadvmax + 2 > 256 || d.nact + 1 > 128) d.tiled = 0;
     d.planes = nullptr;
     d.rec3 = nullptr;
     d.wcol = nullptr;
     d.ptab[0] = d.ptab[1] = d.ttab[0] = d.ttab[1] = nullptr;
+    // the strips' buffers: hand-off words, coefficient records, pressure tables
+    auto strip_alloc = [&]() -> int {
+        int e;
+        // k-eps: the momentum sweeps' records (12 or 8 floats per cell, then {C,
+        // denominator, P} at 12..14) and, in turn, the TKE sweep's 20 floats per
+        // cell share the planes; mixing length and no diffusion: 12 (U, V) or 8
+        // (W) floats per cell, then 3.  The U/V wall terms follow.
+        const size_t rec = (p->turbulence_model == 2) ? 20 : 15;
+        float *pl, *tab[4];
+        if ((e = dalloc(h, &d.hand, 2 * d.hand_words)) || (e = dalloc(h, &pl, rec * n3 + n2))) return e;
+        for (auto &q : tab)
+            if ((e = dalloc(h, &q, n3))) return e;
+        d.planes = pl;
+        d.rec3 = pl + 12 * n3;
+        d.wcol = pl + rec * n3;
+        d.ptab[0] = tab[0]; d.ttab[0] = tab[1]; d.ptab[1] = tab[2]; d.ttab[1] = tab[3];
+        return 0;
+    };
     if (d.tiled) {
-        if (p->turbulence_model == 2) {
-            // the momentum sweeps' records (12 or 8 floats per cell, then
-            // {C, denominator, P} at 12..14) and, in turn, the TKE sweep's 20
-            // floats per cell share the planes; the U/V wall terms follow
-            float *pl;
-            if ((rc = dalloc(h, &pl, 20 * n3 + n2))) return rc;
-            d.planes = pl;
-            d.rec3 = pl + 12 * n3;
-            d.wcol = pl + 20 * n3;
+        const size_t mark = h->dev.size(), bytes = h->dev_bytes;
+        rc = strip_alloc();
+        if (rc && !tall(h)) return rc;
+        if (rc) {
+            // a tall column's situation whose strips find no memory still runs
+            // per-diagonal
+            (void)hipGetLastError();
+            for (; h->dev.size() > mark; h->dev.pop_back()) (void)hipFree(h->dev.back());
+            h->dev_bytes = bytes;
+            h->err.clear();
+            d.hand = nullptr;
+            d.planes = d.rec3 = d.wcol = nullptr;
+            d.ptab[0] = d.ptab[1] = d.ttab[0] = d.ttab[1] = nullptr;
+            d.tiled = 0;
         }
-        if (p->turbulence_model != 2) {          // mixing length and no diffusion
-            float *pl;
-            if ((rc = dalloc(h, &pl, 15 * n3 + n2))) return rc;
-            d.planes = pl;                       // 12 (U, V) or 8 (W) floats per cell
-            d.rec3 = pl + 12 * n3;               // then 3 per cell
-            d.wcol = pl + 15 * n3;               // then 1 per column
-        }
+    }
+    if (d.tiled) {
+        HIPCHK(h, hipMemsetAsync(d.hand, 0, 2 * d.hand_words * sizeof(unsigned long long), h->stream));
         // PIMP/TERMP of the pressure TDMA for every column, in the reference's
         // row order (fresh row arrays per j row, columns in i1 order for IS=+1 and
         // IS=-1), so the stale top value PIMP[VI+1] is part of the table
@@ -771,11 +792,7 @@ extern "C" int gral_pf_prepare(gral_pf_handle *h, const gral_pf_params *p) {
                     }
                 }
             });
-            float *dp, *dt;
-            if ((rc = dalloc(h, &dp, n3)) || (rc = dalloc(h, &dt, n3)) || (rc = put_vec(h, dp, tp)) || (rc = put_vec(h, dt, tt)))
-                return rc;
-            d.ptab[v] = dp;
-            d.ttab[v] = dt;
+            if ((rc = put_vec(h, const_cast<float *>(d.ptab[v]), tp)) || (rc = put_vec(h, const_cast<float *>(d.ttab[v]), tt))) return rc;
         }
     }
     // per-column metadata of the tiled kernels: KK, VI, KSTART | adv<<16 | vegp<<17,
@@ -1665,7 +1682,7 @@ extern "C" int gral_pf_batch_create(gral_pf_handle *const *handles, int32_t n, g
         for (int r = 0; r < q; ++r)
             if (handles[r] == handles[q]) return GRAL_PF_EINVAL;
         const Dom &a = handles[0]->d, &c = handles[q]->d;
-        if (a.model != c.model || a.tiled != c.tiled) return GRAL_PF_EINVAL;
+        if (a.model != c.model || a.tiled != c.tiled || tall(handles[0]) != tall(handles[q])) return GRAL_PF_EINVAL;
     }
     gral_pf_batch *b = new (std::nothrow) gral_pf_batch();
     if (!b) return GRAL_PF_ENOMEM;
@@ -1697,7 +1714,7 @@ extern "C" int gral_pf_batch_add(gral_pf_batch *b, gral_pf_handle *h) {
     for (auto *x : b->pending)
         if (x == h) return bfail(b, GRAL_PF_EINVAL, "batch add: the situation is already queued");
     const gral_pf_handle *ref = !b->hs.empty() ? b->hs[0] : (!b->pending.empty() ? b->pending[0] : nullptr);
-    if (ref && (ref->d.model != h->d.model || ref->d.tiled != h->d.tiled))
+    if (ref && (ref->d.model != h->d.model || ref->d.tiled != h->d.tiled || tall(ref) != tall(h)))
         return bfail(b, GRAL_PF_EINVAL, "batch add: situations of a batch must share the turbulence model and sweep kind");
     const size_t need = b->hs.size() + b->pending.size() + 1;
     if (need > b->dd_cap) {

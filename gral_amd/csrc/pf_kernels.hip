@@ -3163,15 +3163,15 @@ __global__ __launch_bounds__(STRIP_WAVES * WAVE) void k_tke_strip(const Dom *__r
 // device's is 160 KB) the first time a launch needs it; 1 on failure
 static inline int lds_limit(const void *kern, size_t bytes) {
     static std::mutex mu;
-    static const void *keys[32];
-    static size_t set[32];
+    static const void *keys[64];                 // more than there are strip and coefficient kernels
+    static size_t set[64];
     static int n = 0;
     if (bytes <= 65536) return 0;
     std::lock_guard<std::mutex> g(mu);
     int q = 0;
     while (q < n && keys[q] != kern) ++q;
     if (q < n && bytes <= set[q]) return 0;
-    if (q == n && n == 32) return 1;
+    if (q == n && n == 64) return 1;
     if (hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess) return 1;
     keys[q] = kern;
     set[q] = bytes;
@@ -3240,6 +3240,8 @@ template <int COMP, int WFIX, int KIND>
 static StripKernel ml_strip(const Dom *hd, int nsit) {
     int n = 0;
     for (int q = 0; q < nsit; ++q) n = max(n, (COMP == 2 ? hd[q].nlow : 0) + hd[q].nact + 1);
+    if constexpr (COMP == 2)                                  // buildings add to the W sweep's columns
+        if (n > 2 * WAVE) return n <= 3 * WAVE ? k_ml_strip<COMP, WFIX, KIND, 3> : k_ml_strip<COMP, WFIX, KIND, 4>;
     return n <= WAVE ? k_ml_strip<COMP, WFIX, KIND, 1> : k_ml_strip<COMP, WFIX, KIND, 2>;
 }
 template <int COMP>
@@ -3391,7 +3393,7 @@ static int launch_iteration(const Dom *hd, int nsit, const Dom *dd, int iter, in
             nblk = max(nblk, ((na * nb + COEF_COLS - 1) / COEF_COLS + NXCD - 1) / NXCD * NXCD);
             nst = max(nst, (ib - ia + rows) / rows);
         }
-        size_t shm_c = sizeof(float) * 3 * (nkp | 1) * COEF_COLS + sizeof(int) * (SCOL * COEF_COLS + 4);
+        const size_t shm_c = sizeof(float) * 3 * (nkp | 1) * COEF_COLS + sizeof(int) * (SCOL * COEF_COLS + 4);
         L.go(FAM_COEF, [&] { hipLaunchKernelGGL(coef, dim3(nblk, 1, Z), dim3(4 * WAVE), shm_c, s, dd, is, js); });
         const size_t shm_t = ml_strip_lds(hd, nsit, oa == 2 && ia == 2, rows);
         L.go(fam, [&] { hipLaunchKernelGGL(strip, dim3(nst, 1, Z), dim3((rows + 2) * WAVE), shm_t, s, dd, is, js); });

@@ -16,8 +16,10 @@ from gral_amd import domain
 from tests.helpers import FIELDS, KE_FIELDS, diff_report
 
 
-def _city(nii, njj, vcf, model=1, width=8, hmax=14.0, dz1=1.0, stretch=1.01, direction=250.0, seed=5):
+def _city(nii, njj, vcf, model=1, width=8, hmax=14.0, dz1=1.0, stretch=1.01, direction=250.0, seed=5, tower=None):
     bl = domain.city_buildings(nii, njj, 2.0, seed, density=0.2, fmin=4.0, fmax=12.0, hmin=3.0, hmax=hmax, margin=2)
+    if tower:
+        bl.append(domain.Building(6, 9, 5, 8, tower))
     c = domain.build_case(f"s{nii}x{njj}x{vcf}", nii, njj, bl, dx=2.0, dz1=dz1, stretch=stretch, vertcellsff=vcf, speed10=4.0,
                           direction=direction, z0=0.5, turbulence_model=model, iterations=3)
     c.simd_width = width
@@ -42,6 +44,10 @@ CASES = [
     dict(nii=12, njj=11, vcf=63), dict(nii=11, njj=12, vcf=64, model=2), dict(nii=12, njj=13, vcf=65, width=16), dict(nii=13, njj=12, vcf=66, model=0),
     # W columns over one group: 40 levels above buildings of up to 35
     dict(nii=30, njj=29, vcf=40, hmax=40.0), dict(nii=29, njj=30, vcf=40, hmax=40.0, model=2),
+    # towers: W columns over two and three groups (KADVMAX 127 and 190 and one level to either side)
+    dict(nii=16, njj=15, vcf=48, tower=118.0), dict(nii=15, njj=16, vcf=49, tower=118.0, model=2), dict(nii=15, njj=15, vcf=50, tower=118.0, width=16),
+    dict(nii=15, njj=14, vcf=60, tower=263.0), dict(nii=14, njj=15, vcf=61, tower=263.0, model=2), dict(nii=14, njj=14, vcf=62, tower=263.0, width=16),
+    dict(nii=14, njj=13, vcf=63, tower=263.0, model=0),
 ]
 
 
@@ -65,3 +71,26 @@ def test_many_strips():
         ref = pf.run(cases[q], iterations=2)
         for f, r in diff_report(got[q], ref, FIELDS).items():
             assert r["n_bits_differ"] == 0, (q, f, r)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("model", [1, 2])
+def test_tower_without_strip_memory(monkeypatch, model):
+    """Columns over 126 levels run per-diagonal when the strips' buffers do not fit, and a batch takes no
+    such columns together with lower ones."""
+    from gral_amd import pf
+    from oracle import pyoracle
+    c = _city(16, 15, 50, tower=118.0, model=model)
+    monkeypatch.setenv("GRAL_PF_DEVICE_MB", "4")
+    with pf.PrognosticFlowfield(c) as s:
+        s.prepare(3)
+        s.iterate(3)
+        assert s.timing()["launches"] > 200                   # a launch per anti-diagonal and sweep
+        got = {**s.download(), "stats": s.finish()}
+    monkeypatch.delenv("GRAL_PF_DEVICE_MB")
+    _check(c, got, pyoracle.run(c, iterations=3))
+    with pf.PrognosticFlowfield(c) as a, pf.PrognosticFlowfield(_city(16, 15, 50, model=model)) as b:
+        a.prepare(3)
+        b.prepare(3)
+        with pytest.raises(RuntimeError):
+            pf.Batch([a, b])
