@@ -41,6 +41,7 @@ extern "C" int pf_launch_iteration(const Dom *hd, int nsit, const Dom *dd, int i
                                    long long *launches, Probe *probe);
 extern "C" int pf_fill_u32(unsigned *p, size_t n, unsigned v, hipStream_t s);
 extern "C" int pf_launch_diagnostic(const DiagArgs *ga, int iterations, hipStream_t s);
+extern "C" size_t pf_diag_hand(int nii, int njj, int nkh);
 extern "C" int pf_launch_gff(const GffArgs *ga, hipStream_t s);
 extern "C" int pf_launch_wind(const WindArgs *wa, hipStream_t s);
 extern "C" int pf_launch_mass(const Dom *dd, int nsit, int nblk, double *partial, double *out, hipStream_t s);
@@ -1539,6 +1540,9 @@ extern "C" int gral_pf_momentum_sweep(gral_pf_handle *h, int32_t comp) {
     HIPCHK(h, hipEventRecord(h->ev1, h->stream));
     if (e) return fail(h, GRAL_PF_EDEVICE, std::string("momentum_sweep: launch failed: ") + hipGetErrorString((hipError_t)e));
     HIPCHK(h, hipEventSynchronize(h->ev1));
+    int serr = 0;
+    HIPCHK(h, hipMemcpy(&serr, h->d.sync, sizeof(int), hipMemcpyDeviceToHost));
+    if (serr) return fail(h, GRAL_PF_EDEVICE, "momentum_sweep: a strip wait timed out (results invalid)");
     float ms = 0;
     HIPCHK(h, hipEventElapsedTime(&ms, h->ev0, h->ev1));
     h->timing = gral_pf_timing{};
@@ -1939,11 +1943,30 @@ extern "C" int gral_pf_diagnostic(gral_pf_handle *h, int32_t flow_field_level, i
     g.p_in = (const float *)p[3]; g.p_bot = (const float *)p[4];
     g.kk = (const int *)p[5]; g.adv = (const uint8_t *)p[6];
     g.uk = (float *)p[7]; g.vk = (float *)p[8]; g.wk = (float *)p[9]; g.dpm = (float *)p[10]; g.div = (float *)p[11];
+    // the strips' hand-off words; without memory for them the sweeps run per diagonal
+    const size_t hb = pf_diag_hand(h->nii, h->njj, (int)nkh) * sizeof(unsigned long long) + DG_SYNC * sizeof(int);
+    if (hb > DG_SYNC * sizeof(int)) {
+        void *q = nullptr;
+        if (hipMalloc(&q, hb) == hipSuccess) {
+            tmp.push_back(q);
+            if (pf_fill_u32((unsigned *)q, hb / sizeof(unsigned), 0u, h->stream)) {
+                cleanup();
+                return fail(h, GRAL_PF_EDEVICE, "diagnostic: fill failed");
+            }
+            g.hand = (unsigned long long *)q;
+            g.sync = (int *)((char *)q + hb) - DG_SYNC;
+        } else (void)hipGetLastError();
+    }
     int iters = (flow_field_level == 2) ? 10 : 5;
-    int e = pf_launch_diagnostic(&g, iters, h->stream);
+    int e = pf_launch_diagnostic(&g, iters, h->stream), serr = 0;
+    if (!e && g.sync && hipMemcpyAsync(&serr, g.sync, sizeof(int), hipMemcpyDeviceToHost, h->stream) != hipSuccess) e = 1;
     if (e || hipStreamSynchronize(h->stream) != hipSuccess) {
         cleanup();
         return fail(h, GRAL_PF_EDEVICE, "diagnostic: kernel launch failed");
+    }
+    if (serr) {
+        cleanup();
+        return fail(h, GRAL_PF_EDEVICE, "diagnostic: a strip wait timed out (results invalid)");
     }
     float *dst[4] = {h->uk.data(), h->vk.data(), h->wk.data(), h->dpm.data()};
     for (int q = 0; q < 4; ++q)

@@ -153,7 +153,10 @@ struct DiagArgs {
     const int *kk;                 // [nii+2][njj+2]
     const uint8_t *adv;
     float *uk, *vk, *wk, *dpm, *div;   // [nii+2][njj+2][nkh]
+    int *sync;                     // [DG_SYNC] strip synchronisation: error flag, 0, then a ticket per sweep
+    unsigned long long *hand;      // [pf_diag_hand()] hand-off words, or null: one launch per anti-diagonal
 };
+#define DG_SYNC 16
 
 // Buffers of one step of the adjoint (pf_adjoint.hip), each [nii+2][njj+2][nkp]
 // except the per-column source table.

@@ -13,6 +13,7 @@
 //                      parallel (lanes over k), stages them in LDS, and one lane
 //                      runs the Thomas recurrences, which are serial in k.
 // This replays the reference's deterministic (single-thread) order exactly.
+#include <cmath>
 #include <mutex>
 #include "pf_device.h"
 
@@ -2522,6 +2523,205 @@ __global__ __launch_bounds__(STRIP_WAVES * WAVE) void k_pressure_strip(const Dom
     if (lane == 0 && rmax > 0.0f && slot >= 0 && rsl >= 0 && rsl < d.resid_cap) atomicMax((unsigned *)&d.resid[rsl], __float_as_uint(rmax));
 }
 
+static inline int lds_limit(const void *kern, size_t bytes);
+// ------------------------------------------------------------------------
+// Strips for sweeps whose column system is two first-order recurrences (the
+// diagnostic pressure sweep, the transposed momentum sweep): the strip and
+// hand-off scheme of k_ml_strip, with the LDS arrays of a row indexed by the level
+// itself and 0 outside a column's levels, so that a neighbour's value needs no
+// offset and the recurrences of all rows run over the same chunks.  R row waves
+// own a sweep row each, wave R runs the recurrences (lane = row) and hands the
+// last row's results on; the steps and phases are those of k_ml_strip, without
+// a control wave: a row leaves its column's levels in LDS a step ahead.  Bound by
+// the recurrences.  OP supplies the operands and the recurrences (DgOp, MomOp);
+// M: 64-level groups of a column.
+// ------------------------------------------------------------------------
+struct LineSweep {
+    int ni, nj;                  // rows, steps of the sweep
+    int c0, di, dj;              // column index of (0, 0), its change per row and per step
+    int nk;                      // levels of a stored column
+    int *sync;                   // [0] error flag, [1] tag base, [ticket] 0 before the launch
+    int ticket, kind;            // kind: names the sweep in the tag
+    unsigned long long *hand;    // [strips][nj][nk]
+};
+struct LineCol { int lo, hi, x; };                             // its levels (lo > hi: none) and the OP's own datum
+typedef int __attribute__((address_space(4))) ci32;
+__host__ __device__ inline int line_len(int nk) { return (nk + 2 * CHK - 1) / CHK * CHK; }      // one spare chunk
+template <class OP>
+__host__ __device__ inline int line_arrays() { return 3 + 2 * OP::NBUF; }
+template <class OP>
+static size_t line_lds(int nk, int rows) {
+    const int len = line_len(nk);
+    return sizeof(float) * ((size_t)rows * strip_stride(line_arrays<OP>(), len) + (size_t)OP::NTAB * len) + 32 * sizeof(int4) + 16;
+}
+template <class OP, int M>
+__global__ __launch_bounds__(STRIP_WAVES * WAVE) void k_line_strip(OP op, LineSweep w) {
+    extern __shared__ __align__(16) float sm[];
+    const int nk = w.nk, len = line_len(nk), rs = strip_stride(line_arrays<OP>(), len);
+    const int R = blockDim.x / WAVE - 1;
+    const int nstrip = (w.ni + R - 1) / R, nsteps = w.nj + R - 1;
+    const int r = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
+    gi32 *sync = (gi32 *)w.sync;
+    // per row: D (or what the recurrences make of it), the results of even and odd
+    // steps, the operands of even and odd steps
+    float *tab = sm + (size_t)R * rs;                         // [NTAB][len] operands that depend on the level alone
+    int4 *sinfo = (int4 *)(tab + OP::NTAB * len);             // [2][16] levels of the rows' columns by step parity
+    int *sctl = (int *)(sinfo + 32);
+    const LineCol none{1 << 20, -1, 0};
+    if (threadIdx.x == 0) sctl[0] = __hip_atomic_fetch_add(&sync[w.ticket], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (threadIdx.x < 32) sinfo[threadIdx.x] = make_int4(none.lo, none.hi, 0, 0);
+    for (int k = threadIdx.x; k < OP::NTAB * len; k += blockDim.x) tab[k] = (k % len < nk) ? op.table(k / len, k % len) : 0.0f;
+    __syncthreads();
+    const int B = __builtin_amdgcn_readfirstlane(sctl[0]);
+    if (B >= nstrip) return;                                  // uniform over the workgroup
+    const unsigned tag = 8u * (unsigned)sync[1] + (unsigned)w.kind;
+    gu64 *hand = (gu64 *)w.hand;
+    if (r == R) {                                             // chain wave
+        __builtin_amdgcn_s_setprio(3);
+        float *L = sm + (size_t)(lane < R ? lane : 0) * rs;
+        const float *xl = sm + (size_t)(R - 1) * rs + len;
+        gu64 *h = hand + ((size_t)B * w.nj - R) * nk;         // + s*nk: the last row's column of step s - 1
+        const bool send = B + 1 < nstrip;
+        int lo = none.lo, hi = none.hi;
+        auto send_last = [&](int s) {
+            if (!send || s < R) return;                       // l = s - R is a step of the last row
+            const int a = __builtin_amdgcn_readlane(lo, R - 1), b = __builtin_amdgcn_readlane(hi, R - 1);
+            for (int k = lane; k < nk; k += WAVE)
+                hand_put(h + (size_t)s * nk + k, (k >= a && k <= b) ? xl[((s - 1) & 1) * len + k] : 0.0f, tag);
+        };
+        lds_barrier();                                        // the rows' operands and levels of step 0
+        for (int s = 0; s < nsteps; ++s) {
+            const int4 si = sinfo[(s & 1) * 16 + (lane & 15)];
+            send_last(s);
+            lo = lane < R ? si.x : none.lo;
+            hi = lane < R ? si.y : none.hi;
+            const bool on = lo <= hi;
+            // chunks of the lowest bottom, the highest bottom and the highest top
+            const int NC = len / CHK;
+            const int clo = NC - __builtin_amdgcn_readfirstlane(row_max(on ? NC - lo / CHK : 0));
+            const int chi = __builtin_amdgcn_readfirstlane(row_max(on ? lo / CHK : 0));
+            const int ct = __builtin_amdgcn_readfirstlane(row_max(on ? hi / CHK : 0));
+            lds_barrier();                                    // the rows' sources are assembled
+            if (on) op.chain(L, L + (1 + (s & 1)) * len, L + (3 + (s & 1) * OP::NBUF) * len, tab, len, lo, clo, chi, ct);
+            lds_barrier();                                    // the recurrences are done
+        }
+        send_last(nsteps);
+        return;
+    }
+    const int b = B * R + r;
+    const bool row_ok = b < w.ni, from_prev = r == 0 && B > 0;
+    HandWait hwait{sync, wall_clock64() + STRIP_TIMEOUT_TICKS, false};
+    const int rowb = 4 * r * rs, c00 = w.c0 + b * w.di;
+    LineCol q2 = none, c2 = none, c1 = none, c0 = none, cm = none;    // requested, steps s+2, s+1, s, s-1
+    int l2 = -r - 1;                                          // step (of this row) q2 belongs to
+    typename OP::Raw raw[M];
+    typename OP::In in[M];
+    unsigned long long hw[M];
+    float vin[M] = {};                                        // row 0: the new values of the previous strip's last row
+    auto located = [&]() {                                    // q2 arrives, the next is requested
+        c2 = q2;
+        ++l2;
+        q2 = none;
+        if (row_ok && l2 >= 0 && l2 < w.nj) q2 = op.levels(c00 + l2 * w.dj);
+    };
+    auto issue = [&]() {                                      // loads of the column at c2, l = l2 - 1
+        c1 = c2;
+        if (c1.lo > c1.hi) return;
+        const int l = l2 - 1, c = c00 + l * w.dj;
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+            const int k = lane + WAVE * m;
+            if (k >= c1.lo && k <= c1.hi) op.load(raw[m], c, w.di, w.dj, k);
+            if (from_prev && k < nk) hw[m] = hand_get(hand + ((size_t)(B - 1) * w.nj + l) * nk + k);
+        }
+    };
+    auto work_up = [&](int s) {                               // c1 is the column of step s
+        if (lane == 0) sinfo[(s & 1) * 16 + r] = make_int4(c1.lo, c1.hi, 0, 0);
+        if (c1.lo > c1.hi) return;
+        const int ob = rowb + 4 * (3 + (s & 1) * OP::NBUF) * len;
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+            const int k = lane + WAVE * m;
+            const bool on = k >= c1.lo && k <= c1.hi;
+            if (k < len) op.stage(raw[m], in[m], on, k, &lds_at(sm, ob + 4 * k), len, tab);
+        }
+        if (from_prev) {
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+                const int k = lane + WAVE * m;
+                hwait.wait(hand + ((size_t)(B - 1) * w.nj + (s - r)) * nk + k, k < nk, tag, hw[m]);
+                vin[m] = k < nk ? __uint_as_float((unsigned)hw[m]) : 0.0f;
+            }
+        }
+    };
+    located();                                                // requests step 0's column
+    located();
+    issue();
+    located();
+    work_up(0);
+    c0 = c1;
+    issue();
+    lds_barrier();
+    for (int s = 0; s < nsteps; ++s) {
+        const int xn = rowb + 4 * (2 - (s & 1)) * len;        // new values of step s - 1: own, row r - 1's at xn - 4*rs
+        if (c0.lo <= c0.hi) {                                 // phase 1
+            LineCol ci = none;
+            if (r > 0) {
+                const int4 si = sinfo[((s + 1) & 1) * 16 + r - 1];
+                ci.lo = si.x;
+                ci.hi = si.y;
+            }
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+                const int k = lane + WAVE * m;
+                if (k < len) {
+                    float vi = vin[m], vj = 0.0f;
+                    if (k >= ci.lo && k <= ci.hi) vi = lds_at(sm, xn - 4 * rs + 4 * k);
+                    if (k >= cm.lo && k <= cm.hi) vj = lds_at(sm, xn + 4 * k);
+                    lds_at(sm, rowb + 4 * k) = (k >= c0.lo && k <= c0.hi) ? op.source(in[m], k, c0, vi, vj) : 0.0f;
+                }
+            }
+        }
+        lds_barrier();
+        // phase 2, beside the recurrences
+        float xst[M];
+        const LineCol done = cm;
+        const int cd = c00 + (s - 1 - r) * w.dj;
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+            const int k = lane + WAVE * m;
+            if (k >= done.lo && k <= done.hi) xst[m] = lds_at(sm, xn + 4 * k);
+        }
+        located();
+        if (s + 1 < nsteps) work_up(s + 1);
+        cm = c0;
+        c0 = s + 1 < nsteps ? c1 : none;
+        if (s + 1 < nsteps) issue();
+        if (done.lo <= done.hi)
+#pragma unroll
+            for (int m = 0; m < M; ++m) op.store(cd, lane + WAVE * m, done, xst[m]);
+        lds_barrier();
+    }
+    if (cm.lo <= cm.hi) {
+        const int cd = c00 + (nsteps - 1 - r) * w.dj, xn = rowb + 4 * (1 + ((nsteps - 1) & 1)) * len;
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+            const int k = lane + WAVE * m;
+            op.store(cd, k, cm, k < len ? lds_at(sm, xn + 4 * k) : 0.0f);
+        }
+    }
+}
+// rows of a strip: as strip_rows() for one situation
+static inline int line_rows(int ni) { return ni > 40 ? 10 : STRIP_ROWS_MIN; }
+template <class OP, int M>
+static int launch_line(const OP &op, const LineSweep &w, hipStream_t s) {
+    const int rows = line_rows(w.ni);
+    const size_t shm = line_lds<OP>(w.nk, rows);
+    if (lds_limit((const void *)k_line_strip<OP, M>, shm)) return (int)hipErrorInvalidValue;
+    hipLaunchKernelGGL((k_line_strip<OP, M>), dim3((w.ni + rows - 1) / rows), dim3((rows + 1) * WAVE), shm, s, op, w);
+    return 0;
+}
+
 static inline int ndiag(int oa, int ob, int ia, int ib) { return (ob - oa) + (ib - ia) + 1; }
 static inline int diag_len(int t, int oa, int ob, int ia, int ib) {
     int nb = ib - ia;
@@ -2539,12 +2739,14 @@ static inline int diag_len(int t, int oa, int ob, int ia, int ib) {
 // ------------------------------------------------------------------------
 __device__ __forceinline__ size_t dg3(const DiagArgs &g, int i, int j) { return ((size_t)i * g.nj2 + j) * (size_t)g.nkh; }
 
-// DPM = 0 for i in [1,NII], j in [1,NJJ], k in [1,NKK+1] (DiagnosticFlowfield.cs:40-49)
+// DPM = 0 for i in [1,NII], j in [1,NJJ], k in [1,NKK+1] (DiagnosticFlowfield.cs:40-49);
+// the columns the sweep visits from k = 0, where the sweep writes 0
 __global__ void k_dg_zero(DiagArgs g) {
     int c = blockIdx.x, i = 1 + c / g.njj, j = 1 + c % g.njj;
     if (i > g.nii) return;
     size_t o = dg3(g, i, j);
-    for (int k = 1 + threadIdx.x; k <= g.nkk + 1; k += blockDim.x) g.dpm[o + k] = 0.0f;
+    const bool inner = i > 1 && i < g.nii && j > 1 && j < g.njj;
+    for (int k = (inner ? 0 : 1) + threadIdx.x; k <= g.nkk + 1; k += blockDim.x) g.dpm[o + k] = 0.0f;
 }
 
 // mass divergence of every interior column (:53-80); block = one column
@@ -2560,14 +2762,102 @@ __global__ void k_dg_divergence(DiagArgs g) {
     }
 }
 
-// pressure correction (:84-341), one anti-diagonal of the sweep per launch,
-// one wave per column.  Every column is solved from NKK-1 down to KKART+1 and
-// PIMP[NKK] is never written, so TERMP and PIMP at level k are the same in
-// every column whose bottom lies below k; at the bottom level only ABP (and so
-// PIMP) differs.  The host runs that recurrence once (term, p_in, p_bot);
-// here the lanes build DIM and stage the tables in LDS, and lane 0 runs the
-// two recurrences that depend on the column (QIMP top-down from QIMP[NKK] = 0,
-// then the new DPM bottom-up from DPM[KKART] = 0) over LDS.
+// pressure correction of the diagnostic pass (:84-341).  Every column is solved
+// from NKK-1 down to KKART+1 and PIMP[NKK] is never written, so TERMP and PIMP at
+// level k are the same in every column whose bottom lies below k; at the bottom
+// level only ABP (and so PIMP) differs, and there PIMP multiplies DPM[KKART] = 0.
+// The host runs that recurrence once (term, p_in); the recurrences left to a
+// column are QIMP[k] = (ATP[k] QIMP[k+1] + DIM[k]) TERMP[k] from QIMP[NKK] = 0
+// down and DPM[k] = PIMP[k] DPM[k-1] + QIMP[k] from DPM[KKART] = 0 up.  Columns
+// outside the sweep hold DPM = 0.  Bound by the 5 dependent operations a level:
+// 4.6 us a step of 222 levels, 3.7 ms a sweep of 399 x 399 columns, against
+// 11.1 ms with one launch per anti-diagonal.
+struct DgOp {
+    enum { NTAB = 4, NBUF = 0 };                              // tables: ATP, TERMP, PIMP, DZK
+    DiagArgs g;
+    float rx, ry;                                             // 1 / DXK, 1 / DYK
+    int p2, jp;                                               // both powers of two (their reciprocals are exact); JS == 1
+    struct Raw { float div, pa, pb; };                        // old DPM in the sweep's directions i and j
+    struct In { float div, pa, pb, dz; };
+    __device__ __forceinline__ float table(int a, int k) const {
+        return a == 0 ? g.atp[k] : a == 1 ? g.term[k] : a == 2 ? g.p_in[k] : g.dzk[k];
+    }
+    __device__ __forceinline__ LineCol levels(int c) const { return LineCol{((const ci32 *)g.kk)[c] + 1, g.nkk - 1, 0}; }
+    __device__ __forceinline__ void load(Raw &q, int c, int di, int dj, int k) const {
+        const gf32 *X = (const gf32 *)g.dpm;
+        q.div = ((const gf32 *)g.div)[(size_t)c * g.nkh + k];
+        q.pa = X[(size_t)(c + di) * g.nkh + k];
+        q.pb = X[(size_t)(c + dj) * g.nkh + k];
+    }
+    __device__ __forceinline__ void stage(const Raw &q, In &a, bool on, int k, float *, int len, const float *tab) const {
+        if (!on) return;
+        a.div = q.div / g.dtime;
+        a.pa = q.pa;
+        a.pb = q.pb;
+        a.dz = tab[3 * len + k];
+    }
+    __device__ __forceinline__ float source(const In &a, int, const LineCol &, float vi, float vj) const {
+        const float sx = vi + a.pa, sy = (jp ? vj : a.pb) - (jp ? a.pb : vj);
+        const float qx = p2 ? sx * rx : sx / g.dxk, qy = p2 ? sy * ry : sy / g.dyk;
+        return a.div + qx * g.dyk * a.dz + qy * g.dxk * a.dz;
+    }
+    __device__ __forceinline__ void chain(float *L, float *N, float *, const float *tab, int len, int lo, int clo, int chi,
+                                          int ct) const {
+        const float *A = tab, *T = tab + len;
+        const int top = g.nkk - 1;
+        {
+            float q = 0.0f;
+            Chunk d[2], a[2], t[2];
+            int o = ct * CHK;
+            d[0] = ld_chunk(L + o); a[0] = ld_chunk(A + o); t[0] = ld_chunk(T + o);
+#pragma unroll
+            for (int u = 0; u < CHK; ++u) {                   // Q stays 0 above the top
+                d[0].v[u] = o + u > top ? 0.0f : d[0].v[u];
+                a[0].v[u] = o + u > top ? 0.0f : a[0].v[u];
+            }
+            for (int c = ct; c >= clo;) {
+#pragma unroll
+                for (int h = 0; h < CHK_BLOCK; ++h) {
+                    if (c < clo) break;
+                    const int k = h & 1, m = k ^ 1, on = max(o - CHK, 0);
+                    d[m] = ld_chunk(L + on); a[m] = ld_chunk(A + on); t[m] = ld_chunk(T + on);
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int u = CHK - 1; u >= 0; --u) {
+                        q = (a[k].v[u] * q + d[k].v[u]) * t[k].v[u];
+                        d[k].v[u] = q;
+                    }
+                    st_chunk(L + o, d[k]);
+                    o = on;
+                    --c;
+                }
+            }
+        }
+        // up to the chunk of the highest bottom a lane starts when its level comes
+        const float *P = tab + 2 * len + clo * CHK, *Q = L + clo * CHK;
+        N += clo * CHK;
+        float x = 0.0f;
+        int c = clo;
+        for (; c <= chi; ++c) {
+            Chunk p = ld_chunk(P), w = ld_chunk(Q);
+#pragma unroll
+            for (int u = 0; u < CHK; ++u) {
+                x = (c * CHK + u >= lo) ? p.v[u] * x + w.v[u] : 0.0f;
+                w.v[u] = x;
+            }
+            st_chunk(N, w);
+            P += CHK; Q += CHK; N += CHK;
+        }
+        if (c <= ct) strip_pup(P, Q, N, x, ct - c + 1);
+    }
+    __device__ __forceinline__ void store(int c, int k, const LineCol &q, float x) const {
+        if (k >= q.lo && k <= q.hi) ((gf32 *)g.dpm)[(size_t)c * g.nkh + k] = x;
+    }
+};
+
+// The same sweep with one launch per anti-diagonal and one wave per column, for
+// columns of more levels than k_line_strip holds: the lanes build DIM and stage the
+// tables in LDS, and lane 0 runs the two recurrences over LDS.
 #define DG_UNROLL 8
 __global__ __launch_bounds__(WAVE) void k_dg_pressure(DiagArgs g, int t, int IS, int JS) {
     extern __shared__ float sm[];
@@ -2672,9 +2962,18 @@ __global__ void k_dg_wmass(DiagArgs g) {
     }
 }
 
+static bool pow2(float x) { int e; return x > 0.0f && std::frexp(x, &e) == 0.5f && e > -100 && e < 100; }
+// 8-byte words of the diagnostic sweep's hand-off buffer; 0: its columns have more
+// levels than the strips hold
+extern "C" size_t pf_diag_hand(int nii, int njj, int nkh) {
+    if (nkh > 4 * WAVE || nii < 3 || njj < 3) return 0;
+    const int rows = line_rows(nii - 2);
+    return (size_t)((nii - 2 + rows - 1) / rows) * (njj - 2) * nkh;
+}
 extern "C" int pf_launch_diagnostic(const DiagArgs *ga, int iterations, hipStream_t s) {
     const DiagArgs &g = *ga;
     int ncol = (g.nii - 2) * (g.njj - 2);
+    const bool strips = g.hand != nullptr;                    // pf_diag_hand() words, cleared, and DG_SYNC cleared ints
     hipLaunchKernelGGL(k_dg_zero, dim3(g.nii * g.njj), dim3(64), 0, s, g);
     for (int it = 1; it <= iterations; ++it) {
         hipLaunchKernelGGL(k_dg_divergence, dim3(ncol), dim3(64), 0, s, g);
@@ -2687,8 +2986,15 @@ extern "C" int pf_launch_diagnostic(const DiagArgs *ga, int iterations, hipStrea
         }
         int oa = 2, ob = g.njj - 1, ia = 2, ib = g.nii - 1;
         size_t shm = sizeof(float) * 5 * (size_t)g.nkh;
-        for (int t = 0; t < ndiag(oa, ob, ia, ib); ++t)
-            hipLaunchKernelGGL(k_dg_pressure, dim3(diag_len(t, oa, ob, ia, ib)), dim3(WAVE), shm, s, g, t, IS, JS);
+        if (strips) {
+            const int i0 = IS == -1 ? ib : ia, j0 = JS == -1 ? ob : oa;
+            const DgOp op{g, 1.0f / g.dxk, 1.0f / g.dyk, pow2(g.dxk) && pow2(g.dyk), JS == 1};
+            const LineSweep w{ib - ia + 1, ob - oa + 1, i0 * g.nj2 + j0, IS * g.nj2, JS, g.nkh, g.sync, 1 + it, it, g.hand};
+            const int e = g.nkh <= 2 * WAVE ? launch_line<DgOp, 2>(op, w, s) : launch_line<DgOp, 4>(op, w, s);
+            if (e) return e;
+        } else
+            for (int t = 0; t < ndiag(oa, ob, ia, ib); ++t)
+                hipLaunchKernelGGL(k_dg_pressure, dim3(diag_len(t, oa, ob, ia, ib)), dim3(WAVE), shm, s, g, t, IS, JS);
         hipLaunchKernelGGL(k_dg_correction, dim3(ncol), dim3(64), 0, s, g);
     }
     hipLaunchKernelGGL(k_dg_wmass, dim3((ncol + 63) / 64), dim3(64), 0, s, g);
@@ -3286,6 +3592,26 @@ struct Launcher {
     }
 };
 
+// One momentum sweep on strips (the coefficient pre-pass, then the strips) over
+// a in [oa, nii-1], b in [ia, njj-1]; go(family, launch), family -1: the sweep's own.
+template <class Go>
+static void launch_ml_strip(const Dom *hd, int nsit, const Dom *dd, StripKernel coef, StripKernel strip, int oa, int ia,
+                            int is, int js, int rows, hipStream_t s, Go &&go) {
+    int nblk = 0, nst = 0, nkp = 0;
+    for (int q = 0; q < nsit; ++q) {
+        int ob = hd[q].nii - 1, ib = hd[q].njj - 1;
+        int na = ob - oa + 1, nb = ib - ia + 1;
+        nblk = max(nblk, ((na * nb + COEF_COLS - 1) / COEF_COLS + NXCD - 1) / NXCD * NXCD);
+        nst = max(nst, (ib - ia + rows) / rows);
+        nkp = max(nkp, hd[q].nkp);
+    }
+    const unsigned Z = (unsigned)nsit;
+    const size_t shm_c = sizeof(float) * 3 * (nkp | 1) * COEF_COLS + sizeof(int) * (SCOL * COEF_COLS + 4);
+    go(FAM_COEF, [&] { hipLaunchKernelGGL(coef, dim3(nblk, 1, Z), dim3(4 * WAVE), shm_c, s, dd, is, js); });
+    const size_t shm_t = ml_strip_lds(hd, nsit, oa == 2 && ia == 2, rows);
+    go(-1, [&] { hipLaunchKernelGGL(strip, dim3(nst, 1, Z), dim3((rows + 2) * WAVE), shm_t, s, dd, is, js); });
+}
+
 // Launches one SIMPLE iteration of nsit situations that advance in lock step
 // (same iteration number, hence the same sweep directions).  hd: host copies
 // of the situations' Dom, dd: the same array in device memory.  Grid slice z
@@ -3385,18 +3711,9 @@ static int launch_iteration(const Dom *hd, int nsit, const Dom *dd, int iter, in
                 L.go(fam, [&] { hipLaunchKernelGGL(kern, dim3(len, 1, Z), dim3(WAVE), shm, s, dd, t, is, js); });
         }
     };
-    auto strip_sweep = [&](int fam, auto coef, auto strip, int oa, int ia, int is, int js) {
-        int nblk = 0, nst = 0;
-        for (int q = 0; q < nsit; ++q) {
-            int ob = hd[q].nii - 1, ib = hd[q].njj - 1;
-            int na = ob - oa + 1, nb = ib - ia + 1;
-            nblk = max(nblk, ((na * nb + COEF_COLS - 1) / COEF_COLS + NXCD - 1) / NXCD * NXCD);
-            nst = max(nst, (ib - ia + rows) / rows);
-        }
-        const size_t shm_c = sizeof(float) * 3 * (nkp | 1) * COEF_COLS + sizeof(int) * (SCOL * COEF_COLS + 4);
-        L.go(FAM_COEF, [&] { hipLaunchKernelGGL(coef, dim3(nblk, 1, Z), dim3(4 * WAVE), shm_c, s, dd, is, js); });
-        const size_t shm_t = ml_strip_lds(hd, nsit, oa == 2 && ia == 2, rows);
-        L.go(fam, [&] { hipLaunchKernelGGL(strip, dim3(nst, 1, Z), dim3((rows + 2) * WAVE), shm_t, s, dd, is, js); });
+    auto strip_sweep = [&](int fam, StripKernel coef, StripKernel strip, int oa, int ia, int is, int js) {
+        launch_ml_strip(hd, nsit, dd, coef, strip, oa, ia, is, js, rows, s,
+                        [&](int f, auto &&go) { L.go(f < 0 ? fam : f, go); });
     };
     bool all_w8 = true;
     for (int q = 0; q < nsit; ++q) all_w8 = all_w8 && hd[q].simd == 8;
@@ -3994,12 +4311,28 @@ __global__ void k_mom_fill(float *p, size_t n) {
 }
 
 // One sweep of momentum component comp (0 U, 1 V, 2 W) of the mixing-length
-// model in the directions (IS, JS) the iteration gives it, one launch per
-// anti-diagonal (bit for bit the strip sweep's result).
+// model in the directions (IS, JS) the iteration gives it: the strips where the
+// situation has them, else one launch per anti-diagonal (the same result bit for
+// bit; 254 x 254 columns: 9.1 ms).
 extern "C" int pf_launch_momentum_sweep(const Dom *hd, const Dom *dd, int comp, int IS, int JS, hipStream_t s) {
     const Dom &h = *hd;
     if (h.model != 1 || comp < 0 || comp > 2) return (int)hipErrorInvalidValue;
     const int oa = (comp == 0) ? 3 : 2, ia = (comp == 1) ? 3 : 2, ob = h.nii - 1, ib = h.njj - 1;
+    if (ob < oa || ib < ia) return 0;
+    if (h.tiled == 2) {
+        const int rows = strip_rows(hd, 1, false, ml_strip_lds_w);
+        if (comp == 0 ? ml_strip_limit<0>(1, hd, 1) : comp == 1 ? ml_strip_limit<1>(1, hd, 1) : ml_strip_limit<2>(1, hd, 1))
+            return (int)hipErrorInvalidValue;
+        const bool w8 = h.simd == 8;
+        const StripKernel strip = comp == 0 ? (w8 ? ml_strip<0, 8, 0>(hd, 1) : ml_strip<0, 0, 0>(hd, 1)) :
+                                  comp == 1 ? (w8 ? ml_strip<1, 8, 0>(hd, 1) : ml_strip<1, 0, 0>(hd, 1)) :
+                                              (w8 ? ml_strip<2, 8, 0>(hd, 1) : ml_strip<2, 0, 0>(hd, 1));
+        const StripKernel coef = comp == 0 ? (w8 ? k_ml_coef<0, 8> : k_ml_coef<0, 0>) :
+                                 comp == 1 ? (w8 ? k_ml_coef<1, 8> : k_ml_coef<1, 0>) : (w8 ? k_ml_coef<2, 8> : k_ml_coef<2, 0>);
+        hipLaunchKernelGGL(k_zero_rows, dim3((unsigned)((5 * h.sync_stride + 255) / 256)), dim3(256), 0, s, dd, 0);
+        launch_ml_strip(hd, 1, dd, coef, strip, oa, ia, IS, JS, rows, s, [](int, auto &&f) { f(); });
+        return (int)hipGetLastError();
+    }
     const size_t shm = sizeof(float) * 5 * h.nkp;
     for (int t = 0; t < ndiag(oa, ob, ia, ib); ++t) {
         const unsigned len = (unsigned)diag_len(t, oa, ob, ia, ib);

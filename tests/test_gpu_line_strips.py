@@ -1,0 +1,49 @@
+"""Sweeps of two first-order recurrences on strips, at the edges of their layout.
+
+The diagnostic pressure sweep: one, two and four groups of 64 levels a column,
+columns too tall for the strips, strips of 7 and 10 rows that end in a partial
+strip, cell sizes that are no power of two; every field bit for bit against the
+oracle.  One momentum sweep: on strips bit for bit what it is with one launch
+per anti-diagonal.
+"""
+import numpy as np
+import pytest
+
+from gral_amd import domain
+from tests.test_gpu_diagnostic import FIELDS, _compare
+
+DIAG = [
+    # nii, njj, dx, first level, stretch: NKK 25, 62, 63, 126, 127, 221, 254 and 255
+    (9, 8, 2.0, 2.0, 1.2), (16, 17, 3.0, 1.0, 1.067), (43, 42, 2.0, 1.0, 1.0655), (17, 45, 2.0, 1.0, 1.02425),
+    (44, 9, 2.5, 1.0, 1.02395), (12, 11, 2.0, 1.0, 1.01), (10, 12, 2.0, 1.0, 1.00785), (11, 10, 2.0, 1.0, 1.0078),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nii,njj,dx,dz1,stretch", DIAG)
+def test_diagnostic_edges(nii, njj, dx, dz1, stretch):
+    bl = domain.city_buildings(nii, njj, dx, 3, density=0.25, fmin=3.0, fmax=9.0, hmin=3.0, hmax=25.0, margin=1)
+    c = domain.build_case("dgs", nii, njj, bl, dx=dx, dz1=dz1, stretch=stretch, vertcellsff=8, direction=215.0, iterations=2)
+    _compare(c, 0, 2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("width", [8, 16])
+@pytest.mark.parametrize("nii,njj", [(9, 11), (18, 16), (46, 43)])
+def test_momentum_sweep_kinds(monkeypatch, nii, njj, width):
+    from gral_amd import pf
+    bl = domain.city_buildings(nii, njj, 2.0, 5, density=0.2, fmin=4.0, fmax=12.0, hmin=3.0, hmax=14.0, margin=2)
+    c = domain.build_case("ms", nii, njj, bl, dx=2.0, vertcellsff=17, direction=235.0, z0=0.5, iterations=4)
+    c.simd_width = width
+    out = {}
+    for sw in ("strip", "diag"):
+        monkeypatch.setenv("GRAL_PF_SWEEP", sw)
+        with pf.PrognosticFlowfield(c) as s:
+            s.prepare(iterations=4)
+            s.iterate(3)
+            for comp in range(3):
+                print(f"[line strips] sweep {comp} of {nii}x{njj} {sw}", flush=True)
+                s.momentum_sweep(comp)
+            out[sw] = s.download()
+    for f in FIELDS:
+        assert np.array_equal(out["strip"][f].view(np.uint32), out["diag"][f].view(np.uint32)), f
