@@ -197,6 +197,8 @@ struct gral_pf_handle {
     // adjoint of the pressure-correction steps (gral_pf_forward_ckpt / gral_pf_vjp)
     std::vector<float> app, abp, atp;   // per-level pressure coefficients of the prologue
     float *adj = nullptr;           // ub vb wb pb qb mb db, checkpoint uk vk wk, ptab[2] ttab[2]: 15 fields
+    float *mom_rec = nullptr;       // momentum_vjp's column data and hand-off words (per-diagonal situations)
+    unsigned long long *mom_hand = nullptr;
     int *adj_src = nullptr;         // stale-top source column per column, for IS = +1 and -1
     int adj_first = 0, adj_n = 0;   // iterations of the last forward
     int mom_comp = -1, mom_is = 1, mom_js = 1;   // the last gral_pf_momentum_sweep: component, directions
@@ -397,6 +399,8 @@ static void free_device(gral_pf_handle *h) {
     if (h->graphs) h->graphs->clear();
     h->adj = nullptr;
     h->adj_src = nullptr;
+    h->mom_rec = nullptr;
+    h->mom_hand = nullptr;
     h->adj_n = 0;
     h->mom_comp = -1;
     h->mom_vjp_ok = false;
@@ -1578,14 +1582,36 @@ extern "C" int gral_pf_momentum_vjp(gral_pf_handle *h, const float *dx, float *g
     MomAdj m{};
     m.xa = xa;
     m.gin = a;
-    m.gout = a + n3; m.gpa = a + 2 * n3; m.gpb = a + 3 * n3; m.gna = a + 4 * n3; m.gnb = a + 5 * n3; m.gres = a + 6 * n3;
+    m.gout = a + n3; m.db = a + 2 * n3; m.gna = a + 4 * n3; m.gnb = a + 5 * n3; m.gres = a + 6 * n3;
     int rc;
+    // the columns' data: in the sweeps' coefficient records, which hold nothing
+    // between two sweeps, or where the situation has none in a buffer of its own
+    float *rec = h->d.planes;
+    m.hand = h->d.hand;
+    if (!h->d.tiled) {
+        if (!h->mom_rec) {
+            float *q;
+            unsigned long long *hw;
+            if ((rc = dalloc(h, &hw, h->d.hand_words)) || (rc = dalloc(h, &q, 8 * n3 + 4))) return rc;
+            HIPCHK(h, hipMemsetAsync(hw, 0, h->d.hand_words * sizeof(unsigned long long), h->stream));
+            h->mom_rec = q;
+            h->mom_hand = hw;
+        }
+        rec = h->mom_rec;
+        m.hand = h->mom_hand;
+    }
+    m.T = rec; m.P = rec + n3; m.C = rec + 2 * n3; m.Q = rec + 3 * n3;
+    m.ca = rec + 4 * n3; m.cb = rec + 5 * n3; m.cc = rec + 6 * n3;
+    m.col = reinterpret_cast<int4 *>((reinterpret_cast<uintptr_t>(rec + 7 * n3) + 15) & ~(uintptr_t)15);
     if ((rc = put_raw(h, a, dx))) return rc;
     HIPCHK(h, hipEventRecord(h->ev0, h->stream));
     const int e = pf_launch_momentum_vjp(&hb, db, &m, comp, h->mom_is, h->mom_js, h->stream);
     HIPCHK(h, hipEventRecord(h->ev1, h->stream));
     if (e) return fail(h, GRAL_PF_EDEVICE, std::string("momentum_vjp: launch failed: ") + hipGetErrorString((hipError_t)e));
     HIPCHK(h, hipEventSynchronize(h->ev1));
+    int serr = 0;
+    HIPCHK(h, hipMemcpy(&serr, h->d.sync, sizeof(int), hipMemcpyDeviceToHost));
+    if (serr) return fail(h, GRAL_PF_EDEVICE, "momentum_vjp: a strip wait timed out (results invalid)");
     float ms = 0;
     HIPCHK(h, hipEventElapsedTime(&ms, h->ev0, h->ev1));
     h->timing = gral_pf_timing{};

@@ -176,7 +176,10 @@ struct MomAdj {
     const float *xa;    // X after the sweep (the device field)
     const float *gin;   // dL/dX after
     float *gout;        // dL/dX before: the swept columns' own levels KSTART-1..VI+1
-    float *gpa, *gpb;   // per column and level: adjoint for the new X of its a- / b-predecessor
+    float *db;          // per column and level: adjoint of the source D
+    float *T, *P, *C, *Q, *ca, *cb, *cc;   // what its columns need (k_adj_mom_pre)
+    int4 *col;          // per column: levels of the sweep
+    unsigned long long *hand;   // hand-off words, laid out as Dom::hand
     float *gna, *gnb;   // per column and level: adjoint for the old X of its a- / b-successor
     float *gres;        // dL/dX before, complete
 };

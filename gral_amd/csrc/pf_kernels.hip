@@ -15,6 +15,7 @@
 // This replays the reference's deterministic (single-thread) order exactly.
 #include <cmath>
 #include <mutex>
+#include <type_traits>
 #include "pf_device.h"
 
 #define WAVE 64
@@ -2586,8 +2587,14 @@ __global__ __launch_bounds__(STRIP_WAVES * WAVE) void k_line_strip(OP op, LineSw
         auto send_last = [&](int s) {
             if (!send || s < R) return;                       // l = s - R is a step of the last row
             const int a = __builtin_amdgcn_readlane(lo, R - 1), b = __builtin_amdgcn_readlane(hi, R - 1);
-            for (int k = lane; k < nk; k += WAVE)
-                hand_put(h + (size_t)s * nk + k, (k >= a && k <= b) ? xl[((s - 1) & 1) * len + k] : 0.0f, tag);
+            float v[M];
+#pragma unroll
+            for (int m = 0; m < M; ++m) v[m] = xl[((s - 1) & 1) * len + min(lane + WAVE * m, len - 1)];
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+                const int k = lane + WAVE * m;
+                if (k < nk) hand_put(h + (size_t)s * nk + k, (k >= a && k <= b) ? v[m] : 0.0f, tag);
+            }
         };
         lds_barrier();                                        // the rows' operands and levels of step 0
         for (int s = 0; s < nsteps; ++s) {
@@ -2615,8 +2622,11 @@ __global__ __launch_bounds__(STRIP_WAVES * WAVE) void k_line_strip(OP op, LineSw
     LineCol q2 = none, c2 = none, c1 = none, c0 = none, cm = none;    // requested, steps s+2, s+1, s, s-1
     int l2 = -r - 1;                                          // step (of this row) q2 belongs to
     typename OP::Raw raw[M];
-    typename OP::In in[M];
+    typename OP::In in[M] = {};
     unsigned long long hw[M];
+    int kb[M];                                                // byte offsets of the lane's levels in an array
+#pragma unroll
+    for (int m = 0; m < M; ++m) kb[m] = 4 * min(lane + WAVE * m, len - 1);
     float vin[M] = {};                                        // row 0: the new values of the previous strip's last row
     auto located = [&]() {                                    // q2 arrives, the next is requested
         c2 = q2;
@@ -2666,20 +2676,24 @@ __global__ __launch_bounds__(STRIP_WAVES * WAVE) void k_line_strip(OP op, LineSw
         const int xn = rowb + 4 * (2 - (s & 1)) * len;        // new values of step s - 1: own, row r - 1's at xn - 4*rs
         if (c0.lo <= c0.hi) {                                 // phase 1
             LineCol ci = none;
+            const int xi = xn - (r > 0 ? 4 * rs : 0);
             if (r > 0) {
                 const int4 si = sinfo[((s + 1) & 1) * 16 + r - 1];
                 ci.lo = si.x;
                 ci.hi = si.y;
             }
+            float vi[M], vj[M];                               // all reads ahead of the operations, without branches
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+                vi[m] = lds_at(sm, xi + kb[m]);
+                vj[m] = lds_at(sm, xn + kb[m]);
+            }
 #pragma unroll
             for (int m = 0; m < M; ++m) {
                 const int k = lane + WAVE * m;
-                if (k < len) {
-                    float vi = vin[m], vj = 0.0f;
-                    if (k >= ci.lo && k <= ci.hi) vi = lds_at(sm, xn - 4 * rs + 4 * k);
-                    if (k >= cm.lo && k <= cm.hi) vj = lds_at(sm, xn + 4 * k);
-                    lds_at(sm, rowb + 4 * k) = (k >= c0.lo && k <= c0.hi) ? op.source(in[m], k, c0, vi, vj) : 0.0f;
-                }
+                const float a = (k >= ci.lo && k <= ci.hi) ? vi[m] : vin[m], b = (k >= cm.lo && k <= cm.hi) ? vj[m] : 0.0f;
+                const float d = op.source(in[m], k, c0, a, b);
+                if (k < len) lds_at(sm, rowb + 4 * k) = (k >= c0.lo && k <= c0.hi) ? d : 0.0f;
             }
         }
         lds_barrier();
@@ -2769,9 +2783,9 @@ __global__ void k_dg_divergence(DiagArgs g) {
 // The host runs that recurrence once (term, p_in); the recurrences left to a
 // column are QIMP[k] = (ATP[k] QIMP[k+1] + DIM[k]) TERMP[k] from QIMP[NKK] = 0
 // down and DPM[k] = PIMP[k] DPM[k-1] + QIMP[k] from DPM[KKART] = 0 up.  Columns
-// outside the sweep hold DPM = 0.  Bound by the 5 dependent operations a level:
-// 4.6 us a step of 222 levels, 3.7 ms a sweep of 399 x 399 columns, against
-// 11.1 ms with one launch per anti-diagonal.
+// outside the sweep hold DPM = 0.  Bound by the 5 dependent operations a level (56
+// cycles with their LDS accesses): 5.5 ms a sweep of 397 x 397 columns of 221
+// levels, 11.1 ms with one launch per anti-diagonal (4 to 12 rows a strip: within 3%).
 struct DgOp {
     enum { NTAB = 4, NBUF = 0 };                              // tables: ATP, TERMP, PIMP, DZK
     DiagArgs g;
@@ -4038,14 +4052,15 @@ extern "C" int pf_launch_mass(const Dom *dd, int nsit, int nblk, double *partial
 // cross-term factor), the Coriolis/vegetation and wall terms (own level), the
 // cross terms (own level and the two neighbours along the component), the four
 // neighbour couplings (new values of the two columns visited before it, old
-// values of the two after it) and the relaxation.  The transpose runs the
-// sweep's anti-diagonals from the last to the first, one wave per column: the
-// lanes recompute the column's coefficients from the checkpointed fields, lane
-// 0 runs the Thomas recurrences forward and then both recurrences transposed,
-// and the lanes push the adjoints back through the coefficient assembly.  The
-// adjoint handed to another column has one writer (buffers indexed by the
-// handing column, per direction) and is gathered by its receiver, so the
-// result is deterministic.
+// values of the two after it) and the relaxation.  Of a column's transpose only the
+// recurrence through Q and the couplings to the two columns visited before it
+// reach other columns, so three kernels do the transpose: k_adj_mom_pre computes
+// every column's Thomas coefficients and couplings from the checkpointed fields
+// (all columns at once), a strip sweep in reverse order carries the adjoint from
+// column to column, and k_adj_mom runs the rest of each column's transpose (all
+// columns at once) back through the coefficient assembly.  The adjoint handed to
+// another column has one writer and is gathered by its receiver, so the result
+// is deterministic.
 // ------------------------------------------------------------------------
 
 // d VIS / d X[k+1] of ml_visc (d VIS / d X[k-1] is its negative) for the
@@ -4092,17 +4107,215 @@ __device__ __forceinline__ void ml_coeffs_dvis(const DomG &d, const ColInfo &q, 
     g[5] = face(!(k > q.KK + 1), gT, FB);
 }
 
+// What the transposed sweep needs of each column besides the adjoints handed to
+// it, for every cell of the situation (0 where the sweep does not go): the Thomas
+// coefficients T, P, C (0 where the recurrence starts) and Q, and the couplings
+// through which its DIM adjoint reaches the columns visited before it (ca, cb:
+// along i and j; cc: VIS/DXK of the cross terms along the component's own
+// direction, else 0); per column {KSTART, first level the sweep updates, VI}
+// (VI = -1: none).  Blocks of MA_COLS columns: the lanes work the cells, then
+// lane c runs column c's recurrence.
+#define MA_COLS 8
+template <int COMP>
+__global__ __launch_bounds__(4 * WAVE) void k_adj_mom_pre(const Dom *__restrict__ ds, MomAdj m, int IS, int JS) {
+    const DomG &d = *reinterpret_cast<const DomG *>(ds);
+    extern __shared__ float sm[];
+    const int nkp = d.nkp, nkl = nkp | 1, ncol = (d.nii + 2) * d.nj2, col0 = blockIdx.x * MA_COLS;
+    float *sA = sm, *sB = sA + MA_COLS * nkl, *sC = sB + MA_COLS * nkl, *sD = sC + MA_COLS * nkl, *sT = sD + MA_COLS * nkl;
+    int *scol = (int *)(sT + MA_COLS * nkl);                  // [MA_COLS][4]
+    const int oa = (COMP == 0) ? 3 : 2, ia = (COMP == 1) ? 3 : 2;
+    const gf32 *XA = (const gf32 *)m.xa, *XB = (COMP == 0) ? d.uk : (COMP == 1) ? d.vk : d.wk;
+    if (threadIdx.x < MA_COLS) {
+        const int c = col0 + threadIdx.x, i = c / d.nj2, j = c % d.nj2;
+        int *sc = scol + 4 * threadIdx.x;
+        sc[0] = 1; sc[1] = 0; sc[2] = -1; sc[3] = 0;
+        if (c < ncol) {
+            const int a = (IS == -1) ? d.nii - i + 1 : i, b = (JS == -1) ? d.njj - j + 1 : j;
+            if (a >= oa && a <= d.nii - 1 && b >= ia && b <= d.njj - 1 && d.adv[c] == 1) {
+                const ColInfo q = col_info(d, i, j);
+                int KKm = 0;
+                if (COMP == 0) KKm = max(q.KK, d.kk[c2(d, i - 1, j)]);
+                if (COMP == 1) KKm = max(q.KK, d.kk[c2(d, i, j - 1)]);
+                sc[0] = q.KSTART;
+                sc[1] = max(q.KSTART, KKm + 1);
+                if (COMP == 2) sc[1] = q.KSTART;
+                sc[2] = q.VI;
+                sc[3] = q.KK;
+            }
+            m.col[c] = make_int4(sc[0], sc[1], sc[2], 0);
+        }
+    }
+    __syncthreads();
+    const int cl = threadIdx.x / (4 * WAVE / MA_COLS), lv = threadIdx.x % (4 * WAVE / MA_COLS), c = col0 + cl;
+    const int ks = scol[4 * cl], vi = scol[4 * cl + 2], KK = scol[4 * cl + 3];
+    if (c < ncol) {
+        const int i = c / d.nj2, j = c % d.nj2;
+        const size_t o = (size_t)c * nkp;
+        ColInfo q{};
+        if (vi >= ks) q = col_info(d, i, j);
+        for (int k = lv; k < nkp; k += 4 * WAVE / MA_COLS) {
+            float ca = 0.0f, cb = 0.0f, cc = 0.0f;
+            if (k >= ks && k <= vi) {
+                const MlPieces pc = ml_pieces<COMP>(d, q, k);
+                const size_t di = (size_t)d.nj2 * nkp;
+                const float xpa = XA[o - IS * (ptrdiff_t)di + k], xna = XB[o + IS * (ptrdiff_t)di + k];
+                const float xpb = XA[o - JS * (ptrdiff_t)nkp + k], xnb = XB[o + JS * (ptrdiff_t)nkp + k], x = XB[o + k];
+                const float xw = (IS == 1) ? xpa : xna, xe = (IS == 1) ? xna : xpa;
+                const float xs = (JS == 1) ? xpb : xnb, xn = (JS == 1) ? xnb : xpb;
+                const int p = cl * nkl + k;
+                sA[p] = pc.A; sB[p] = pc.B; sC[p] = pc.C;
+                sD[p] = ml_source<COMP>(d, q, k, d.dzk[k], pc, xw, xs, xe, xn, x);
+                ca = (IS == 1) ? pc.AW1 : pc.AE1;
+                cb = (JS == 1) ? pc.AS1 : pc.AN1;
+                if (COMP != 2 && ml_cross_on(q, k)) cc = pc.c0;
+            }
+            m.ca[o + k] = ca; m.cb[o + k] = cb; m.cc[o + k] = cc;
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < MA_COLS) {
+        const int *sc = scol + 4 * threadIdx.x;
+        float Pp = 0.0f, Qp = 0.0f;
+        for (int k = sc[0]; k <= sc[2]; ++k) {                // as the sweep ran it
+            const int p = threadIdx.x * nkl + k;
+            float T;
+            if (k > sc[3] + 1) { T = 1 / (sA[p] - sC[p] * Pp); Pp = sB[p] * T; Qp = (sD[p] + sC[p] * Qp) * T; }
+            else { T = 1 / sA[p]; Pp = sB[p] * T; Qp = sD[p] * T; }
+            sT[p] = T; sB[p] = Pp; sD[p] = Qp;
+        }
+    }
+    __syncthreads();
+    if (c < ncol)
+        for (int k = lv; k < nkp; k += 4 * WAVE / MA_COLS) {
+            const size_t g = (size_t)c * nkp + k;
+            const int p = cl * nkl + k;
+            const bool on = k >= ks && k <= vi;
+            m.T[g] = on ? sT[p] : 0.0f;
+            m.P[g] = on ? sB[p] : 0.0f;
+            m.Q[g] = on ? sD[p] : 0.0f;
+            m.C[g] = on && k > KK + 1 ? sC[p] : 0.0f;
+            m.db[g] = 0.0f;
+        }
+}
+
+// the adjoint column c hands to the a- (along i) and b-predecessor at level k
+template <int COMP>
+__device__ __forceinline__ float adj_mom_pa(float db, float ca, float cc, float dk) {
+    return (COMP == 0 && cc != 0.0f) ? db * ca + db * cc * dk : db * ca;
+}
+template <int COMP>
+__device__ __forceinline__ float adj_mom_pb(float db, float cb, float cc, float dk) {
+    return (COMP == 1 && cc != 0.0f) ? db * cb + db * cc * dk : db * cb;
+}
+
+// The transposed sweep itself, on strips, in the reverse order of the sweep: the
+// adjoint of a column's X after is gin and what its two successors hand it, and
+// of the column's transposed recurrences only the one through Q reaches another
+// column: g[k] = sG[k] + ub, Q_bar[k] = g relax, ub = Q_bar[k] P[k] up from the
+// first updated level, then Qt = Q_bar[k] + Qc, D_bar[k] = Qt T[k],
+// Qc = Qt C[k] T[k] down.  Bound by these.  The transpose of one component on 254 x
+// 254 columns of up to 47 levels: pre-pass 0.18, strips 1.21, the rest 0.49 ms;
+// with the whole column's transpose in one launch per anti-diagonal 19.5 ms.
+template <int COMP>
+struct MomOp {
+    enum { NTAB = 1, NBUF = 3 };                              // table: DYK DZK (U) or DXK DZK (V); operands: P, C, T
+    MomAdj m;
+    const float *dzk;
+    float h, relax;                                           // DYK (U), DXK (V)
+    int nkp;
+    struct Raw { float g, P, C, T, ca, cb, cc; };
+    struct In { float g, ca, cb, cc, dk; };
+    __device__ __forceinline__ float table(int, int k) const { return h * dzk[k]; }
+    __device__ __forceinline__ LineCol levels(int c) const {
+        const int4 v = ldc4i((const DomG::P<const int4>)m.col + c);
+        return LineCol{v.x, v.z, v.y};
+    }
+    __device__ __forceinline__ void load(Raw &q, int c, int di, int dj, int k) const {
+        const size_t o = (size_t)c * nkp + k, oi = (size_t)(c - di) * nkp + k, oj = (size_t)(c - dj) * nkp + k;
+        q.g = ((const gf32 *)m.gin)[o];
+        q.P = ((const gf32 *)m.P)[o];
+        q.C = ((const gf32 *)m.C)[o];
+        q.T = ((const gf32 *)m.T)[o];
+        q.ca = ((const gf32 *)m.ca)[oi];
+        q.cb = ((const gf32 *)m.cb)[oj];
+        if (COMP != 2) q.cc = ((const gf32 *)m.cc)[COMP == 0 ? oi : oj];
+    }
+    __device__ __forceinline__ void stage(const Raw &q, In &a, bool on, int k, float *buf, int len, const float *tab) const {
+        buf[0] = on ? q.P : 0.0f;
+        buf[len] = on ? q.C : 0.0f;
+        buf[2 * len] = on ? q.T : 0.0f;
+        a.g = q.g; a.ca = q.ca; a.cb = q.cb; a.cc = q.cc;
+        a.dk = tab[k];
+    }
+    __device__ __forceinline__ float source(const In &a, int k, const LineCol &q, float vi, float vj) const {
+        const float g = a.g + adj_mom_pa<COMP>(vi, a.ca, a.cc, a.dk) + adj_mom_pb<COMP>(vj, a.cb, a.cc, a.dk);
+        return k >= q.x ? g : 0.0f;                           // below, the sweep left X as it was
+    }
+    __device__ __forceinline__ void chain(float *L, float *N, float *buf, const float *, int len, int, int clo, int,
+                                          int ct) const {
+        const float *P = buf + clo * CHK, *C = buf + len, *T = buf + 2 * len;
+        float *D = L + clo * CHK;
+        {
+            float ub = 0.0f;
+            Chunk d[2], p[2];
+            d[0] = ld_chunk(D); p[0] = ld_chunk(P);
+            for (int c = clo; c <= ct;) {
+#pragma unroll
+                for (int h8 = 0; h8 < CHK_BLOCK; ++h8) {
+                    if (c > ct) break;
+                    const int k = h8 & 1, n = k ^ 1;
+                    d[n] = ld_chunk(D + CHK); p[n] = ld_chunk(P + CHK);
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int u = 0; u < CHK; ++u) {
+                        const float qb = (d[k].v[u] + ub) * relax;
+                        ub = qb * p[k].v[u];
+                        d[k].v[u] = qb;
+                    }
+                    st_chunk(D, d[k]);
+                    D += CHK; P += CHK;
+                    ++c;
+                }
+            }
+        }
+        float qc = 0.0f;
+        Chunk b[2], e[2], t[2];
+        int o = ct * CHK;
+        b[0] = ld_chunk(L + o); e[0] = ld_chunk(C + o); t[0] = ld_chunk(T + o);
+        for (int c = ct; c >= clo;) {
+#pragma unroll
+            for (int h8 = 0; h8 < CHK_BLOCK; ++h8) {
+                if (c < clo) break;
+                const int k = h8 & 1, n = k ^ 1, on = max(o - CHK, 0);
+                b[n] = ld_chunk(L + on); e[n] = ld_chunk(C + on); t[n] = ld_chunk(T + on);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int u = CHK - 1; u >= 0; --u) {
+                    const float qt = b[k].v[u] + qc;
+                    b[k].v[u] = qt * t[k].v[u];
+                    qc = qt * e[k].v[u] * t[k].v[u];
+                }
+                st_chunk(N + o, b[k]);
+                o = on;
+                --c;
+            }
+        }
+    }
+    __device__ __forceinline__ void store(int c, int k, const LineCol &q, float x) const {
+        if (k >= q.lo && k <= q.hi) ((gf32 *)m.db)[(size_t)c * nkp + k] = x;
+    }
+};
+
+// The rest of a column's transpose, which no other column waits for: both
+// transposed recurrences with the handed adjoints known, and the assembly
+// transposed.  One wave per column.
 #define MA_SLOTS 18
 template <int COMP>
-__global__ __launch_bounds__(WAVE) void k_adj_mom(const Dom *__restrict__ ds, MomAdj m, int t, int IS, int JS) {
+__global__ __launch_bounds__(WAVE) void k_adj_mom(const Dom *__restrict__ ds, MomAdj m, int IS, int JS) {
     const DomG &d = *reinterpret_cast<const DomG *>(ds);       // its swept field is X before the sweep
     extern __shared__ float sm[];
-    const int oa = (COMP == 0) ? 3 : 2, ia = (COMP == 1) ? 3 : 2;
-    int a, b;
-    if (!diag_col(t, oa, d.nii - 1, ia, d.njj - 1, blockIdx.x, a, b)) return;
-    int i, j;
-    sweep_to_ij(d, 0, a, b, IS, JS, i, j);
-    if (d.adv[c2(d, i, j)] != 1) return;
+    const int i = blockIdx.x / d.nj2, j = blockIdx.x % d.nj2;
+    if (m.col[blockIdx.x].z < 0) return;
     const ColInfo q = col_info(d, i, j);
     const int nkp = d.nkp, lane = threadIdx.x;
     const int KK = q.KK, KKP1 = KK + 1, KSTART = q.KSTART, VI = q.VI;
@@ -4127,20 +4340,14 @@ __global__ __launch_bounds__(WAVE) void k_adj_mom(const Dom *__restrict__ ds, Mo
         const float xs = (JS == 1) ? xpb : xnb, xn = (JS == 1) ? xnb : xpb;
         sA[k] = pc.A; sB[k] = pc.B; sC[k] = pc.C;
         sD[k] = ml_source<COMP>(d, q, k, d.dzk[k], pc, xw, xs, xe, xn, x);
-        sG[k] = m.gin[o + k] + m.gpa[c3(d, i + IS, j) + k] + m.gpb[c3(d, i, j + JS) + k];
+        const float dk = (COMP == 0 ? dyk : dxk) * d.dzk[k];
+        sG[k] = m.gin[o + k] + adj_mom_pa<COMP>(m.db[ona + k], m.ca[ona + k], m.cc[ona + k], dk) +
+                adj_mom_pb<COMP>(m.db[onb + k], m.cb[onb + k], m.cc[onb + k], dk);
+        sT[k] = m.T[o + k]; sP[k] = m.P[o + k]; sQ[k] = m.Q[o + k];
     }
     for (int k = KSTART + lane; k <= VI + 1; k += WAVE) sXa[k] = XA[o + k];
     __syncthreads();
     if (lane == 0) {
-        // Thomas forward, as the sweep ran it
-        float Pp = 0.0f, Qp = 0.0f;
-        for (int k = KSTART; k <= VI; ++k) {
-            float T, P, Q;
-            if (k > KKP1) { T = 1 / (sA[k] - sC[k] * Pp); P = sB[k] * T; Q = (sD[k] + sC[k] * Qp) * T; }
-            else { T = 1 / sA[k]; P = sB[k] * T; Q = sD[k] * T; }
-            sT[k] = T; sP[k] = P; sQ[k] = Q;
-            Pp = P; Qp = Q;
-        }
         // relaxed back-substitution X_k += relax (P_k X_{k+1} + Q_k - X_k) from VI down, transposed
         const float rl = d.relax;
         float ub = 0.0f;
@@ -4252,10 +4459,8 @@ __global__ __launch_bounds__(WAVE) void k_adj_mom(const Dom *__restrict__ ds, Mo
             }
         }
         sUp[k] = up; sDn[k] = dn; sMid[k] = xb;
-        // the four neighbours' adjoints, handed on by direction
-        m.gpa[o + k] = (IS == 1) ? xwb : xeb;
+        // the adjoints of the successors' old values
         m.gna[o + k] = (IS == 1) ? xeb : xwb;
-        m.gpb[o + k] = (JS == 1) ? xsb : xnb_;
         m.gnb[o + k] = (JS == 1) ? xnb_ : xsb;
     }
     __syncthreads();
@@ -4299,8 +4504,10 @@ __global__ void k_adj_mom_combine(const Dom *__restrict__ ds, MomAdj m, int IS, 
     }
     if (!done) {
         v += m.gin[g];
-        if (inside(i + IS, j)) v += m.gpa[c3(d, i + IS, j) + k];
-        if (inside(i, j + JS)) v += m.gpb[c3(d, i, j + JS) + k];
+        const float dk = (COMP == 0 ? d.dyk : d.dxk) * d.dzk[k];
+        const size_t na = c3(d, i + IS, j) + k, nb = c3(d, i, j + JS) + k;
+        if (inside(i + IS, j)) v += adj_mom_pa<COMP>(m.db[na], m.ca[na], m.cc[na], dk);
+        if (inside(i, j + JS)) v += adj_mom_pb<COMP>(m.db[nb], m.cb[nb], m.cc[nb], dk);
     }
     m.gres[g] = v;
 }
@@ -4352,16 +4559,28 @@ extern "C" int pf_launch_momentum_vjp(const Dom *hd, const Dom *dd, const MomAdj
     const MomAdj m = *ma;
     const size_t n3 = (size_t)(h.nii + 2) * h.nj2 * h.nkp;
     const unsigned fb = (unsigned)((n3 + 255) / 256);
-    float *z[5] = {m.gout, m.gpa, m.gpb, m.gna, m.gnb};
+    float *z[3] = {m.gout, m.gna, m.gnb};
     for (float *p : z) hipLaunchKernelGGL(k_mom_fill, dim3(fb), dim3(256), 0, s, p, n3);
-    const int oa = (comp == 0) ? 3 : 2, ia = (comp == 1) ? 3 : 2, ob = h.nii - 1, ib = h.njj - 1;
-    const size_t shm = sizeof(float) * MA_SLOTS * h.nkp;
-    for (int t = ndiag(oa, ob, ia, ib) - 1; t >= 0; --t) {
-        const unsigned len = (unsigned)diag_len(t, oa, ob, ia, ib);
-        if (comp == 0) hipLaunchKernelGGL(k_adj_mom<0>, dim3(len), dim3(WAVE), shm, s, dd, m, t, IS, JS);
-        else if (comp == 1) hipLaunchKernelGGL(k_adj_mom<1>, dim3(len), dim3(WAVE), shm, s, dd, m, t, IS, JS);
-        else hipLaunchKernelGGL(k_adj_mom<2>, dim3(len), dim3(WAVE), shm, s, dd, m, t, IS, JS);
-    }
+    const int oa = (comp == 0) ? 3 : 2, ia = (comp == 1) ? 3 : 2, ni = h.nii - oa, nj = h.njj - ia;
+    const int ncol = (h.nii + 2) * h.nj2;
+    const size_t shm_p = (sizeof(float) * 5 * (h.nkp | 1) + sizeof(int) * 4) * MA_COLS, shm = sizeof(float) * MA_SLOTS * h.nkp;
+    hipLaunchKernelGGL(k_zero_rows, dim3((unsigned)((5 * h.sync_stride + 255) / 256)), dim3(256), 0, s, dd, 0);
+    int e = 0;
+    auto run = [&](auto tag) {
+        constexpr int C = decltype(tag)::value;
+        hipLaunchKernelGGL(k_adj_mom_pre<C>, dim3((ncol + MA_COLS - 1) / MA_COLS), dim3(4 * WAVE), shm_p, s, dd, m, IS, JS);
+        if (ni > 0 && nj > 0) {
+            // the sweep's order reversed: from its last row and column back
+            const int i0 = IS == 1 ? h.nii - 1 : 2, j0 = JS == 1 ? h.njj - 1 : 2;
+            const MomOp<C> op{m, h.dzk, C == 0 ? h.dyk : h.dxk, h.relax, h.nkp};
+            const LineSweep w{ni, nj, i0 * h.nj2 + j0, -IS * h.nj2, -JS, h.nkp, h.sync, SYNC_BLOCK0, 6, m.hand};
+            e = h.nkp <= WAVE ? launch_line<MomOp<C>, 1>(op, w, s) : launch_line<MomOp<C>, 2>(op, w, s);
+            if (!e) hipLaunchKernelGGL(k_adj_mom<C>, dim3(ncol), dim3(WAVE), shm, s, dd, m, IS, JS);
+        }
+    };
+    if (comp == 0) run(std::integral_constant<int, 0>()); else if (comp == 1) run(std::integral_constant<int, 1>());
+    else run(std::integral_constant<int, 2>());
+    if (e) return e;
     if (comp == 0) hipLaunchKernelGGL(k_adj_mom_combine<0>, dim3(fb), dim3(256), 0, s, dd, m, IS, JS);
     else if (comp == 1) hipLaunchKernelGGL(k_adj_mom_combine<1>, dim3(fb), dim3(256), 0, s, dd, m, IS, JS);
     else hipLaunchKernelGGL(k_adj_mom_combine<2>, dim3(fb), dim3(256), 0, s, dd, m, IS, JS);

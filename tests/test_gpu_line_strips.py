@@ -4,7 +4,8 @@ The diagnostic pressure sweep: one, two and four groups of 64 levels a column,
 columns too tall for the strips, strips of 7 and 10 rows that end in a partial
 strip, cell sizes that are no power of two; every field bit for bit against the
 oracle.  One momentum sweep: on strips bit for bit what it is with one launch
-per anti-diagonal.
+per anti-diagonal.  Its transpose: against central differences, for columns of
+one and two groups of levels.
 """
 import numpy as np
 import pytest
@@ -47,3 +48,43 @@ def test_momentum_sweep_kinds(monkeypatch, nii, njj, width):
             out[sw] = s.download()
     for f in FIELDS:
         assert np.array_equal(out["strip"][f].view(np.uint32), out["diag"][f].view(np.uint32)), f
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("comp", [0, 1, 2])
+@pytest.mark.parametrize("nii,njj,vcf,width", [(9, 11, 17, 8), (46, 43, 17, 16), (12, 45, 70, 8), (43, 12, 60, 16)])
+def test_momentum_vjp_edges(nii, njj, vcf, width, comp):
+    # <g, M(x + h d) - M(x - h d)> / 2h against <VJP(g), d>: for random g and d over N
+    # cells both are sums of N terms of random sign, of size sqrt(N) where the
+    # Jacobian is near the identity; the differences' float rounding (6e-8 / 2h with
+    # h = 1e-3) leaves 3e-5 of that, the bound is 1e-3 of it
+    from gral_amd import pf
+    f = ("uk", "vk", "wk")[comp]
+    bl = domain.city_buildings(nii, njj, 2.0, 5, density=0.2, fmin=4.0, fmax=12.0, hmin=3.0, hmax=14.0, margin=2)
+    c = domain.build_case("mv", nii, njj, bl, dx=2.0, vertcellsff=vcf, direction=235.0, z0=0.5, iterations=6)
+    c.simd_width, c.relax = width, 1.0
+    lev = np.zeros(c.uk.shape, dtype=bool)
+    lev[:, :, :c.kadvmax + 2] = True
+    rng = np.random.default_rng(7 + comp)
+    g = np.where(lev, rng.standard_normal(c.uk.shape), 0.0).astype(np.float32)
+    d = np.where(lev, rng.standard_normal(c.uk.shape), 0.0)
+    print(f"[line strips] vjp of {f}, {nii}x{njj}, {c.kadvmax + 2} levels, width {width}", flush=True)
+    with pf.PrognosticFlowfield(c) as s:
+        s.prepare(iterations=6)
+        s.iterate(2)
+        base = {k: v.copy() for k, v in s.download().items() if k in ("uk", "vk", "wk")}
+        s.momentum_sweep(comp)
+        ad = s.momentum_vjp(g)
+        s.restore_ckpt()
+        h = 1e-3 * float(np.abs(base[f][lev]).max())
+        x, y = [], []
+        for sgn in (1.0, -1.0):
+            v = {k: a.copy() for k, a in base.items()}
+            v[f] = (base[f].astype(np.float64) + sgn * h * d).astype(np.float32)
+            s.set_velocity(v["uk"], v["vk"], v["wk"])
+            s.momentum_sweep(comp)
+            x.append(v[f].astype(np.float64))
+            y.append(s.download()[f].astype(np.float64))
+    fd = float((g * (y[0] - y[1])).sum()) / (2 * h)
+    av = float((ad.astype(np.float64) * (x[0] - x[1])).sum()) / (2 * h)
+    assert abs(av - fd) <= 1e-3 * np.sqrt(lev.sum()), (av, fd)
