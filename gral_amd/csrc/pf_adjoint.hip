@@ -77,8 +77,10 @@ __global__ void k_adj_correction(const Dom *__restrict__ ds, AdjArgs a) {
         for (int k = 1 + threadIdx.x; k <= min(KK + 1, VI); k += blockDim.x) a.wb[o + k] = 0.0f;
 }
 
-// S^T on anti-diagonal t of the sweep (a = j1 outer, b = i1 inner, mirrored by
-// IS/JS as in the forward), launched from the last diagonal to the first.
+// S^T runs on strips (pf_launch_adjoint_sweep: 256 x 256 columns of up to 47 levels
+// 1.37 ms, with one launch per anti-diagonal 2.5 ms), whose columns hold 256 levels.  For
+// taller ones: anti-diagonal t of the sweep (a = j1 outer, b = i1 inner, mirrored
+// by IS/JS as in the forward), launched from the last diagonal to the first.
 // One wave per column: the lanes stage the column's vectors and its P, TERMP
 // and ATP in LDS, lane 0 runs the transposed recurrences over LDS in blocks of
 // AU levels whose operands are read before the block's chain.
@@ -173,8 +175,9 @@ __global__ void k_adj_divergence(const Dom *__restrict__ ds, AdjArgs a) {
 }
 
 // One step of the VJP, for forward iteration iter (its sweep directions).
-// n3: floats of one [n2][nkp] field.
-extern "C" int pf_launch_adjoint_step(const Dom *hd, const Dom *dd, const AdjArgs *args, int iter, size_t n3,
+// n3: floats of one [n2][nkp] field; first: the first step of a VJP.
+extern "C" int pf_launch_adjoint_sweep(const Dom *hd, const Dom *dd, const AdjArgs *args, int IS, int JS, hipStream_t s);
+extern "C" int pf_launch_adjoint_step(const Dom *hd, const Dom *dd, const AdjArgs *args, int iter, size_t n3, int first,
                                       hipStream_t s) {
     const Dom &h = *hd;
     int IS = 1, JS = 1;
@@ -186,18 +189,24 @@ extern "C" int pf_launch_adjoint_step(const Dom *hd, const Dom *dd, const AdjArg
     }
     AdjArgs a = *args;
     const unsigned fb = (unsigned)((n3 + 255) / 256);
-    hipLaunchKernelGGL(k_adj_fill, dim3(fb), dim3(256), 0, s, a.pb, n3);
-    hipLaunchKernelGGL(k_adj_fill, dim3(fb), dim3(256), 0, s, a.qb, n3);
-    hipLaunchKernelGGL(k_adj_fill, dim3(fb), dim3(256), 0, s, a.mb, n3);
-    hipLaunchKernelGGL(k_adj_fill, dim3(fb), dim3(256), 0, s, a.db, n3);
+    auto fill = [&](float *p) { hipLaunchKernelGGL(k_adj_fill, dim3(fb), dim3(256), 0, s, p, n3); };
+    // every step writes PB and DB of the same cells: DB's others are cleared once
+    if (first) fill(a.db);
     hipLaunchKernelGGL(k_adj_correction, dim3((unsigned)((h.nii - 2) * (h.njj - 2))), dim3(64), 0, s, dd, a);
-    const int oa = 2, ob = h.njj - 1, ia = 2, ib = h.nii - 1;
-    const int nd = (ob - oa) + (ib - ia) + 1;
-    const size_t shm = sizeof(float) * 6 * (size_t)h.nkp;
-    for (int t = nd - 1; t >= 0; --t) {
-        const int amin = max(oa, oa + t - (ib - ia)), amax = min(ob, oa + t);
-        if (amax >= amin)
-            hipLaunchKernelGGL(k_adj_pressure, dim3((unsigned)(amax - amin + 1)), dim3(AWAVE), shm, s, dd, a, t, IS, JS);
+    if (a.hand) {
+        const int e = pf_launch_adjoint_sweep(hd, dd, args, IS, JS, s);
+        if (e) return e;
+    } else {
+        fill(a.qb);
+        if (first) fill(a.mb);
+        const int oa = 2, ob = h.njj - 1, ia = 2, ib = h.nii - 1;
+        const int nd = (ob - oa) + (ib - ia) + 1;
+        const size_t shm = sizeof(float) * 6 * (size_t)h.nkp;
+        for (int t = nd - 1; t >= 0; --t) {
+            const int amin = max(oa, oa + t - (ib - ia)), amax = min(ob, oa + t);
+            if (amax >= amin)
+                hipLaunchKernelGGL(k_adj_pressure, dim3((unsigned)(amax - amin + 1)), dim3(AWAVE), shm, s, dd, a, t, IS, JS);
+        }
     }
     hipLaunchKernelGGL(k_adj_divergence, dim3((unsigned)((h.nii - 1) * (h.njj - 1))), dim3(64), 0, s, dd, a);
     return (int)hipGetLastError();

@@ -49,7 +49,7 @@ extern "C" int pf_launch_projection(const Dom *hd, const Dom *dd, int iter, hipS
 extern "C" int pf_launch_momentum_sweep(const Dom *hd, const Dom *dd, int comp, int IS, int JS, hipStream_t s);
 extern "C" int pf_launch_momentum_vjp(const Dom *hd, const Dom *dd, const MomAdj *ma, int comp, int IS, int JS,
                                       hipStream_t s);
-extern "C" int pf_launch_adjoint_step(const Dom *hd, const Dom *dd, const AdjArgs *args, int iter, size_t n3,
+extern "C" int pf_launch_adjoint_step(const Dom *hd, const Dom *dd, const AdjArgs *args, int iter, size_t n3, int first,
                                       hipStream_t s);
 
 namespace {
@@ -197,8 +197,9 @@ struct gral_pf_handle {
     // adjoint of the pressure-correction steps (gral_pf_forward_ckpt / gral_pf_vjp)
     std::vector<float> app, abp, atp;   // per-level pressure coefficients of the prologue
     float *adj = nullptr;           // ub vb wb pb qb mb db, checkpoint uk vk wk, ptab[2] ttab[2]: 15 fields
-    float *mom_rec = nullptr;       // momentum_vjp's column data and hand-off words (per-diagonal situations)
-    unsigned long long *mom_hand = nullptr;
+    int4 *adj_col = nullptr;        // levels of the transposed pressure sweep's columns
+    float *mom_rec = nullptr;       // momentum_vjp's column data (per-diagonal situations)
+    unsigned long long *adj_hand = nullptr;   // the transposed sweeps' hand-off words (per-diagonal situations)
     int *adj_src = nullptr;         // stale-top source column per column, for IS = +1 and -1
     int adj_first = 0, adj_n = 0;   // iterations of the last forward
     int mom_comp = -1, mom_is = 1, mom_js = 1;   // the last gral_pf_momentum_sweep: component, directions
@@ -399,8 +400,9 @@ static void free_device(gral_pf_handle *h) {
     if (h->graphs) h->graphs->clear();
     h->adj = nullptr;
     h->adj_src = nullptr;
+    h->adj_col = nullptr;
     h->mom_rec = nullptr;
-    h->mom_hand = nullptr;
+    h->adj_hand = nullptr;
     h->adj_n = 0;
     h->mom_comp = -1;
     h->mom_vjp_ok = false;
@@ -1374,7 +1376,15 @@ static int adj_alloc(gral_pf_handle *h) {
     float *a;
     int *src;
     int rc;
-    if ((rc = dalloc(h, &a, 15 * n3)) || (rc = dalloc(h, &src, 2 * n2))) return rc;
+    int4 *col;
+    if ((rc = dalloc(h, &a, 15 * n3)) || (rc = dalloc(h, &src, 2 * n2)) || (rc = dalloc(h, &col, n2))) return rc;
+    std::vector<int4> cv(n2, int4{1 << 20, -1, 0, 0});   // levels of the columns the pressure sweep visits
+    for (int i = 2; i <= h->nii - 1; ++i)
+        for (int j = 2; j <= h->njj - 1; ++j) {
+            const size_t c = h->i2(i, j);
+            if (h->adv[c] == 1) cv[c] = int4{h->kk[c] + 1, h->vi[c], 0, 0};
+        }
+    HIPCHK(h, hipMemcpyAsync(col, cv.data(), n2 * sizeof(int4), hipMemcpyHostToDevice, h->stream));
     std::vector<float> tp, tt;
     std::vector<int> sv;
     for (int v = 0; v < 2; ++v) {
@@ -1386,6 +1396,23 @@ static int adj_alloc(gral_pf_handle *h) {
     }
     h->adj = a;
     h->adj_src = src;
+    h->adj_col = col;
+    return 0;
+}
+
+// the transposed sweeps' hand-off words: the strip sweeps', or for a per-diagonal
+// situation words of their own
+static int adj_hand(gral_pf_handle *h, unsigned long long *&p) {
+    p = h->d.hand;
+    if (p) return 0;
+    if (!h->adj_hand) {
+        unsigned long long *q;
+        int rc = dalloc(h, &q, 2 * h->d.hand_words);
+        if (rc) return rc;
+        HIPCHK(h, hipMemsetAsync(q, 0, 2 * h->d.hand_words * sizeof(unsigned long long), h->stream));
+        h->adj_hand = q;
+    }
+    p = h->adj_hand;
     return 0;
 }
 
@@ -1459,6 +1486,14 @@ extern "C" int gral_pf_vjp(gral_pf_handle *h, const float *du, const float *dv, 
     AdjArgs g{};
     g.ub = a; g.vb = a + n3; g.wb = a + 2 * n3; g.pb = a + 3 * n3; g.qb = a + 4 * n3; g.mb = a + 5 * n3; g.db = a + 6 * n3;
     int rc;
+    g.col = h->adj_col;
+    if (h->nkp <= 256) {
+        if (adj_hand(h, g.hand) == 0) g.handq = g.hand + h->d.hand_words;
+        else {                                           // no memory for them: per anti-diagonal
+            (void)hipGetLastError();
+            h->err.clear();
+        }
+    }
     if ((rc = put_raw(h, g.ub, du)) || (rc = put_raw(h, g.vb, dv)) || (rc = put_raw(h, g.wb, dw))) return rc;
     HIPCHK(h, hipEventRecord(h->ev0, h->stream));
     for (int q = h->adj_n - 1; q >= 0; --q) {
@@ -1472,11 +1507,14 @@ extern "C" int gral_pf_vjp(gral_pf_handle *h, const float *du, const float *dv, 
         g.ptab = a + (size_t)(10 + v) * n3;
         g.ttab = a + (size_t)(12 + v) * n3;
         g.src = h->adj_src + (size_t)v * n2;
-        int e = pf_launch_adjoint_step(&h->d, h->dd, &g, it, n3, h->stream);
+        int e = pf_launch_adjoint_step(&h->d, h->dd, &g, it, n3, q == h->adj_n - 1, h->stream);
         if (e) return fail(h, GRAL_PF_EDEVICE, std::string("vjp: launch failed: ") + hipGetErrorString((hipError_t)e));
     }
     HIPCHK(h, hipEventRecord(h->ev1, h->stream));
     HIPCHK(h, hipEventSynchronize(h->ev1));
+    int serr = 0;
+    HIPCHK(h, hipMemcpy(&serr, h->d.sync, sizeof(int), hipMemcpyDeviceToHost));
+    if (serr) return fail(h, GRAL_PF_EDEVICE, "vjp: a strip wait timed out (results invalid)");
     float ms = 0;
     HIPCHK(h, hipEventElapsedTime(&ms, h->ev0, h->ev1));
     h->timing = gral_pf_timing{};
@@ -1587,19 +1625,11 @@ extern "C" int gral_pf_momentum_vjp(gral_pf_handle *h, const float *dx, float *g
     // the columns' data: in the sweeps' coefficient records, which hold nothing
     // between two sweeps, or where the situation has none in a buffer of its own
     float *rec = h->d.planes;
-    m.hand = h->d.hand;
     if (!h->d.tiled) {
-        if (!h->mom_rec) {
-            float *q;
-            unsigned long long *hw;
-            if ((rc = dalloc(h, &hw, h->d.hand_words)) || (rc = dalloc(h, &q, 8 * n3 + 4))) return rc;
-            HIPCHK(h, hipMemsetAsync(hw, 0, h->d.hand_words * sizeof(unsigned long long), h->stream));
-            h->mom_rec = q;
-            h->mom_hand = hw;
-        }
+        if (!h->mom_rec && (rc = dalloc(h, &h->mom_rec, 8 * n3 + 4))) return rc;
         rec = h->mom_rec;
-        m.hand = h->mom_hand;
     }
+    if ((rc = adj_hand(h, m.hand))) return rc;
     m.T = rec; m.P = rec + n3; m.C = rec + 2 * n3; m.Q = rec + 3 * n3;
     m.ca = rec + 4 * n3; m.cb = rec + 5 * n3; m.cc = rec + 6 * n3;
     m.col = reinterpret_cast<int4 *>((reinterpret_cast<uintptr_t>(rec + 7 * n3) + 15) & ~(uintptr_t)15);

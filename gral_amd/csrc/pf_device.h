@@ -168,6 +168,8 @@ struct AdjArgs {
     float *db;                  // adjoint of DIV
     const float *ptab, *ttab;   // P and TERMP of every column for this step's IS
     const int *src;             // per column: i of the column whose Q the elimination starts from, or -1
+    const int4 *col;            // per column: KKART+1, VI (swept columns; else first > last)
+    unsigned long long *hand, *handq;   // the strips' hand-off words, laid out as Dom::hand; null: per anti-diagonal
 };
 
 // Buffers of the adjoint of one momentum sweep (pf_kernels.hip), each

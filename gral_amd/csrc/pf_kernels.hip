@@ -2534,8 +2534,10 @@ static inline int lds_limit(const void *kern, size_t bytes);
 // own a sweep row each, wave R runs the recurrences (lane = row) and hands the
 // last row's results on; the steps and phases are those of k_ml_strip, without
 // a control wave: a row leaves its column's levels in LDS a step ahead.  Bound by
-// the recurrences.  OP supplies the operands and the recurrences (DgOp, MomOp);
-// M: 64-level groups of a column.
+// the recurrences.  OP supplies the operands and the recurrences (DgOp, MomOp,
+// PrAdjOp); M: 64-level groups of a column.  OP::SCRATCH: each step has a row of
+// values by level that its columns, one after another along the rows, take (and
+// clear) at their own levels and add to at the level above them; it starts at 0.
 // ------------------------------------------------------------------------
 struct LineSweep {
     int ni, nj;                  // rows, steps of the sweep
@@ -2544,16 +2546,17 @@ struct LineSweep {
     int *sync;                   // [0] error flag, [1] tag base, [ticket] 0 before the launch
     int ticket, kind;            // kind: names the sweep in the tag
     unsigned long long *hand;    // [strips][nj][nk]
+    unsigned long long *handq;   // [strips][nj][nk], the row scratch of the OPs that have one
 };
 struct LineCol { int lo, hi, x; };                             // its levels (lo > hi: none) and the OP's own datum
 typedef int __attribute__((address_space(4))) ci32;
 __host__ __device__ inline int line_len(int nk) { return (nk + 2 * CHK - 1) / CHK * CHK; }      // one spare chunk
 template <class OP>
-__host__ __device__ inline int line_arrays() { return 3 + 2 * OP::NBUF; }
+__host__ __device__ inline int line_arrays() { return 3 + 2 * OP::NBUF + OP::SCRATCH; }
 template <class OP>
 static size_t line_lds(int nk, int rows) {
     const int len = line_len(nk);
-    return sizeof(float) * ((size_t)rows * strip_stride(line_arrays<OP>(), len) + (size_t)OP::NTAB * len) + 32 * sizeof(int4) + 16;
+    return sizeof(float) * ((size_t)rows * strip_stride(line_arrays<OP>(), len) + (size_t)(OP::NTAB + OP::SCRATCH * RING) * len) + 32 * sizeof(int4) + 16;
 }
 template <class OP, int M>
 __global__ __launch_bounds__(STRIP_WAVES * WAVE) void k_line_strip(OP op, LineSweep w) {
@@ -2564,9 +2567,10 @@ __global__ __launch_bounds__(STRIP_WAVES * WAVE) void k_line_strip(OP op, LineSw
     const int r = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
     gi32 *sync = (gi32 *)w.sync;
     // per row: D (or what the recurrences make of it), the results of even and odd
-    // steps, the operands of even and odd steps
+    // steps, the operands of even and odd steps, the scratch values taken
     float *tab = sm + (size_t)R * rs;                         // [NTAB][len] operands that depend on the level alone
-    int4 *sinfo = (int4 *)(tab + OP::NTAB * len);             // [2][16] levels of the rows' columns by step parity
+    float *ring = tab + OP::NTAB * len;                       // [RING][len] row scratch of a step (slot: step mod RING)
+    int4 *sinfo = (int4 *)(ring + OP::SCRATCH * RING * len);             // [2][16] levels of the rows' columns by step parity
     int *sctl = (int *)(sinfo + 32);
     const LineCol none{1 << 20, -1, 0};
     if (threadIdx.x == 0) sctl[0] = __hip_atomic_fetch_add(&sync[w.ticket], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -2576,12 +2580,13 @@ __global__ __launch_bounds__(STRIP_WAVES * WAVE) void k_line_strip(OP op, LineSw
     const int B = __builtin_amdgcn_readfirstlane(sctl[0]);
     if (B >= nstrip) return;                                  // uniform over the workgroup
     const unsigned tag = 8u * (unsigned)sync[1] + (unsigned)w.kind;
-    gu64 *hand = (gu64 *)w.hand;
+    gu64 *hand = (gu64 *)w.hand, *handq = (gu64 *)w.handq;
     if (r == R) {                                             // chain wave
         __builtin_amdgcn_s_setprio(3);
         float *L = sm + (size_t)(lane < R ? lane : 0) * rs;
         const float *xl = sm + (size_t)(R - 1) * rs + len;
         gu64 *h = hand + ((size_t)B * w.nj - R) * nk;         // + s*nk: the last row's column of step s - 1
+        gu64 *hq = handq + ((size_t)B * w.nj - R) * nk;
         const bool send = B + 1 < nstrip;
         int lo = none.lo, hi = none.hi;
         auto send_last = [&](int s) {
@@ -2594,6 +2599,7 @@ __global__ __launch_bounds__(STRIP_WAVES * WAVE) void k_line_strip(OP op, LineSw
             for (int m = 0; m < M; ++m) {
                 const int k = lane + WAVE * m;
                 if (k < nk) hand_put(h + (size_t)s * nk + k, (k >= a && k <= b) ? v[m] : 0.0f, tag);
+                if (OP::SCRATCH && k < nk) hand_put(hq + (size_t)s * nk + k, ring[((s - R) & (RING - 1)) * len + k], tag);
             }
         };
         lds_barrier();                                        // the rows' operands and levels of step 0
@@ -2607,9 +2613,12 @@ __global__ __launch_bounds__(STRIP_WAVES * WAVE) void k_line_strip(OP op, LineSw
             const int NC = len / CHK;
             const int clo = NC - __builtin_amdgcn_readfirstlane(row_max(on ? NC - lo / CHK : 0));
             const int chi = __builtin_amdgcn_readfirstlane(row_max(on ? lo / CHK : 0));
-            const int ct = __builtin_amdgcn_readfirstlane(row_max(on ? hi / CHK : 0));
+            const int ct = __builtin_amdgcn_readfirstlane(row_max(on ? (hi + OP::SCRATCH) / CHK : 0));
             lds_barrier();                                    // the rows' sources are assembled
-            if (on) op.chain(L, L + (1 + (s & 1)) * len, L + (3 + (s & 1) * OP::NBUF) * len, tab, len, lo, clo, chi, ct);
+            if (on) {
+                op.chain(L, L + (1 + (s & 1)) * len, L + (3 + (s & 1) * OP::NBUF) * len, tab, len, lo, clo, chi, ct);
+                if (OP::SCRATCH) ring[((s - lane) & (RING - 1)) * len + hi + 1] += L[hi + 1];
+            }
             lds_barrier();                                    // the recurrences are done
         }
         send_last(nsteps);
@@ -2623,7 +2632,7 @@ __global__ __launch_bounds__(STRIP_WAVES * WAVE) void k_line_strip(OP op, LineSw
     int l2 = -r - 1;                                          // step (of this row) q2 belongs to
     typename OP::Raw raw[M];
     typename OP::In in[M] = {};
-    unsigned long long hw[M];
+    unsigned long long hw[M], hs[M];
     int kb[M];                                                // byte offsets of the lane's levels in an array
 #pragma unroll
     for (int m = 0; m < M; ++m) kb[m] = 4 * min(lane + WAVE * m, len - 1);
@@ -2636,8 +2645,12 @@ __global__ __launch_bounds__(STRIP_WAVES * WAVE) void k_line_strip(OP op, LineSw
     };
     auto issue = [&]() {                                      // loads of the column at c2, l = l2 - 1
         c1 = c2;
-        if (c1.lo > c1.hi) return;
         const int l = l2 - 1, c = c00 + l * w.dj;
+        if (OP::SCRATCH && from_prev && l >= 0 && l < w.nj)
+#pragma unroll
+            for (int m = 0; m < M; ++m)
+                if (lane + WAVE * m < nk) hs[m] = hand_get(handq + ((size_t)(B - 1) * w.nj + l) * nk + lane + WAVE * m);
+        if (c1.lo > c1.hi) return;
 #pragma unroll
         for (int m = 0; m < M; ++m) {
             const int k = lane + WAVE * m;
@@ -2647,6 +2660,13 @@ __global__ __launch_bounds__(STRIP_WAVES * WAVE) void k_line_strip(OP op, LineSw
     };
     auto work_up = [&](int s) {                               // c1 is the column of step s
         if (lane == 0) sinfo[(s & 1) * 16 + r] = make_int4(c1.lo, c1.hi, 0, 0);
+        if (OP::SCRATCH && r == 0 && s < w.nj)                // the scratch of step s as the rows before this strip left it
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+                const int k = lane + WAVE * m;
+                if (B > 0) hwait.wait(handq + ((size_t)(B - 1) * w.nj + s) * nk + k, k < nk, tag, hs[m]);
+                if (k < len) ring[(s & (RING - 1)) * len + k] = (B > 0 && k < nk) ? __uint_as_float((unsigned)hs[m]) : 0.0f;
+            }
         if (c1.lo > c1.hi) return;
         const int ob = rowb + 4 * (3 + (s & 1) * OP::NBUF) * len;
 #pragma unroll
@@ -2693,7 +2713,13 @@ __global__ __launch_bounds__(STRIP_WAVES * WAVE) void k_line_strip(OP op, LineSw
                 const int k = lane + WAVE * m;
                 const float a = (k >= ci.lo && k <= ci.hi) ? vi[m] : vin[m], b = (k >= cm.lo && k <= cm.hi) ? vj[m] : 0.0f;
                 const float d = op.source(in[m], k, c0, a, b);
-                if (k < len) lds_at(sm, rowb + 4 * k) = (k >= c0.lo && k <= c0.hi) ? d : 0.0f;
+                const bool on = k >= c0.lo && k <= c0.hi;
+                if (k < len) lds_at(sm, rowb + 4 * k) = on ? d : 0.0f;
+                if (OP::SCRATCH && k < len) {
+                    float *q = ring + ((s - r) & (RING - 1)) * len + k;
+                    lds_at(sm, rowb + 4 * ((3 + 2 * OP::NBUF) * len + k)) = on ? *q : 0.0f;
+                    if (on) *q = 0.0f;
+                }
             }
         }
         lds_barrier();
@@ -2787,7 +2813,7 @@ __global__ void k_dg_divergence(DiagArgs g) {
 // cycles with their LDS accesses): 5.5 ms a sweep of 397 x 397 columns of 221
 // levels, 11.1 ms with one launch per anti-diagonal (4 to 12 rows a strip: within 3%).
 struct DgOp {
-    enum { NTAB = 4, NBUF = 0 };                              // tables: ATP, TERMP, PIMP, DZK
+    enum { NTAB = 4, NBUF = 0, SCRATCH = 0 };                              // tables: ATP, TERMP, PIMP, DZK
     DiagArgs g;
     float rx, ry;                                             // 1 / DXK, 1 / DYK
     int p2, jp;                                               // both powers of two (their reciprocals are exact); JS == 1
@@ -3003,7 +3029,7 @@ extern "C" int pf_launch_diagnostic(const DiagArgs *ga, int iterations, hipStrea
         if (strips) {
             const int i0 = IS == -1 ? ib : ia, j0 = JS == -1 ? ob : oa;
             const DgOp op{g, 1.0f / g.dxk, 1.0f / g.dyk, pow2(g.dxk) && pow2(g.dyk), JS == 1};
-            const LineSweep w{ib - ia + 1, ob - oa + 1, i0 * g.nj2 + j0, IS * g.nj2, JS, g.nkh, g.sync, 1 + it, it, g.hand};
+            const LineSweep w{ib - ia + 1, ob - oa + 1, i0 * g.nj2 + j0, IS * g.nj2, JS, g.nkh, g.sync, 1 + it, it, g.hand, nullptr};
             const int e = g.nkh <= 2 * WAVE ? launch_line<DgOp, 2>(op, w, s) : launch_line<DgOp, 4>(op, w, s);
             if (e) return e;
         } else
@@ -4218,7 +4244,7 @@ __device__ __forceinline__ float adj_mom_pb(float db, float cb, float cc, float 
 // with the whole column's transpose in one launch per anti-diagonal 19.5 ms.
 template <int COMP>
 struct MomOp {
-    enum { NTAB = 1, NBUF = 3 };                              // table: DYK DZK (U) or DXK DZK (V); operands: P, C, T
+    enum { NTAB = 1, NBUF = 3, SCRATCH = 0 };                              // table: DYK DZK (U) or DXK DZK (V); operands: P, C, T
     MomAdj m;
     const float *dzk;
     float h, relax;                                           // DYK (U), DXK (V)
@@ -4573,7 +4599,7 @@ extern "C" int pf_launch_momentum_vjp(const Dom *hd, const Dom *dd, const MomAdj
             // the sweep's order reversed: from its last row and column back
             const int i0 = IS == 1 ? h.nii - 1 : 2, j0 = JS == 1 ? h.njj - 1 : 2;
             const MomOp<C> op{m, h.dzk, C == 0 ? h.dyk : h.dxk, h.relax, h.nkp};
-            const LineSweep w{ni, nj, i0 * h.nj2 + j0, -IS * h.nj2, -JS, h.nkp, h.sync, SYNC_BLOCK0, 6, m.hand};
+            const LineSweep w{ni, nj, i0 * h.nj2 + j0, -IS * h.nj2, -JS, h.nkp, h.sync, SYNC_BLOCK0, 6, m.hand, nullptr};
             e = h.nkp <= WAVE ? launch_line<MomOp<C>, 1>(op, w, s) : launch_line<MomOp<C>, 2>(op, w, s);
             if (!e) hipLaunchKernelGGL(k_adj_mom<C>, dim3(ncol), dim3(WAVE), shm, s, dd, m, IS, JS);
         }
@@ -4585,4 +4611,118 @@ extern "C" int pf_launch_momentum_vjp(const Dom *hd, const Dom *dd, const MomAdj
     else if (comp == 1) hipLaunchKernelGGL(k_adj_mom_combine<1>, dim3(fb), dim3(256), 0, s, dd, m, IS, JS);
     else hipLaunchKernelGGL(k_adj_mom_combine<2>, dim3(fb), dim3(256), 0, s, dd, m, IS, JS);
     return (int)hipGetLastError();
+}
+
+// ------------------------------------------------------------------------
+// The transposed pressure sweep (S^T of pf_adjoint.hip) on strips, in the reverse
+// order of the sweep.  x_bar[k] = pb[k] + what the two successors hand down, then
+// the transposed substitution x_bar[k-1] += P[k] x_bar[k] top-down with Q_bar[k] =
+// (Q_bar handed by later columns) + x_bar[k], and the transposed elimination
+// bottom-up: DIM_bar[k] = TERMP[k] (Q_bar[k] + carry), carry = ATP[k] TERMP[k] (..).
+// The carry above the column's top goes to the last earlier column of the same
+// sweep row that holds level VI+1: the row scratch.  Bound by the recurrences (3500
+// of a step's 5500 cycles, 66 levels of the rows' columns together): 1.37 ms a
+// sweep of 254 x 254 columns, 2.5 ms with one launch per anti-diagonal.
+// ------------------------------------------------------------------------
+struct PrAdjOp {
+    enum { NTAB = 3, NBUF = 3, SCRATCH = 1 };                 // tables: DYK DZK/DXK, DXK DZK/DYK, ATP; operands: P, TERMP, ATP*TERMP
+    AdjArgs a;
+    const float *dzk, *atp;
+    float dxk, dyk, dtime, sgn;                               // sgn: the sign with which the columns along j enter DIM
+    int nkp;
+    struct Raw { float x, p, t; };
+    struct In { float x, ui, uj; };
+    __device__ __forceinline__ float table(int q, int k) const {
+        return q == 0 ? dyk * dzk[k] / dxk : q == 1 ? dxk * dzk[k] / dyk : atp[k];
+    }
+    __device__ __forceinline__ LineCol levels(int c) const {
+        const int4 v = ldc4i((const DomG::P<const int4>)a.col + c);
+        return LineCol{v.x, v.y, 0};
+    }
+    __device__ __forceinline__ void load(Raw &q, int c, int, int, int k) const {
+        const size_t o = (size_t)c * nkp + k;
+        q.x = ((const gf32 *)a.pb)[o];
+        q.p = ((const gf32 *)a.ptab)[o];
+        q.t = ((const gf32 *)a.ttab)[o];
+    }
+    __device__ __forceinline__ void stage(const Raw &q, In &i, bool on, int k, float *buf, int len, const float *tab) const {
+        buf[0] = on ? q.p : 0.0f;
+        buf[len] = on ? q.t : 0.0f;
+        buf[2 * len] = on ? tab[2 * len + k] * q.t : 0.0f;
+        i.x = q.x;
+        i.ui = tab[k];
+        i.uj = tab[len + k];
+    }
+    __device__ __forceinline__ float source(const In &i, int, const LineCol &, float vi, float vj) const {
+        return i.x + vi * i.ui + sgn * vj * i.uj;
+    }
+    __device__ __forceinline__ void chain(float *L, float *N, float *buf, const float *, int len, int, int clo, int,
+                                          int ct) const {
+        const float *E = L + (3 + 2 * NBUF) * len, *P = buf, *T = buf + len + clo * CHK, *A = buf + 2 * len + clo * CHK;
+        {
+            float t = 0.0f;                                   // P[k+1] x_bar[k+1]
+            Chunk d[2], e[2], p[2];
+            int o = ct * CHK;
+            d[0] = ld_chunk(L + o); e[0] = ld_chunk(E + o); p[0] = ld_chunk(P + o);
+            for (int c = ct; c >= clo;) {
+#pragma unroll
+                for (int h8 = 0; h8 < CHK_BLOCK; ++h8) {
+                    if (c < clo) break;
+                    const int k = h8 & 1, n = k ^ 1, on = max(o - CHK, 0);
+                    d[n] = ld_chunk(L + on); e[n] = ld_chunk(E + on); p[n] = ld_chunk(P + on);
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int u = CHK - 1; u >= 0; --u) {
+                        const float x = d[k].v[u] + t;
+                        t = p[k].v[u] * x;
+                        e[k].v[u] += x;
+                    }
+                    st_chunk(L + o, e[k]);
+                    o = on;
+                    --c;
+                }
+            }
+        }
+        float carry = 0.0f;
+        float *Q = L + clo * CHK;
+        N += clo * CHK;
+        Chunk q[2], t[2], b[2];
+        q[0] = ld_chunk(Q); t[0] = ld_chunk(T); b[0] = ld_chunk(A);
+        for (int c = clo; c <= ct;) {
+#pragma unroll
+            for (int h8 = 0; h8 < CHK_BLOCK; ++h8) {
+                if (c > ct) break;
+                const int k = h8 & 1, n = k ^ 1;
+                q[n] = ld_chunk(Q + CHK); t[n] = ld_chunk(T + CHK); b[n] = ld_chunk(A + CHK);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int u = 0; u < CHK; ++u) {
+                    const float qt = q[k].v[u] + carry;
+                    carry = b[k].v[u] * qt;
+                    t[k].v[u] *= qt;
+                    q[k].v[u] = qt;
+                }
+                st_chunk(N, t[k]);
+                st_chunk(Q, q[k]);                            // at VI+1: the carry
+                Q += CHK; T += CHK; A += CHK; N += CHK;
+                ++c;
+            }
+        }
+    }
+    __device__ __forceinline__ void store(int c, int k, const LineCol &q, float x) const {
+        if (k >= q.lo && k <= q.hi) ((gf32 *)a.db)[(size_t)c * nkp + k] = x / dtime;      // DIM = DIV / DTIME + ...
+    }
+};
+// launches it; hipErrorInvalidValue where the columns have more levels than the strips hold
+extern "C" int pf_launch_adjoint_sweep(const Dom *hd, const Dom *dd, const AdjArgs *args, int IS, int JS, hipStream_t s) {
+    const Dom &h = *hd;
+    if (h.nkp > 4 * WAVE) return (int)hipErrorInvalidValue;
+    const int ni = h.nii - 2, nj = h.njj - 2;
+    if (ni < 1 || nj < 1) return 0;
+    hipLaunchKernelGGL(k_zero_rows, dim3((unsigned)((5 * h.sync_stride + 255) / 256)), dim3(256), 0, s, dd, 0);
+    const int i0 = IS == 1 ? h.nii - 1 : 2, j0 = JS == 1 ? h.njj - 1 : 2;
+    const PrAdjOp op{*args, h.dzk, h.atp, h.dxk, h.dyk, h.dtime, JS == 1 ? 1.0f : -1.0f, h.nkp};
+    const LineSweep w{ni, nj, i0 * h.nj2 + j0, -IS * h.nj2, -JS, h.nkp, h.sync, SYNC_BLOCK0, 7, args->hand, args->handq};
+    return h.nkp <= WAVE ? launch_line<PrAdjOp, 1>(op, w, s) : h.nkp <= 2 * WAVE ? launch_line<PrAdjOp, 2>(op, w, s) :
+                                                                                  launch_line<PrAdjOp, 4>(op, w, s);
 }

@@ -5,7 +5,8 @@ columns too tall for the strips, strips of 7 and 10 rows that end in a partial
 strip, cell sizes that are no power of two; every field bit for bit against the
 oracle.  One momentum sweep: on strips bit for bit what it is with one launch
 per anti-diagonal.  Its transpose: against central differences, for columns of
-one and two groups of levels.
+one and two groups of levels.  The transposed pressure sweep: against the oracle
+in float64.
 """
 import numpy as np
 import pytest
@@ -88,3 +89,44 @@ def test_momentum_vjp_edges(nii, njj, vcf, width, comp):
     fd = float((g * (y[0] - y[1])).sum()) / (2 * h)
     av = float((ad.astype(np.float64) * (x[0] - x[1])).sum()) / (2 * h)
     assert abs(av - fd) <= 1e-3 * np.sqrt(lev.sum()), (av, fd)
+
+
+VJP = [
+    # one, two and four groups of 64 levels; strips of 7 and 10 rows; columns cut off by the grid's top, whose
+    # eliminations start from an earlier column's value; columns per anti-diagonal
+    dict(nii=9, njj=11, vcf=9), dict(nii=46, njj=43, vcf=17, hmax=30.0), dict(nii=12, njj=45, vcf=70),
+    dict(nii=14, njj=13, vcf=63, tower=263.0), dict(nii=26, njj=24, vcf=16, hmax=60.0, dz1=2.0, stretch=1.2),
+    dict(nii=24, njj=60, vcf=12, hmax=60.0, dz1=2.0, stretch=1.25), dict(nii=18, njj=16, vcf=8, sweep="diag"),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("spec", VJP, ids=lambda s: "-".join(f"{k}{v}" for k, v in s.items()))
+def test_window_vjp_edges(monkeypatch, spec):
+    # <g, F(x + d) - F(x)> by the oracle in float64 against <VJP(g), d>: both of size
+    # sqrt(N) for random g and d over N cells; float32 rounding over the window's
+    # sweeps (6e-8 times some hundred operations) is below the bound of 1e-4 of that
+    from gral_amd import pf
+    from oracle import pyoracle
+    from tests.test_gpu_adjoint import _direction, _dot, _shifted
+    spec = dict(spec)
+    monkeypatch.setenv("GRAL_PF_SWEEP", spec.pop("sweep", "strip"))
+    vcf, hmax, tower = spec.pop("vcf"), spec.pop("hmax", 14.0), spec.pop("tower", None)
+    bl = domain.city_buildings(spec["nii"], spec["njj"], 2.0, 5, density=0.2, fmin=4.0, fmax=12.0, hmin=3.0, hmax=hmax, margin=2)
+    if tower:
+        bl.append(domain.Building(6, 9, 5, 8, tower))
+    c = domain.build_case("wv", buildings=bl, dx=2.0, vertcellsff=vcf, direction=235.0, z0=0.5, iterations=4, **spec)
+    lev = np.zeros(c.uk.shape, dtype=bool)
+    lev[:, :, :c.kadvmax + 2] = True
+    rng = np.random.default_rng(3)
+    g = tuple(np.where(lev, rng.standard_normal(c.uk.shape), 0.0).astype(np.float32) for _ in range(3))
+    print(f"[line strips] window vjp {c.nii}x{c.njj}, {c.kadvmax + 2} levels", flush=True)
+    with pf.PrognosticFlowfield(c) as s:
+        s.prepare(iterations=4)
+        s.forward_ckpt(4)
+        v = s.vjp(*g)
+    d = _direction(c, 11)
+    base = pyoracle.run(c, iterations=4, project=0, fp64=True)
+    pert = pyoracle.run(_shifted(c, d, 1.0), iterations=4, project=0, fp64=True)
+    lhs = _dot(g, [pert[f] - base[f] for f in ("uk", "vk", "wk")])
+    assert abs(_dot(v, d) - lhs) <= 1e-4 * np.sqrt(3.0 * lev.sum()), (_dot(v, d), lhs)
