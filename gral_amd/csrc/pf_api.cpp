@@ -14,6 +14,7 @@
 #include <cstdlib>
 #include <atomic>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <thread>
@@ -625,13 +626,20 @@ static int move_all(gral_pf_handle *h, bool to_dev, const std::vector<Move> &mv)
         if (h->stage_buf) (void)hipHostFree(h->stage_buf);
         h->stage_buf = nullptr;
         h->stage_bytes = 0;
-        if (hipHostMalloc(&h->stage_buf, slots * slot_bytes, hipHostMallocDefault) != hipSuccess) {
+        if (hipHostMalloc(&h->stage_buf, slots * slot_bytes, hipHostMallocDefault) == hipSuccess) h->stage_bytes = slots * slot_bytes;
+        else {
+            (void)hipGetLastError();
             h->stage_buf = nullptr;
-            return fail(h, GRAL_PF_ENOMEM, "hipHostMalloc of the staging buffer failed");
         }
-        h->stage_bytes = slots * slot_bytes;
     }
+    // no pinned memory left: a pageable ring, which the copies below take as well
+    std::unique_ptr<char, void (*)(void *)> pageable(nullptr, std::free);
     char *ring = static_cast<char *>(h->stage_buf);
+    if (!ring) {
+        pageable.reset(static_cast<char *>(std::malloc(slots * slot_bytes)));
+        ring = pageable.get();
+        if (!ring) return fail(h, GRAL_PF_ENOMEM, "no memory for the staging buffer");
+    }
     std::vector<int> chunk_of(np);
     for (int c = 0; c < n; ++c) std::fill(chunk_of.begin() + ch[c].p0, chunk_of.begin() + ch[c].p1, c);
     std::vector<std::atomic<int>> done(n);
