@@ -7,11 +7,13 @@
 //                      the reference updates columns in place in lexicographic
 //                      sweep order (a outer, b inner).  A column depends on the
 //                      new values of (a-1,b) and (a,b-1) only, so all columns of
-//                      one anti-diagonal a+b=t are independent.  Each pass is a
-//                      sequence of per-diagonal launches; one 64-lane wavefront
-//                      per column computes the coefficients of all levels in
-//                      parallel (lanes over k), stages them in LDS, and one lane
-//                      runs the Thomas recurrences, which are serial in k.
+//                      one anti-diagonal a+b=t are independent.  A pass is one
+//                      launch of strips: workgroups of consecutive rows that
+//                      advance as a wavefront, the Thomas recurrences, serial in
+//                      k, of a strip's columns on one wave (lane = row).  Very
+//                      tall columns take one launch per anti-diagonal instead,
+//                      one wave per column (lanes over k for the coefficients,
+//                      one lane for the recurrences).
 // This replays the reference's deterministic (single-thread) order exactly.
 #include <cmath>
 #include <mutex>
@@ -1355,12 +1357,11 @@ __global__ __launch_bounds__(WAVE) void k_tke(const Dom *__restrict__ ds, int t,
 // A workgroup owns consecutive sweep rows (b) with one wave per row, a chain
 // wave and a control wave.  Row wave r owns row b0 + r and at local step s handles column
 // a = oa + s - r, so every local step is one anti-diagonal of the strip.  Each
-// step is three phases separated by workgroup barriers: (1) every active row
-// wave assembles its column's source terms (lanes over k) into LDS, (2) the
-// chain wave runs the serial Thomas recurrences of all the strip's columns
-// (lane = row) while the row waves prefetch their next columns, (3) the row
-// waves write their columns back.  Neighbours updated in the previous step are
-// exchanged through LDS column buffers.
+// step is two phases separated by workgroup barriers: (1) every active row wave
+// finishes its column's source terms (lanes over k) with the two neighbours the
+// step before updated, read from LDS, (2) the chain wave runs the serial Thomas
+// recurrences of all the strip's columns (lane = row) while the row waves store
+// the column before, work up the next one and load the one after.
 #define STRIP_WAVES 16            // waves of a strip at most: 14 rows, the chain and the control wave
 
 // coefficient records written by k_ml_coef and read by the strip sweeps; per
