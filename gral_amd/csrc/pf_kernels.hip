@@ -19,6 +19,7 @@
 #include <mutex>
 #include <type_traits>
 #include "pf_device.h"
+#include "pf_strip.h"
 
 #define WAVE 64
 
@@ -1677,7 +1678,10 @@ __device__ __forceinline__ void strip_back(const float *P, const float *Q, float
 // counts the situation's iterations (sync[1], advanced by k_zero_rows) and
 // names the sweep, so no word of an earlier sweep matches.  Against a progress
 // counter the writer need not wait for its stores and the reader not for a poll
-// before its loads.
+// before its loads.  The words also keep the next strip from overwriting old
+// values this one still reads: a momentum sweep hands on every level the last row's
+// column reads, updated or not (hand_sent(), hand_needed()); the pressure and TKE
+// sweeps and the line strips update all the levels they read.
 typedef unsigned long long __attribute__((address_space(1))) gu64;
 __device__ __forceinline__ unsigned hand_tag(const DomG &d, int kind) { return 8u * (unsigned)d.sync[1] + (unsigned)kind; }
 __device__ __forceinline__ void hand_put(gu64 *p, float v, unsigned tag) {
@@ -1715,21 +1719,8 @@ __device__ __forceinline__ const gf32 *lane_at(const gf32 *base, unsigned byte_o
     return (const gf32 *)((gc8 *)base + byte_off);
 }
 
-// Metadata of a sweep position as the strips' rows keep it (uniform); a column
-// outside the sub-domains or the sweep has VI = -1.
-struct StripCol { int KK, VI, ks, kend, veg; };   // ks: KSTART, kend: first level the sweep updates
 template <int COMP>
-__device__ __forceinline__ StripCol strip_col(int4 m) {
-    StripCol c;
-    c.KK = m.x;
-    c.VI = (m.z & 0x10000) ? m.y : -1;
-    c.ks = m.z & 0xffff;
-    // U and V skip the levels inside the building or its upstream neighbour; W
-    // updates every level from KSTART
-    c.kend = (COMP == 2) ? c.ks : (COMP == 0) ? (m.w & 0xffff) + 1 : ((m.w >> 16) & 0xffff) + 1;
-    c.veg = m.z & 0x20000;
-    return c;
-}
+__device__ __forceinline__ StripCol strip_col(int4 m) { return strip_col<COMP>(m.x, m.y, m.z, m.w); }
 
 // Raw operands of one column, as loaded one step before they are worked up:
 // records, own and old neighbour values, the -IS / -JS neighbours' values as
@@ -1859,13 +1850,15 @@ __global__ __launch_bounds__(STRIP_WAVES * WAVE) void k_ml_strip(const Dom *__re
             lds_barrier();
             const StripCol cn = info(s + 1);
             lds_barrier();                                    // the recurrences are done
-            const int vil = __builtin_amdgcn_readlane(c.VI, R - 1);
-            if (send && vil >= 0) {
+            const StripLevels hl = hand_sent<COMP>(c);
+            const int hi = __builtin_amdgcn_readlane(hl.hi, R - 1);
+            if (send && hi >= 0) {
                 // the last row's results, the only column another strip reads, go
-                // out while the rows assemble the next step
-                const int kel = __builtin_amdgcn_readlane(c.kend, R - 1), kkl = __builtin_amdgcn_readlane(c.KK, R - 1);
+                // out while the rows assemble the next step; below the first updated
+                // level only the tag counts
+                const int lo = __builtin_amdgcn_readlane(hl.lo, R - 1), kkl = __builtin_amdgcn_readlane(c.KK, R - 1);
                 const float *xn = sm + (size_t)(R - 1) * rs + (4 + 4 * (s & 1)) * len + low - (kkl + 1);
-                for (int k = kel + lane; k <= vil; k += WAVE) hand_put(h + (size_t)s * nkp + k, xn[k], tag);
+                for (int k = lo + lane; k <= hi; k += WAVE) hand_put(h + (size_t)s * nkp + k, xn[k], tag);
             }
             c = cn;
         }
@@ -1998,12 +1991,13 @@ __global__ __launch_bounds__(STRIP_WAVES * WAVE) void k_ml_strip(const Dom *__re
         }
         if (from_prev) {
             const gu64 *h = hand + ((size_t)(B - 1) * hcols + (s - r)) * nkp;
+            const StripLevels hl = hand_needed<COMP>(c, c1j);
 #pragma unroll
             for (int m = 0; m < M; ++m) {
                 const int k = kb + lane + WAVE * m;
-                const bool need = k <= c.VI && k >= c1j.kend && k <= c1j.VI;
+                const bool need = k >= hl.lo && k <= hl.hi;
                 hwait.wait(h + k, need, tag, raw[m].hw);
-                if (need) in[m].nj = __uint_as_float((unsigned)raw[m].hw);
+                if (need && k >= c1j.kend) in[m].nj = __uint_as_float((unsigned)raw[m].hw);
                 in[m].sj = false;                             // the value is in nj
                 in[m].lj = 0;
             }
