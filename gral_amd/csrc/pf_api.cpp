@@ -179,6 +179,7 @@ struct gral_pf_handle {
     // grid
     int device = -1;                // the HIP device current at create
     int nii = 0, njj = 0, nkk = 0, kadvmax = 0, vcf = 0, nkp = 0, nkh = 0;
+    bool diag = false;              // prepared with GRAL_PF_SWEEP=diag
     float dxk = 0, dyk = 0;
     std::vector<float> dzk, hok;
     // host state (full depth nkh = nkk+2)
@@ -750,9 +751,15 @@ static int put_vec(gral_pf_handle *h, T *dptr, const std::vector<T> &v) {
     return move_all(h, true, {move_bytes(dptr, v.data(), v.size() * sizeof(T))});
 }
 
-// columns of more than 126 levels: a batch holds situations of one kind (see
-// gral_pf_batch_create), since such a situation may run per-diagonal
+// columns of more than 126 levels: such a situation runs per-diagonal where the
+// strips cannot hold it or find no memory
 static bool tall(const gral_pf_handle *h) { return h->kadvmax + 2 > 128; }
+// A batch takes situations of one kind, those that always run on strips or those
+// that may run per-diagonal (whichever sweeps each of them has: run_lockstep
+// launches the two apart)
+static bool same_kind(const gral_pf_handle *a, const gral_pf_handle *b) {
+    return a->d.model == b->d.model && (tall(a) || a->diag) == (tall(b) || b->diag);
+}
 
 // the fields the device holds, with their host copies
 static std::vector<Move> solver_fields(const gral_pf_handle *h) {
@@ -846,8 +853,8 @@ extern "C" int gral_pf_prepare(gral_pf_handle *h, const gral_pf_params *p) {
     // sweep kernels: strip-pipelined (default) or one launch per anti-diagonal
     // (GRAL_PF_SWEEP = strip | diag)
     const char *sw = std::getenv("GRAL_PF_SWEEP");
-    d.tiled = 2;
-    if (sw && std::strcmp(sw, "diag") == 0) d.tiled = 0;
+    h->diag = sw && std::strcmp(sw, "diag") == 0;
+    d.tiled = h->diag ? 0 : 2;
     {
         // strip synchronisation: header + one block per sweep kind (pressure, U, V, W, TKE)
         d.sync_stride = 64;
@@ -1242,18 +1249,21 @@ static void run_lockstep(const std::vector<gral_pf_handle *> &hs, Dom *dd, hipSt
         // own iteration - 1; with graphs the slot counts from the chunk's start
         if (upload || gc) {
             // group g takes situations g, g+G, g+2G, ... of act (act is ordered
-            // largest first by the callers that care), stored contiguously
+            // largest first by the callers that care), stored contiguously, those
+            // with strips first
             ng = want;
             if (ng > 1 && !sg->ensure(ng - 1)) return bad(GRAL_PF_EDEVICE, "stream creation failed");
             hd.resize(act.size());
             size_t pos = 0;
             for (int g = 0; g < ng; ++g) {
                 goff[g] = (int)pos;
-                for (size_t q = (size_t)g; q < act.size(); q += (size_t)ng) {
-                    hd[pos] = act[q]->d;
-                    hd[pos].iter_off = gc ? 1 - act[q]->iter_loops : it0 - act[q]->iter_loops;
-                    ++pos;
-                }
+                for (const bool tiled : {true, false})
+                    for (size_t q = (size_t)g; q < act.size(); q += (size_t)ng) {
+                        if ((act[q]->d.tiled != 0) != tiled) continue;
+                        hd[pos] = act[q]->d;
+                        hd[pos].iter_off = gc ? 1 - act[q]->iter_loops : it0 - act[q]->iter_loops;
+                        ++pos;
+                    }
                 gcnt[g] = (int)pos - goff[g];
             }
             if (hipMemcpyAsync(dd, hd.data(), sizeof(Dom) * hd.size(), hipMemcpyHostToDevice, s) != hipSuccess)
@@ -1271,12 +1281,15 @@ static void run_lockstep(const std::vector<gral_pf_handle *> &hs, Dom *dd, hipSt
                 const int it = it0 + c;
                 for (int g = 0; g < ng; ++g) {
                     hipStream_t sgs = g == 0 ? s : sg->s[g - 1];
-                    int e = pf_launch_iteration(hd.data() + goff[g], gcnt[g], dd + goff[g], it, gc ? c : it - 1, sgs,
-                                                launches, probe);
-                    if (e) {
-                        bad(GRAL_PF_EDEVICE, std::string("kernel launch failed at iteration ") + std::to_string(it) + ": " +
-                                                 hipGetErrorString((hipError_t)e));
-                        return e;
+                    // one launch set for those with strips, one for the others
+                    for (int a = goff[g], b; a < goff[g] + gcnt[g]; a = b) {
+                        for (b = a + 1; b < goff[g] + gcnt[g] && hd[b].tiled == hd[a].tiled; ++b) {}
+                        int e = pf_launch_iteration(hd.data() + a, b - a, dd + a, it, gc ? c : it - 1, sgs, launches, probe);
+                        if (e) {
+                            bad(GRAL_PF_EDEVICE, std::string("kernel launch failed at iteration ") + std::to_string(it) + ": " +
+                                                     hipGetErrorString((hipError_t)e));
+                            return e;
+                        }
                     }
                 }
             }
@@ -1876,8 +1889,7 @@ extern "C" int gral_pf_batch_create(gral_pf_handle *const *handles, int32_t n, g
         if (!handles[q] || !handles[q]->prepared) return GRAL_PF_ESTATE;
         for (int r = 0; r < q; ++r)
             if (handles[r] == handles[q]) return GRAL_PF_EINVAL;
-        const Dom &a = handles[0]->d, &c = handles[q]->d;
-        if (a.model != c.model || a.tiled != c.tiled || tall(handles[0]) != tall(handles[q])) return GRAL_PF_EINVAL;
+        if (!same_kind(handles[0], handles[q])) return GRAL_PF_EINVAL;
     }
     gral_pf_batch *b = new (std::nothrow) gral_pf_batch();
     if (!b) return GRAL_PF_ENOMEM;
@@ -1909,7 +1921,7 @@ extern "C" int gral_pf_batch_add(gral_pf_batch *b, gral_pf_handle *h) {
     for (auto *x : b->pending)
         if (x == h) return bfail(b, GRAL_PF_EINVAL, "batch add: the situation is already queued");
     const gral_pf_handle *ref = !b->hs.empty() ? b->hs[0] : (!b->pending.empty() ? b->pending[0] : nullptr);
-    if (ref && (ref->d.model != h->d.model || ref->d.tiled != h->d.tiled || tall(ref) != tall(h)))
+    if (ref && !same_kind(ref, h))
         return bfail(b, GRAL_PF_EINVAL, "batch add: situations of a batch must share the turbulence model and sweep kind");
     const size_t need = b->hs.size() + b->pending.size() + 1;
     if (need > b->dd_cap) {
