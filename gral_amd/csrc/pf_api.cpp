@@ -22,6 +22,7 @@
 
 #include "../../include/gral_pf.h"
 #include "pf_device.h"
+#include "pf_spare.h"
 
 // Levels per device column: KADVMAX + 2 rounded up to a multiple of NKP_ALIGN
 // (a power of two >= 4: the cell kernels move 16-byte quads of levels).  With
@@ -193,6 +194,9 @@ struct gral_pf_handle {
     int istat = 4, nprof = 0;
     std::vector<float> mh, u0, v0;
     size_t dev_bytes = 0;           // device bytes allocated by prepare
+    std::shared_ptr<Spare> spare;   // a tall situation's strip buffers, which it can give back
+    size_t spare_bytes = 0;         // their share of dev_bytes
+    bool preparing = false;         // in gral_pf_prepare: no spare, no lock held
     double *mass_buf = nullptr;     // FP64 mass imbalance: [mass_nblk][2] block partials, then the [2] result
     int mass_nblk = 0;
     double mass[2] = {0, 0};        // sum |DIV|, sum |face flux| at the last finish / mass_imbalance call
@@ -259,13 +263,92 @@ static int fail(gral_pf_handle *h, int code, const std::string &msg) {
             return fail((h), GRAL_PF_EDEVICE, std::string(#call) + ": " + hipGetErrorString(e_)); \
     } while (0)
 
+// the strip buffers that tall situations of this process hold
+static SparePool g_spares;
+static void spare_release(void *p) { (void)hipFree(p); }
+static unsigned long long next_gen() {
+    static std::atomic<unsigned long long> n{1};
+    return n++;
+}
+
+// the situation without its strips: per-diagonal from here on
+static int strips_gone(gral_pf_handle *h) {
+    Dom &d = h->d;
+    d.hand = nullptr;
+    d.planes = d.rec3 = d.wcol = nullptr;
+    d.ptab[0] = d.ptab[1] = d.ttab[0] = d.ttab[1] = nullptr;
+    d.tiled = 0;
+    h->spare.reset();
+    h->dev_bytes -= h->spare_bytes;
+    h->spare_bytes = 0;
+    h->gen = next_gen();                                  // no captured chunk of it is replayed
+    if (h->graphs) h->graphs->clear();
+    return h->dd && hipMemcpy(h->dd, &d, sizeof(Dom), hipMemcpyHostToDevice) != hipSuccess ? 1 : 0;
+}
+
+// Held by every call that may use the strips' buffers or allocate device memory for
+// prepared situations; not recursive.
+struct StripUse {
+    std::vector<std::unique_lock<std::mutex>> held;
+    int rc = 0;
+    explicit StripUse(std::vector<gral_pf_handle *> hs) {
+        std::sort(hs.begin(), hs.end());
+        for (auto *h : hs) {
+            if (!h->spare) continue;
+            const std::shared_ptr<Spare> s = h->spare;
+            std::unique_lock<std::mutex> l(s->use);
+            if (g_spares.keep(s)) held.push_back(std::move(l));
+            else {
+                l.unlock();
+                rc |= strips_gone(h);
+            }
+        }
+    }
+};
+
+// h's own strips make room (StripUse held, or h in prepare); 1 on failure
+static int strips_drop(gral_pf_handle *h) {
+    h->spare->free_all();
+    g_spares.remove(h->spare);
+    return strips_gone(h);
+}
+
+// hipMalloc for h.  What does not fit takes the memory of other tall situations'
+// strips, then of h's own (StripUse held).  Prepare, which holds no lock, gives its
+// own first and waits for calls that use such memory to end.
+static hipError_t dev_malloc(gral_pf_handle *h, void **p, size_t bytes) {
+    for (;;) {
+        const hipError_t e = hipMalloc(p, bytes);
+        if (e == hipSuccess) return e;
+        (void)hipGetLastError();
+        if (h->preparing && h->spare) {
+            if (strips_drop(h)) return e;
+        } else if (!g_spares.give_back(h->device, h->spare.get(), h->preparing)) {
+            if (!h->spare || strips_drop(h)) return e;
+        }
+    }
+}
+// ... for calls without a situation (on the current device; no lock held)
+extern "C" int pf_malloc(void **p, size_t bytes) {
+    for (;;) {
+        const hipError_t e = hipMalloc(p, bytes);
+        if (e == hipSuccess) return 0;
+        (void)hipGetLastError();
+        int dev = -1;
+        if (hipGetDevice(&dev) != hipSuccess || !g_spares.give_back(dev, nullptr, true)) return 1;
+    }
+}
+
+// must: an allocation the caller has no way round
 template <class T>
-static int dalloc(gral_pf_handle *h, T **p, size_t n) {
+static int dalloc(gral_pf_handle *h, T **p, size_t n, bool must = true) {
     void *q = nullptr;
     const size_t bytes = n * sizeof(T) + 256;
+    if (must && h->spare && h->dev_cap && h->dev_bytes + bytes > h->dev_cap && strips_drop(h))
+        return fail(h, GRAL_PF_EDEVICE, "upload of the situation failed");
     if (h->dev_cap && h->dev_bytes + bytes > h->dev_cap)
         return fail(h, GRAL_PF_ENOMEM, "device memory budget (GRAL_PF_DEVICE_MB) exceeded");
-    hipError_t e = hipMalloc(&q, bytes);
+    hipError_t e = must ? dev_malloc(h, &q, bytes) : hipMalloc(&q, bytes);
     if (e != hipSuccess) return fail(h, GRAL_PF_ENOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
     h->dev.push_back(q);
     h->dev_bytes += bytes;
@@ -393,6 +476,13 @@ extern "C" int gral_pf_upload_fields(gral_pf_handle *h, const float *uk, const f
 }
 
 static void free_device(gral_pf_handle *h) {
+    if (h->spare) {
+        std::lock_guard<std::mutex> l(h->spare->use);
+        h->spare->free_all();
+        g_spares.remove(h->spare);
+    }
+    h->spare.reset();
+    h->spare_bytes = 0;
     for (void *p : h->dev) (void)hipFree(p);
     h->dev.clear();
     h->dev_bytes = 0;
@@ -805,6 +895,16 @@ extern "C" int gral_pf_prepare(gral_pf_handle *h, const gral_pf_params *p) {
     prologue(h, p, ap0, ht, ho, ta, tden, tbr, dtime, frund, ug, vg, ufx);
 
     free_device(h);
+    struct Preparing {
+        gral_pf_handle *h;
+        ~Preparing() {
+            h->preparing = false;
+            if (h->prepared || !h->spare) return;
+            h->spare->free_all();                         // a failed prepare keeps no strips
+            h->spare.reset();
+        }
+    } preparing{h};
+    h->preparing = true;
     Dom &d = h->d;
     d = Dom{};
     d.nii = h->nii; d.njj = h->njj; d.nkk = h->nkk; d.nkp = h->nkp; d.nj2 = h->njj + 2; d.kadvmax = h->kadvmax;
@@ -890,9 +990,11 @@ extern "C" int gral_pf_prepare(gral_pf_handle *h, const gral_pf_params *p) {
         // (W) floats per cell, then 3.  The U/V wall terms follow.
         const size_t rec = (p->turbulence_model == 2) ? 20 : 15;
         float *pl, *tab[4];
-        if ((e = dalloc(h, &d.hand, 2 * d.hand_words)) || (e = dalloc(h, &pl, rec * n3 + n2))) return e;
+        const bool must = !tall(h);
+        if ((e = dalloc(h, &pl, rec * n3 + n2, must))) return e;
         for (auto &q : tab)
-            if ((e = dalloc(h, &q, n3))) return e;
+            if ((e = dalloc(h, &q, n3, must))) return e;
+        if ((e = dalloc(h, &d.hand, 2 * d.hand_words, must))) return e;
         d.planes = pl;
         d.rec3 = pl + 12 * n3;
         d.wcol = pl + rec * n3;
@@ -911,9 +1013,14 @@ extern "C" int gral_pf_prepare(gral_pf_handle *h, const gral_pf_params *p) {
             h->dev_bytes = bytes;
             h->err.clear();
             d.hand = nullptr;
-            d.planes = d.rec3 = d.wcol = nullptr;
-            d.ptab[0] = d.ptab[1] = d.ttab[0] = d.ttab[1] = nullptr;
             d.tiled = 0;
+        } else if (tall(h)) {                             // and gives them back where others find none
+            h->spare = std::make_shared<Spare>();
+            h->spare->device = h->device;
+            h->spare->release = spare_release;
+            h->spare->mem.assign(h->dev.begin() + (ptrdiff_t)mark, h->dev.end());
+            h->dev.resize(mark);
+            h->spare_bytes = h->dev_bytes - bytes;
         }
     }
     if (d.tiled) {
@@ -999,9 +1106,9 @@ extern "C" int gral_pf_prepare(gral_pf_handle *h, const gral_pf_params *p) {
             size_t c = h->i2(i, j);
             if (h->adv[c] == 1) h->active += h->vi[c] - h->kk[c];
         }
-    static std::atomic<unsigned long long> next_gen{1};
-    h->gen = next_gen++;
+    h->gen = next_gen();
     h->prepared = true;
+    if (h->spare) g_spares.add(h->spare);
     h->gff_ok = false;
     h->done = false;
     h->host_stale = false;
@@ -1073,6 +1180,8 @@ extern "C" int gral_pf_mass_imbalance_noalloc(gral_pf_handle *h, double *sum_abs
 extern "C" int gral_pf_mass_imbalance(gral_pf_handle *h, double *sum_abs_div, double *sum_abs_flux) {
     if (!h) return GRAL_PF_EINVAL;
     if (!h->prepared) return fail(h, GRAL_PF_ESTATE, "mass_imbalance: call prepare first");
+    StripUse use({h});
+    if (use.rc) return fail(h, GRAL_PF_EDEVICE, "mass_imbalance: upload of the situation failed");
     int rc = mass_handle_run(h);
     if (rc) return rc;
     if (sum_abs_div) *sum_abs_div = h->mass[0];
@@ -1192,6 +1301,8 @@ static void run_lockstep(const std::vector<gral_pf_handle *> &hs, Dom *dd, hipSt
                          int n, bool check, Probe *probe, RunResult &R, GraphCache *gc = nullptr,
                          StreamGroup *sg = nullptr) {
     auto bad = [&](int code, const std::string &m) { R.code = code; R.err = m; };
+    StripUse use(hs);
+    if (use.rc) return bad(GRAL_PF_EDEVICE, "upload of a situation failed");
     if (probe || !graphs_enabled()) gc = nullptr;
     if (probe || gc) sg = nullptr;                  // profiling and graph capture run on the one stream
     std::vector<gral_pf_handle *> act;
@@ -1440,6 +1551,8 @@ static int sync_host(gral_pf_handle *h) {
 extern "C" int gral_pf_finish(gral_pf_handle *h, gral_pf_stats *st) {
     if (!h) return GRAL_PF_EINVAL;
     if (!h->prepared) return fail(h, GRAL_PF_ESTATE, "finish: call prepare first");
+    StripUse use({h});
+    if (use.rc) return fail(h, GRAL_PF_EDEVICE, "finish: upload of the situation failed");
     int rc = mass_handle_run(h);
     if (rc) return rc;
     rc = sync_host(h);
@@ -1552,7 +1665,7 @@ static int adj_hand(gral_pf_handle *h, unsigned long long *&p) {
     if (p) return 0;
     if (!h->adj_hand) {
         unsigned long long *q;
-        int rc = dalloc(h, &q, 2 * h->d.hand_words);
+        int rc = dalloc(h, &q, 2 * h->d.hand_words, false);
         if (rc) return rc;
         HIPCHK(h, hipMemsetAsync(q, 0, 2 * h->d.hand_words * sizeof(unsigned long long), h->stream));
         h->adj_hand = q;
@@ -1566,6 +1679,8 @@ extern "C" int gral_pf_forward_ckpt(gral_pf_handle *h, int32_t n, int32_t quanti
     if (!h->prepared) return fail(h, GRAL_PF_ESTATE, "forward_ckpt: call prepare first");
     if (n < 1 || n > 100000) return fail(h, GRAL_PF_EINVAL, "forward_ckpt: n must be 1..100000");
     if (quantise != 0 && quantise != 1) return fail(h, GRAL_PF_EINVAL, "forward_ckpt: quantise must be 0 or 1");
+    StripUse use({h});
+    if (use.rc) return fail(h, GRAL_PF_EDEVICE, "forward_ckpt: upload of the situation failed");
     int rc = adj_alloc(h);
     if (rc) return rc;
     const size_t n3 = h->n2() * (size_t)h->nkp;
@@ -1626,6 +1741,8 @@ extern "C" int gral_pf_vjp(gral_pf_handle *h, const float *du, const float *dv, 
     if (!h) return GRAL_PF_EINVAL;
     if (!h->prepared || h->adj_n < 1) return fail(h, GRAL_PF_ESTATE, "vjp: call forward_ckpt first");
     if (!du || !dv || !dw || !gu || !gv || !gw) return fail(h, GRAL_PF_EINVAL, "vjp: null argument");
+    StripUse use({h});
+    if (use.rc) return fail(h, GRAL_PF_EDEVICE, "vjp: upload of the situation failed");
     const size_t n2 = h->n2(), n3 = n2 * (size_t)h->nkp;
     float *a = h->adj;
     AdjArgs g{};
@@ -1896,7 +2013,7 @@ extern "C" int gral_pf_batch_create(gral_pf_handle *const *handles, int32_t n, g
     if (n > 0) b->hs.assign(handles, handles + n);
     const size_t cap = std::max<size_t>(1, (size_t)n);
     if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess || hipEventCreate(&b->ev0) != hipSuccess ||
-        hipEventCreate(&b->ev1) != hipSuccess || hipMalloc((void **)&b->dd, sizeof(Dom) * cap) != hipSuccess) {
+        hipEventCreate(&b->ev1) != hipSuccess || pf_malloc((void **)&b->dd, sizeof(Dom) * cap)) {
         gral_pf_batch_destroy(b);
         return GRAL_PF_EDEVICE;
     }
@@ -1927,7 +2044,7 @@ extern "C" int gral_pf_batch_add(gral_pf_batch *b, gral_pf_handle *h) {
     if (need > b->dd_cap) {
         const size_t cap = std::max(need, 2 * b->dd_cap);
         Dom *nd = nullptr;
-        if (hipMalloc((void **)&nd, sizeof(Dom) * cap) != hipSuccess) return bfail(b, GRAL_PF_ENOMEM, "batch add: hipMalloc failed");
+        if (pf_malloc((void **)&nd, sizeof(Dom) * cap)) return bfail(b, GRAL_PF_ENOMEM, "batch add: hipMalloc failed");
         if (hipStreamSynchronize(b->stream) != hipSuccess) return bfail(b, GRAL_PF_EDEVICE, "batch add: stream failed");
         b->graphs.clear();
         (void)hipFree(b->dd);
@@ -2084,6 +2201,8 @@ extern "C" int gral_pf_diagnostic(gral_pf_handle *h, int32_t flow_field_level, i
     if (!h) return GRAL_PF_EINVAL;
     if (flow_field_level != 1 && flow_field_level != 2) return fail(h, GRAL_PF_EINVAL, "diagnostic: flow_field_level must be 1 or 2");
     if (!h->masks || !h->fields) return fail(h, GRAL_PF_ESTATE, "diagnostic: masks and fields must be set first");
+    StripUse use({h});
+    if (use.rc) return fail(h, GRAL_PF_EDEVICE, "diagnostic: upload of the situation failed");
     h->mom_vjp_ok = false;
     int rc = 0;
     if (h->prepared && (rc = sync_host(h))) return rc;
@@ -2121,7 +2240,7 @@ extern "C" int gral_pf_diagnostic(gral_pf_handle *h, int32_t flow_field_level, i
     for (size_t c = 0; c < n2; ++c) kk32[c] = h->kk[c];
     std::vector<void *> tmp;
     auto talloc = [&](void **p, size_t bytes) -> int {
-        if (hipMalloc(p, bytes + 256) != hipSuccess) return fail(h, GRAL_PF_ENOMEM, "diagnostic: hipMalloc failed");
+        if (dev_malloc(h, p, bytes + 256) != hipSuccess) return fail(h, GRAL_PF_ENOMEM, "diagnostic: hipMalloc failed");
         tmp.push_back(*p);
         return 0;
     };
@@ -2217,7 +2336,7 @@ static int gff_upper(gral_pf_handle *h, int nlo) {
         if (h->gff_up) (void)hipFree(h->gff_up);
         h->gff_up = nullptr;
         h->gff_bytes = 0;
-        if (hipMalloc(&h->gff_up, bytes) != hipSuccess) { h->gff_up = nullptr; return fail(h, GRAL_PF_ENOMEM, "gff: hipMalloc failed"); }
+        if (dev_malloc(h, &h->gff_up, bytes) != hipSuccess) { h->gff_up = nullptr; return fail(h, GRAL_PF_ENOMEM, "gff: hipMalloc failed"); }
         h->gff_bytes = bytes;
     }
     const std::vector<float> *src[4] = {&h->uk, &h->vk, &h->wk, &h->turb};
@@ -2263,7 +2382,7 @@ static int gff_pack(gral_pf_handle *h, int kind, const gral_pf_gff_meta *meta, u
         if (h->gff_dbuf) (void)hipFree(h->gff_dbuf);
         h->gff_dbuf = nullptr;
         h->gff_dbuf_bytes = 0;
-        if (hipMalloc(&h->gff_dbuf, bytes) != hipSuccess) { h->gff_dbuf = nullptr; return fail(h, GRAL_PF_ENOMEM, "gff: hipMalloc failed"); }
+        if (dev_malloc(h, &h->gff_dbuf, bytes) != hipSuccess) { h->gff_dbuf = nullptr; return fail(h, GRAL_PF_ENOMEM, "gff: hipMalloc failed"); }
         h->gff_dbuf_bytes = bytes;
     }
     char *db = static_cast<char *>(h->gff_dbuf);
@@ -2337,6 +2456,8 @@ extern "C" int gral_pf_wind_at_particles(gral_pf_handle *h, int32_t topo, int32_
     if (n == 0) return GRAL_PF_OK;
     if (!cell_i || !cell_j || !ahint || !x || !y || !z || !ux || !uy || !uz || !cell_k)
         return fail(h, GRAL_PF_EINVAL, "wind_at_particles: null argument");
+    StripUse use({h});
+    if (use.rc) return fail(h, GRAL_PF_EDEVICE, "wind_at_particles: upload of the situation failed");
     std::atomic<int32_t> bad{n};                          // the first particle outside the grid
     par_for(0, (n + 65535) / 65536, [&](int, long a, long b) {
         const int32_t e = (int32_t)std::min<long>(n, b * 65536);
@@ -2361,7 +2482,7 @@ extern "C" int gral_pf_wind_at_particles(gral_pf_handle *h, int32_t topo, int32_
         if (h->pw_buf) (void)hipFree(h->pw_buf);
         h->pw_buf = nullptr;
         h->pw_bytes = 0;
-        if (hipMalloc(&h->pw_buf, bytes) != hipSuccess) { h->pw_buf = nullptr; return fail(h, GRAL_PF_ENOMEM, "wind_at_particles: hipMalloc failed"); }
+        if (dev_malloc(h, &h->pw_buf, bytes) != hipSuccess) { h->pw_buf = nullptr; return fail(h, GRAL_PF_ENOMEM, "wind_at_particles: hipMalloc failed"); }
         h->pw_bytes = bytes;
     }
     char *db = static_cast<char *>(h->pw_buf);
@@ -2409,6 +2530,8 @@ extern "C" int gral_pf_gff_payload(gral_pf_handle *h, int32_t kind, const gral_p
     *len = gff_size(h, kind);
     if (!out) return GRAL_PF_OK;
     if (cap < *len) return fail(h, GRAL_PF_EINVAL, "gff: output buffer too small");
+    StripUse use({h});
+    if (use.rc) return fail(h, GRAL_PF_EDEVICE, "gff: upload of the situation failed");
     uint8_t *o8 = static_cast<uint8_t *>(out);
     size_t body = 0;
     int rc = gff_pack(h, kind, meta, o8, body);
@@ -2423,6 +2546,8 @@ extern "C" int gral_pf_gff_write(gral_pf_handle *h, int32_t kind, const gral_pf_
     int rc = gral_pf_gff_payload(h, kind, meta, nullptr, 0, &len);
     if (rc) return rc;
     if (len >= 0xffffffffull) return fail(h, GRAL_PF_EINVAL, "gff: payload of 4 GiB or more (zip without ZIP64)");
+    StripUse use({h});
+    if (use.rc) return fail(h, GRAL_PF_EDEVICE, "gff: upload of the situation failed");
     // whole payload into the pinned buffer, deflated from there
     if ((rc = gff_host(h, len))) return rc;
     uint8_t *hb = static_cast<uint8_t *>(h->gff_hbuf);

@@ -21,6 +21,8 @@
 
 #include "../../include/gral_pf.h"
 
+extern "C" int pf_malloc(void **p, size_t bytes);
+
 namespace {
 
 thread_local std::string g_err;
@@ -47,7 +49,7 @@ struct Scratch {
     template <class T>
     T *alloc(size_t n) {
         void *q = nullptr;
-        if (hipMalloc(&q, std::max<size_t>(n, 1) * sizeof(T)) != hipSuccess) return nullptr;
+        if (pf_malloc(&q, std::max<size_t>(n, 1) * sizeof(T))) return nullptr;
         p.push_back(q);
         return static_cast<T *>(q);
     }
