@@ -971,8 +971,9 @@ extern "C" int gral_pf_prepare(gral_pf_handle *h, const gral_pf_params *p) {
                 d.nact = std::max(d.nact, h->vi[c] - h->kk[c]);
                 if (h->cutk[c] != 0) d.nlow = std::max(d.nlow, (int)h->kk[c]);
             }
-        d.hand_cols = std::max(h->nii, h->njj);
-        d.hand_words = (size_t)(d.hand_cols / STRIP_ROWS_MIN + 1) * d.hand_cols * d.nkp;
+        // strips of rows along j hand on columns along i, and the other way round
+        const size_t si = h->nii / STRIP_ROWS_MIN + 1, sj = h->njj / STRIP_ROWS_MIN + 1;
+        d.hand_words = std::max(sj * h->nii, si * h->njj) * d.nkp;
     }
     // The strips hold 256 levels a column, 127 of them above the ground: the W
     // sweep deals a column to at most 4 groups of 64 lanes, the others to 2

@@ -45,9 +45,8 @@ struct DomT {
     int tiled;                       // 2: strip-pipelined sweeps, 0: one launch per anti-diagonal
     P<int> sync;                     // strip sweeps: [64] header (sticky error flag, iteration count), then per
     int sync_stride;                 //   sweep kind sync_stride ints (the ticket, alone in its cache lines)
-    P<unsigned long long> hand;      // values handed from strip to strip: {value, tag} words [2][strip][hand_cols][nkp]
+    P<unsigned long long> hand;      // values handed from strip to strip: {value, tag} words [2][strip][step][nkp]
     size_t hand_words;               // words of one of the two
-    int hand_cols;
     int nact, nlow;                  // largest VI - KKART, and KKART + 1 - KSTART, of the active columns
     P<float> planes;                 // [cells][12 (U, V) or 8 (W)] mixing-length coefficient records
     P<float> rec3;                   // [cells][3]  C, TERMP and P of the same cells

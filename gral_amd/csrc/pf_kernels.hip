@@ -1766,7 +1766,7 @@ __global__ __launch_bounds__(STRIP_WAVES * WAVE) void k_ml_strip(const Dom *__re
     extern __shared__ __align__(16) float sm[];
     // the fields the steps use, read once: a scalar load inside a step would
     // wait for its latency and, sharing its counter, for the LDS accesses
-    const int nkp = d.nkp, nii = d.nii, njj = d.njj, nj2 = d.nj2, hcols = d.hand_cols;
+    const int nkp = d.nkp, nii = d.nii, njj = d.njj, nj2 = d.nj2, hcols = nii;
     const int low = strip_low((COMP == 2) ? d.nlow : 0), len = strip_len((COMP == 2) ? d.nlow : 0, d.nact);
     const int rs = strip_stride(9, len);
     const int oa = (COMP == 0) ? 3 : 2, ia = (COMP == 1) ? 3 : 2, ob = nii - 1, ib = njj - 1, na = ob - oa + 1;
@@ -1785,7 +1785,7 @@ __global__ __launch_bounds__(STRIP_WAVES * WAVE) void k_ml_strip(const Dom *__re
     const int B = __builtin_amdgcn_readfirstlane(sctl[0]);
     if (B >= nstrip) return;                                  // uniform over the workgroup
     const unsigned tag = hand_tag(d, 1 + COMP);
-    gu64 *hand = (gu64 *)d.hand;                              // [strip][hand_cols][nkp] words
+    gu64 *hand = (gu64 *)d.hand;                              // [strip][nii][nkp] words
     const int4 *meta = (const int4 *)d.meta;
     // The chain and the control wave run loops of their own with the same
     // barriers per step as the row waves (s_barrier counts waves, wherever they
@@ -2183,7 +2183,7 @@ template <int M>
 __global__ __launch_bounds__(STRIP_WAVES * WAVE) void k_pressure_strip(const Dom *__restrict__ ds, int IS, int JS, int slot) {
     const DomG &d = reinterpret_cast<const DomG *>(ds)[blockIdx.z];
     extern __shared__ __align__(16) float sm[];
-    const int nkp = d.nkp, nii = d.nii, njj = d.njj, nj2 = d.nj2, hcols = d.hand_cols;
+    const int nkp = d.nkp, nii = d.nii, njj = d.njj, nj2 = d.nj2, hcols = njj;
     const int low = strip_low(0), len = strip_len(0, d.nact), rs = strip_stride(9, len);
     const int oa = 2, ia = 2, ob = njj - 1, ib = nii - 1, na = ob - oa + 1;
     const int R = blockDim.x / WAVE - 2;                      // rows of a strip (strip_rows())
@@ -2201,7 +2201,7 @@ __global__ __launch_bounds__(STRIP_WAVES * WAVE) void k_pressure_strip(const Dom
     const int B = __builtin_amdgcn_readfirstlane(sctl[0]);
     if (B >= nstrip) return;                                  // uniform over the workgroup
     const unsigned tag = hand_tag(d, 0);
-    gu64 *hand = (gu64 *)d.hand, *handq = hand + d.hand_words;        // new DPM, row scratch: [strip][hand_cols][nkp]
+    gu64 *hand = (gu64 *)d.hand, *handq = hand + d.hand_words;        // new DPM, row scratch: [strip][njj][nkp]
     const int4 *meta = (const int4 *)d.meta;
     HandWait hwait{d.sync, wall_clock64() + STRIP_TIMEOUT_TICKS, false};
     const bool send = B + 1 < nstrip;
@@ -3237,7 +3237,7 @@ template <int M>
 __global__ __launch_bounds__(STRIP_WAVES * WAVE) void k_tke_strip(const Dom *__restrict__ ds, int IS, int JS) {
     const DomG &d = reinterpret_cast<const DomG *>(ds)[blockIdx.z];                   // situation of this launch slice
     extern __shared__ __align__(16) float sm[];
-    const int nkp = d.nkp, nii = d.nii, njj = d.njj, nj2 = d.nj2, hcols = d.hand_cols;
+    const int nkp = d.nkp, nii = d.nii, njj = d.njj, nj2 = d.nj2, hcols = nii;
     const int low = strip_low(0), len = strip_len(0, d.nact), rs = strip_stride(TKE_ARRAYS, len), fs = 9 * len;
     const int oa = 2, ia = 2, ob = nii - 1, ib = njj - 1, na = ob - oa + 1;
     const int R = blockDim.x / WAVE - 2;
@@ -3253,7 +3253,7 @@ __global__ __launch_bounds__(STRIP_WAVES * WAVE) void k_tke_strip(const Dom *__r
     const int B = __builtin_amdgcn_readfirstlane(sctl[0]);
     if (B >= nstrip) return;                                  // uniform over the workgroup
     const unsigned tag = hand_tag(d, 4);
-    gu64 *handt = (gu64 *)d.hand, *hande = handt + d.hand_words;      // TURB, TDISS: [strip][hand_cols][nkp]
+    gu64 *handt = (gu64 *)d.hand, *hande = handt + d.hand_words;      // TURB, TDISS: [strip][nii][nkp]
     const int4 *meta = (const int4 *)d.meta;
     const bool send = B + 1 < nstrip;
     if (r == R) {                                             // chain wave
