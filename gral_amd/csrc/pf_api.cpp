@@ -935,7 +935,9 @@ extern "C" int gral_pf_prepare(gral_pf_handle *h, const gral_pf_params *p) {
     float *fveg = F[11];
     if ((rc = dalloc(h, &d.prow_p, (size_t)d.nj2 * d.nkp)) || (rc = dalloc(h, &d.prow_q, (size_t)d.nj2 * d.nkp))) return rc;
     unsigned *fres;
-    if ((rc = dalloc(h, &fres, (size_t)p->iter_max + 1))) return rc;
+    int4 *fmeta;
+    if ((rc = dalloc(h, &fres, (size_t)p->iter_max + 1)) || (rc = dalloc(h, &fmeta, n2)) || (rc = dalloc(h, &h->dd, 1))) return rc;
+    if (h->has_veg && (rc = dalloc(h, &fvegp, n2))) return rc;
     d.resid = fres;
     d.resid_cap = p->iter_max + 1;
     h->mass_nblk = mass_blocks(h->nii, h->njj);
@@ -982,7 +984,10 @@ extern "C" int gral_pf_prepare(gral_pf_handle *h, const gral_pf_params *p) {
     d.rec3 = nullptr;
     d.wcol = nullptr;
     d.ptab[0] = d.ptab[1] = d.ttab[0] = d.ttab[1] = nullptr;
-    // the strips' buffers: hand-off words, coefficient records, pressure tables
+    // The strips' buffers: coefficient records, pressure tables, hand-off words.  A
+    // situation runs per-diagonal without them if it is tall (12 fields and no more
+    // are enough for it) or if only the words, 0.6 of a field, find no memory.
+    bool may_do_without = false;
     auto strip_alloc = [&]() -> int {
         int e;
         // k-eps: the momentum sweeps' records (12 or 8 floats per cell, then {C,
@@ -995,6 +1000,7 @@ extern "C" int gral_pf_prepare(gral_pf_handle *h, const gral_pf_params *p) {
         if ((e = dalloc(h, &pl, rec * n3 + n2, must))) return e;
         for (auto &q : tab)
             if ((e = dalloc(h, &q, n3, must))) return e;
+        may_do_without = true;                            // the hand-off words alone do not fit
         if ((e = dalloc(h, &d.hand, 2 * d.hand_words, must))) return e;
         d.planes = pl;
         d.rec3 = pl + 12 * n3;
@@ -1004,11 +1010,10 @@ extern "C" int gral_pf_prepare(gral_pf_handle *h, const gral_pf_params *p) {
     };
     if (d.tiled) {
         const size_t mark = h->dev.size(), bytes = h->dev_bytes;
+        may_do_without = tall(h);
         rc = strip_alloc();
-        if (rc && !tall(h)) return rc;
+        if (rc && !may_do_without) return rc;
         if (rc) {
-            // a tall column's situation whose strips find no memory still runs
-            // per-diagonal
             (void)hipGetLastError();
             for (; h->dev.size() > mark; h->dev.pop_back()) (void)hipFree(h->dev.back());
             h->dev_bytes = bytes;
@@ -1069,8 +1074,7 @@ extern "C" int gral_pf_prepare(gral_pf_handle *h, const gral_pf_params *p) {
             int kmi = std::max(KK, (int)h->kk[h->i2(i - 1, j)]), kmj = std::max(KK, (int)h->kk[h->i2(i, j - 1)]);
             meta[c] = make_int4(KK, h->vi[c], KSTART | ((int)h->adv[c] << 16) | (vegp << 17), kmi | (kmj << 16));
         }
-    int4 *fmeta;
-    if ((rc = dalloc(h, &fmeta, n2)) || (rc = put_vec(h, fmeta, meta))) return rc;
+    if ((rc = put_vec(h, fmeta, meta))) return rc;
     d.meta = fmeta;
     std::vector<int> kk32(n2);
     for (size_t c = 0; c < n2; ++c) kk32[c] = h->kk[c];
@@ -1085,7 +1089,7 @@ extern "C" int gral_pf_prepare(gral_pf_handle *h, const gral_pf_params *p) {
     d.adv = fadv; d.kk = fkk; d.vi = fvi; d.cutk = fcutk; d.cov = fcov; d.ht = fht; d.ho = fho; d.z0s = fz0s;
     d.tke_a = fta; d.tke_den = ftden; d.tke_br = ftbr;
     if (h->has_veg) {
-        if ((rc = dalloc(h, &fvegp, n2)) || (rc = put_vec(h, fvegp, h->vegp)) || (rc = put_field(h, fveg, h->veg))) return rc;
+        if ((rc = put_vec(h, fvegp, h->vegp)) || (rc = put_field(h, fveg, h->veg))) return rc;
         d.vegp = fvegp; d.veg = fveg;
     } else {
         d.vegp = nullptr; d.veg = nullptr;
@@ -1098,7 +1102,6 @@ extern "C" int gral_pf_prepare(gral_pf_handle *h, const gral_pf_params *p) {
         HIPCHK(h, hipMemsetAsync(d.tdiss, 0, n3 * sizeof(float), h->stream));
     }
     if (pf_fill_u32(d.resid, (size_t)p->iter_max + 1, 0u, h->stream)) return fail(h, GRAL_PF_EDEVICE, "fill resid");
-    if ((rc = dalloc(h, &h->dd, 1))) return rc;
     HIPCHK(h, hipMemcpyAsync(h->dd, &h->d, sizeof(Dom), hipMemcpyHostToDevice, h->stream));
     HIPCHK(h, hipStreamSynchronize(h->stream));
     h->active = 0;
