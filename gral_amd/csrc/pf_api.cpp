@@ -1880,19 +1880,23 @@ extern "C" int gral_pf_momentum_vjp(gral_pf_handle *h, const float *dx, float *g
     MomAdj m{};
     m.xa = xa;
     m.gin = a;
-    m.gout = a + n3; m.db = a + 2 * n3; m.gna = a + 4 * n3; m.gnb = a + 5 * n3; m.gres = a + 6 * n3;
+    m.gout = a + n3; m.db = m.gpa = a + 2 * n3; m.gpb = a + 3 * n3; m.gna = a + 4 * n3; m.gnb = a + 5 * n3; m.gres = a + 6 * n3;
     int rc;
     // the columns' data: in the sweeps' coefficient records, which hold nothing
-    // between two sweeps, or where the situation has none in a buffer of its own
+    // between two sweeps, or where the situation has none in a buffer of its own;
+    // without memory for that or the words (m.hand null) per anti-diagonal
     float *rec = h->d.planes;
-    if (!h->d.tiled) {
-        if (!h->mom_rec && (rc = dalloc(h, &h->mom_rec, 8 * n3 + 4))) return rc;
-        rec = h->mom_rec;
+    if (!h->d.tiled && (h->mom_rec || dalloc(h, &h->mom_rec, 8 * n3 + 4, false) == 0)) rec = h->mom_rec;
+    if (!rec || adj_hand(h, m.hand)) {
+        (void)hipGetLastError();
+        h->err.clear();
+        m.hand = nullptr;
     }
-    if ((rc = adj_hand(h, m.hand))) return rc;
-    m.T = rec; m.P = rec + n3; m.C = rec + 2 * n3; m.Q = rec + 3 * n3;
-    m.ca = rec + 4 * n3; m.cb = rec + 5 * n3; m.cc = rec + 6 * n3;
-    m.col = reinterpret_cast<int4 *>((reinterpret_cast<uintptr_t>(rec + 7 * n3) + 15) & ~(uintptr_t)15);
+    if (m.hand) {
+        m.T = rec; m.P = rec + n3; m.C = rec + 2 * n3; m.Q = rec + 3 * n3;
+        m.ca = rec + 4 * n3; m.cb = rec + 5 * n3; m.cc = rec + 6 * n3;
+        m.col = reinterpret_cast<int4 *>((reinterpret_cast<uintptr_t>(rec + 7 * n3) + 15) & ~(uintptr_t)15);
+    }
     if ((rc = move_all(h, true, {field_move(h, a, dx)}))) return rc;
     HIPCHK(h, hipEventRecord(h->ev0, h->stream));
     const int e = pf_launch_momentum_vjp(&hb, db, &m, comp, h->mom_is, h->mom_js, h->stream);

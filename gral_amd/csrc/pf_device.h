@@ -180,7 +180,8 @@ struct MomAdj {
     float *db;          // per column and level: adjoint of the source D
     float *T, *P, *C, *Q, *ca, *cb, *cc;   // what its columns need (k_adj_mom_pre)
     int4 *col;          // per column: levels of the sweep
-    unsigned long long *hand;   // hand-off words, laid out as Dom::hand
+    unsigned long long *hand;   // hand-off words, laid out as Dom::hand; null: per anti-diagonal, without db to col
+    float *gpa, *gpb;   // then, per column and level: adjoint for the new X of its a- / b-predecessor
     float *gna, *gnb;   // per column and level: adjoint for the old X of its a- / b-successor
     float *gres;        // dL/dX before, complete
 };

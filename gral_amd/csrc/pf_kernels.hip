@@ -4341,14 +4341,22 @@ struct MomOp {
 
 // The rest of a column's transpose, which no other column waits for: both
 // transposed recurrences with the handed adjoints known, and the assembly
-// transposed.  One wave per column.
+// transposed.  One wave per column.  DIAG: the whole of it, for the columns of
+// anti-diagonal t, launched from the last one to the first, where the pre-pass's
+// column data or the hand-off words find no memory (254 x 254 columns 19.5 ms a
+// component, 1.9 in the three kernels).
 #define MA_SLOTS 18
-template <int COMP>
-__global__ __launch_bounds__(WAVE) void k_adj_mom(const Dom *__restrict__ ds, MomAdj m, int IS, int JS) {
+template <int COMP, bool DIAG>
+__global__ __launch_bounds__(WAVE) void k_adj_mom(const Dom *__restrict__ ds, MomAdj m, int t, int IS, int JS) {
     const DomG &d = *reinterpret_cast<const DomG *>(ds);       // its swept field is X before the sweep
     extern __shared__ float sm[];
-    const int i = blockIdx.x / d.nj2, j = blockIdx.x % d.nj2;
-    if (m.col[blockIdx.x].z < 0) return;
+    int i = blockIdx.x / d.nj2, j = blockIdx.x % d.nj2;
+    if (DIAG) {
+        int a, b;
+        if (!diag_col(t, (COMP == 0) ? 3 : 2, d.nii - 1, (COMP == 1) ? 3 : 2, d.njj - 1, blockIdx.x, a, b)) return;
+        sweep_to_ij(d, 0, a, b, IS, JS, i, j);
+        if (d.adv[c2(d, i, j)] != 1) return;
+    } else if (m.col[blockIdx.x].z < 0) return;
     const ColInfo q = col_info(d, i, j);
     const int nkp = d.nkp, lane = threadIdx.x;
     const int KK = q.KK, KKP1 = KK + 1, KSTART = q.KSTART, VI = q.VI;
@@ -4373,14 +4381,27 @@ __global__ __launch_bounds__(WAVE) void k_adj_mom(const Dom *__restrict__ ds, Mo
         const float xs = (JS == 1) ? xpb : xnb, xn = (JS == 1) ? xnb : xpb;
         sA[k] = pc.A; sB[k] = pc.B; sC[k] = pc.C;
         sD[k] = ml_source<COMP>(d, q, k, d.dzk[k], pc, xw, xs, xe, xn, x);
-        const float dk = (COMP == 0 ? dyk : dxk) * d.dzk[k];
-        sG[k] = m.gin[o + k] + adj_mom_pa<COMP>(m.db[ona + k], m.ca[ona + k], m.cc[ona + k], dk) +
-                adj_mom_pb<COMP>(m.db[onb + k], m.cb[onb + k], m.cc[onb + k], dk);
-        sT[k] = m.T[o + k]; sP[k] = m.P[o + k]; sQ[k] = m.Q[o + k];
+        if (DIAG) {
+            sG[k] = m.gin[o + k] + m.gpa[ona + k] + m.gpb[onb + k];
+        } else {
+            const float dk = (COMP == 0 ? dyk : dxk) * d.dzk[k];
+            sG[k] = m.gin[o + k] + adj_mom_pa<COMP>(m.db[ona + k], m.ca[ona + k], m.cc[ona + k], dk) +
+                    adj_mom_pb<COMP>(m.db[onb + k], m.cb[onb + k], m.cc[onb + k], dk);
+            sT[k] = m.T[o + k]; sP[k] = m.P[o + k]; sQ[k] = m.Q[o + k];
+        }
     }
     for (int k = KSTART + lane; k <= VI + 1; k += WAVE) sXa[k] = XA[o + k];
     __syncthreads();
     if (lane == 0) {
+        if (DIAG) {                                           // Thomas forward, as the sweep ran it
+            float Pp = 0.0f, Qp = 0.0f;
+            for (int k = KSTART; k <= VI; ++k) {
+                float T;
+                if (k > KKP1) { T = 1 / (sA[k] - sC[k] * Pp); Pp = sB[k] * T; Qp = (sD[k] + sC[k] * Qp) * T; }
+                else { T = 1 / sA[k]; Pp = sB[k] * T; Qp = sD[k] * T; }
+                sT[k] = T; sP[k] = Pp; sQ[k] = Qp;
+            }
+        }
         // relaxed back-substitution X_k += relax (P_k X_{k+1} + Q_k - X_k) from VI down, transposed
         const float rl = d.relax;
         float ub = 0.0f;
@@ -4492,6 +4513,10 @@ __global__ __launch_bounds__(WAVE) void k_adj_mom(const Dom *__restrict__ ds, Mo
             }
         }
         sUp[k] = up; sDn[k] = dn; sMid[k] = xb;
+        if (DIAG) {                                           // the adjoints of the predecessors' new values
+            m.gpa[o + k] = (IS == 1) ? xwb : xeb;
+            m.gpb[o + k] = (JS == 1) ? xsb : xnb_;
+        }
         // the adjoints of the successors' old values
         m.gna[o + k] = (IS == 1) ? xeb : xwb;
         m.gnb[o + k] = (JS == 1) ? xnb_ : xsb;
@@ -4512,7 +4537,7 @@ __global__ __launch_bounds__(WAVE) void k_adj_mom(const Dom *__restrict__ ds, Mo
 // predecessors handed to its old value, and, where the sweep left X as it was
 // (columns it does not visit, levels outside KSTART..VI), dL/dX after with the
 // adjoints its successors handed to its new value.  Thread per cell and level.
-template <int COMP>
+template <int COMP, bool DIAG>
 __global__ void k_adj_mom_combine(const Dom *__restrict__ ds, MomAdj m, int IS, int JS) {
     const DomG &d = *reinterpret_cast<const DomG *>(ds);
     const size_t n3 = (size_t)(d.nii + 2) * d.nj2 * d.nkp;
@@ -4539,8 +4564,8 @@ __global__ void k_adj_mom_combine(const Dom *__restrict__ ds, MomAdj m, int IS, 
         v += m.gin[g];
         const float dk = (COMP == 0 ? d.dyk : d.dxk) * d.dzk[k];
         const size_t na = c3(d, i + IS, j) + k, nb = c3(d, i, j + JS) + k;
-        if (inside(i + IS, j)) v += adj_mom_pa<COMP>(m.db[na], m.ca[na], m.cc[na], dk);
-        if (inside(i, j + JS)) v += adj_mom_pb<COMP>(m.db[nb], m.cb[nb], m.cc[nb], dk);
+        if (inside(i + IS, j)) v += DIAG ? m.gpa[na] : adj_mom_pa<COMP>(m.db[na], m.ca[na], m.cc[na], dk);
+        if (inside(i, j + JS)) v += DIAG ? m.gpb[nb] : adj_mom_pb<COMP>(m.db[nb], m.cb[nb], m.cc[nb], dk);
     }
     m.gres[g] = v;
 }
@@ -4593,15 +4618,22 @@ extern "C" int pf_launch_momentum_vjp(const Dom *hd, const Dom *dd, const MomAdj
     const MomAdj m = *ma;
     const size_t n3 = (size_t)(h.nii + 2) * h.nj2 * h.nkp;
     const unsigned fb = (unsigned)((n3 + 255) / 256);
-    float *z[3] = {m.gout, m.gna, m.gnb};
-    for (float *p : z) hipLaunchKernelGGL(k_mom_fill, dim3(fb), dim3(256), 0, s, p, n3);
-    const int oa = (comp == 0) ? 3 : 2, ia = (comp == 1) ? 3 : 2, ni = h.nii - oa, nj = h.njj - ia;
+    const bool diag = m.hand == nullptr;                      // no column data and words: per anti-diagonal
+    float *z[5] = {m.gout, m.gna, m.gnb, m.gpa, m.gpb};
+    for (int q = 0; q < (diag ? 5 : 3); ++q) hipLaunchKernelGGL(k_mom_fill, dim3(fb), dim3(256), 0, s, z[q], n3);
+    const int oa = (comp == 0) ? 3 : 2, ia = (comp == 1) ? 3 : 2, ob = h.nii - 1, ib = h.njj - 1, ni = h.nii - oa, nj = h.njj - ia;
     const int ncol = (h.nii + 2) * h.nj2;
     const size_t shm_p = (sizeof(float) * 5 * (h.nkp | 1) + sizeof(int) * 4) * MA_COLS, shm = sizeof(float) * MA_SLOTS * h.nkp;
-    hipLaunchKernelGGL(k_zero_rows, dim3((unsigned)((5 * h.sync_stride + 255) / 256)), dim3(256), 0, s, dd, 0);
     int e = 0;
     auto run = [&](auto tag) {
         constexpr int C = decltype(tag)::value;
+        if (diag) {
+            for (int t = ndiag(oa, ob, ia, ib) - 1; t >= 0; --t)
+                hipLaunchKernelGGL((k_adj_mom<C, true>), dim3((unsigned)diag_len(t, oa, ob, ia, ib)), dim3(WAVE), shm, s, dd, m, t, IS, JS);
+            hipLaunchKernelGGL((k_adj_mom_combine<C, true>), dim3(fb), dim3(256), 0, s, dd, m, IS, JS);
+            return;
+        }
+        hipLaunchKernelGGL(k_zero_rows, dim3((unsigned)((5 * h.sync_stride + 255) / 256)), dim3(256), 0, s, dd, 0);
         hipLaunchKernelGGL(k_adj_mom_pre<C>, dim3((ncol + MA_COLS - 1) / MA_COLS), dim3(4 * WAVE), shm_p, s, dd, m, IS, JS);
         if (ni > 0 && nj > 0) {
             // the sweep's order reversed: from its last row and column back
@@ -4609,15 +4641,14 @@ extern "C" int pf_launch_momentum_vjp(const Dom *hd, const Dom *dd, const MomAdj
             const MomOp<C> op{m, h.dzk, C == 0 ? h.dyk : h.dxk, h.relax, h.nkp};
             const LineSweep w{ni, nj, i0 * h.nj2 + j0, -IS * h.nj2, -JS, h.nkp, h.sync, SYNC_BLOCK0, 6, m.hand, nullptr};
             e = h.nkp <= WAVE ? launch_line<MomOp<C>, 1>(op, w, s) : launch_line<MomOp<C>, 2>(op, w, s);
-            if (!e) hipLaunchKernelGGL(k_adj_mom<C>, dim3(ncol), dim3(WAVE), shm, s, dd, m, IS, JS);
+            if (e) return;
+            hipLaunchKernelGGL((k_adj_mom<C, false>), dim3(ncol), dim3(WAVE), shm, s, dd, m, 0, IS, JS);
         }
+        hipLaunchKernelGGL((k_adj_mom_combine<C, false>), dim3(fb), dim3(256), 0, s, dd, m, IS, JS);
     };
     if (comp == 0) run(std::integral_constant<int, 0>()); else if (comp == 1) run(std::integral_constant<int, 1>());
     else run(std::integral_constant<int, 2>());
     if (e) return e;
-    if (comp == 0) hipLaunchKernelGGL(k_adj_mom_combine<0>, dim3(fb), dim3(256), 0, s, dd, m, IS, JS);
-    else if (comp == 1) hipLaunchKernelGGL(k_adj_mom_combine<1>, dim3(fb), dim3(256), 0, s, dd, m, IS, JS);
-    else hipLaunchKernelGGL(k_adj_mom_combine<2>, dim3(fb), dim3(256), 0, s, dd, m, IS, JS);
     return (int)hipGetLastError();
 }
 
