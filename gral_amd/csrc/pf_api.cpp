@@ -22,6 +22,7 @@
 
 #include "../../include/gral_pf.h"
 #include "pf_device.h"
+#include "pf_host.h"
 #include "pf_spare.h"
 
 // Levels per device column: KADVMAX + 2 rounded up to a multiple of NKP_ALIGN
@@ -70,29 +71,6 @@ inline double dmax_net(double a, double b) {
     return std::signbit(b) ? a : b;
 }
 
-// Host loops over columns or rows run on up to 16 threads: each element is
-// computed as in a serial loop, and the only reductions (a maximum, counts)
-// do not depend on the order.
-unsigned host_threads() {
-    static const unsigned n = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
-    return n;
-}
-template <class Fn>
-void par_for(long lo, long hi, Fn fn) {            // fn(t, a, b): thread t covers [a, b)
-    const long n = hi - lo;
-    if (n <= 0) return;
-    const long T = std::min<long>(host_threads(), n);
-    if (T <= 1) { fn(0, lo, hi); return; }
-    const long chunk = (n + T - 1) / T;
-    std::vector<std::thread> th;
-    th.reserve((size_t)T - 1);
-    for (long t = 1; t < T; ++t) {
-        const long a = lo + t * chunk, b = std::min(hi, a + chunk);
-        if (a < b) th.emplace_back(fn, (int)t, a, b);
-    }
-    fn(0, lo, std::min(hi, lo + chunk));
-    for (auto &x : th) x.join();
-}
 void par_copy(void *dst, const void *src, size_t bytes) {
     const size_t blk = size_t(1) << 22;
     par_for(0, (long)((bytes + blk - 1) / blk), [&](int, long a, long b) {
@@ -2466,18 +2444,9 @@ extern "C" int gral_pf_wind_at_particles(gral_pf_handle *h, int32_t topo, int32_
         return fail(h, GRAL_PF_EINVAL, "wind_at_particles: null argument");
     StripUse use({h});
     if (use.rc) return fail(h, GRAL_PF_EDEVICE, "wind_at_particles: upload of the situation failed");
-    std::atomic<int32_t> bad{n};                          // the first particle outside the grid
-    par_for(0, (n + 65535) / 65536, [&](int, long a, long b) {
-        const int32_t e = (int32_t)std::min<long>(n, b * 65536);
-        for (int32_t p = (int32_t)(a * 65536); p < e; ++p)
-            if (cell_i[p] < 1 || cell_i[p] > h->nii || cell_j[p] < 1 || cell_j[p] > h->njj) {
-                int32_t o = bad.load();
-                while (p < o && !bad.compare_exchange_weak(o, p)) {}
-                break;
-            }
-    });
-    if (bad.load() < n)
-        return fail(h, GRAL_PF_EINVAL, "wind_at_particles: particle " + std::to_string(bad.load()) + " outside the cells 1..NII x 1..NJJ");
+    const int32_t bad = first_outside(n, cell_i, cell_j, h->nii, h->njj);
+    if (bad < n)
+        return fail(h, GRAL_PF_EINVAL, "wind_at_particles: particle " + std::to_string(bad) + " outside the cells 1..NII x 1..NJJ");
     const int nlo = std::min(h->nkp, h->nkh);
     int rc = gff_upper(h, nlo);
     if (rc) return rc;
