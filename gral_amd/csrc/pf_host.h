@@ -8,9 +8,9 @@
 
 namespace {
 
-// Host loops over columns or rows run on up to 16 threads: each element is
-// computed as in a serial loop, and the only reductions (a maximum, counts)
-// do not depend on the order.
+// Host loops over columns or rows run on up to 16 threads, fewer where no more can
+// be started: each element is computed as in a serial loop, and the only
+// reductions (a maximum, counts) do not depend on the order.
 inline unsigned host_threads() {
     static const unsigned n = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
     return n;
@@ -23,12 +23,15 @@ void par_for(long lo, long hi, Fn fn) {            // fn(t, a, b): thread t cove
     if (T <= 1) { fn(0, lo, hi); return; }
     const long chunk = (n + T - 1) / T;
     std::vector<std::thread> th;
-    th.reserve((size_t)T - 1);
-    for (long t = 1; t < T; ++t) {
-        const long a = lo + t * chunk, b = std::min(hi, a + chunk);
-        if (a < b) th.emplace_back(fn, (int)t, a, b);
+    long t = 1;
+    auto from = [&](long q) { return std::min(hi, lo + q * chunk); };
+    try {
+        th.reserve((size_t)T - 1);
+        for (; t < T && from(t) < hi; ++t) th.emplace_back(fn, (int)t, from(t), from(t + 1));
+    } catch (...) {                                // no further thread: its part and the rest here
     }
-    fn(0, lo, std::min(hi, lo + chunk));
+    fn(0, lo, from(1));
+    for (; t < T && from(t) < hi; ++t) fn((int)t, from(t), from(t + 1));
     for (auto &x : th) x.join();
 }
 // the first of n particles outside the cells 1..nii x 1..njj; n if there is none
