@@ -194,7 +194,8 @@ struct gral_pf_handle {
     std::vector<int> vi;
     // run state
     gral_pf_params prm{};
-    bool prepared = false, done = false, host_stale = false;
+    bool prepared = false, done = false;
+    unsigned host_stale = 0;        // fields newer on the device than their host copies (bits in solver_fields()' order)
     int iter_loops = 1, iters_run = 0, processed = 0;
     double delta_mean = 0, last_delta = 0;
     float delta_first = 0, delta_finish = 0;
@@ -644,12 +645,14 @@ static int mass_blocks(int nii, int njj) {
 // One transfer between device memory and pageable host memory: rows of width
 // bytes, pitch_d apart on the device (the rows fill its bytes without other
 // gaps) and pitch_h apart on the host.  To the device, the rest of a row is
-// zeroed; to the host, it comes from rest (the same layout as host) if given.
+// zeroed; to the host, it comes from rest (the same layout as host) if given, and
+// the row goes to also (the same layout) too.
 struct Move {
     char *dev;
     char *host;
     size_t rows, pitch_d, pitch_h, width;
     const char *rest;
+    char *also = nullptr;
 };
 static Move move_bytes(const void *dev, const void *host, size_t bytes) {
     // one array without pitch, in rows of 64 KB; the last one may be partial
@@ -730,6 +733,7 @@ static int move_all(gral_pf_handle *h, bool to_dev, const std::vector<Move> &mv)
                     if (m.width < m.pitch_d) std::memset(s + m.width, 0, m.pitch_d - m.width);
                 } else {
                     std::memcpy(x, s, m.width);
+                    if (m.also) std::memcpy(m.also + r * m.pitch_h, s, m.width);
                     if (m.rest && m.rest != m.host) std::memcpy(x + m.width, m.rest + r * m.pitch_h + m.width, m.pitch_h - m.width);
                 }
             }
@@ -829,16 +833,18 @@ static bool same_kind(const gral_pf_handle *a, const gral_pf_handle *b) {
     return a->d.model == b->d.model && (tall(a) || a->diag) == (tall(b) || b->diag);
 }
 
-// the fields the device holds, with their host copies
-static std::vector<Move> solver_fields(const gral_pf_handle *h) {
+// the fields the device holds, with their host copies; TURB and TDISS last, which
+// the mixing-length model leaves as they are
+static unsigned all_fields(const gral_pf_handle *h) { return h->prm.turbulence_model != 1 ? 0x3ff : 0xff; }
+static std::vector<Move> solver_fields(const gral_pf_handle *h, unsigned which) {
     const Dom &d = h->d;
-    std::vector<Move> v = {field_move(h, d.uk, h->uk.data()), field_move(h, d.vk, h->vk.data()), field_move(h, d.wk, h->wk.data()),
-                           field_move(h, d.uks, h->uks.data()), field_move(h, d.vks, h->vks.data()), field_move(h, d.wks, h->wks.data()),
-                           field_move(h, d.dpm, h->dpm.data()), field_move(h, d.dpmnew, h->dpmnew.data())};
-    if (h->prm.turbulence_model != 1) {
-        v.push_back(field_move(h, d.turb, h->turb.data()));
-        v.push_back(field_move(h, d.tdiss, h->tdiss.data()));
-    }
+    const struct { const float *dev, *host; } f[10] = {
+        {d.uk, h->uk.data()}, {d.vk, h->vk.data()}, {d.wk, h->wk.data()}, {d.uks, h->uks.data()}, {d.vks, h->vks.data()},
+        {d.wks, h->wks.data()}, {d.dpm, h->dpm.data()}, {d.dpmnew, h->dpmnew.data()}, {d.turb, h->turb.data()},
+        {d.tdiss, h->tdiss.data()}};
+    std::vector<Move> v;
+    for (int q = 0; q < 10; ++q)
+        if (which & (1u << q)) v.push_back(field_move(h, f[q].dev, f[q].host));
     return v;
 }
 
@@ -848,7 +854,7 @@ extern "C" int gral_pf_prepare(gral_pf_handle *h, const gral_pf_params *p) {
     // earlier prepare is released below, so nothing may run on it afterwards
     h->prepared = false;
     h->done = false;
-    h->host_stale = false;
+    h->host_stale = 0;
     h->gff_ok = false;
     if (!p) return fail(h, GRAL_PF_EINVAL, "prepare: null params");
     if (!h->masks || !h->rough || !h->fields) return fail(h, GRAL_PF_ESTATE, "prepare: masks, roughness and fields must be set first");
@@ -1073,7 +1079,7 @@ extern "C" int gral_pf_prepare(gral_pf_handle *h, const gral_pf_params *p) {
         d.vegp = nullptr; d.veg = nullptr;
     }
     std::vector<float> zeros;
-    if ((rc = move_all(h, true, solver_fields(h)))) return rc;
+    if ((rc = move_all(h, true, solver_fields(h, all_fields(h))))) return rc;
     HIPCHK(h, hipMemsetAsync(d.div, 0, n3 * sizeof(float), h->stream));
     if (p->turbulence_model == 1) {
         HIPCHK(h, hipMemsetAsync(d.turb, 0, n3 * sizeof(float), h->stream));
@@ -1093,7 +1099,7 @@ extern "C" int gral_pf_prepare(gral_pf_handle *h, const gral_pf_params *p) {
     if (h->spare) g_spares.add(h->spare);
     h->gff_ok = false;
     h->done = false;
-    h->host_stale = false;
+    h->host_stale = 0;
     h->iter_loops = 1;
     h->iters_run = 0;
     h->processed = 0;
@@ -1477,7 +1483,7 @@ static void run_lockstep(const std::vector<gral_pf_handle *> &hs, Dom *dd, hipSt
                 h->iter_loops = it + 1;
             }
             if (h->iter_loops > h->prm.iter_max) h->done = true;
-            h->host_stale = true;
+            h->host_stale = all_fields(h);
             h->mom_vjp_ok = false;
             if (!h->done) keep.push_back(h);
         }
@@ -1523,10 +1529,10 @@ static void vks_upper(gral_pf_handle *h) {
 
 static int sync_host(gral_pf_handle *h) {
     if (!h->host_stale) return 0;
-    const int rc = move_all(h, false, solver_fields(h));
+    const int rc = move_all(h, false, solver_fields(h, h->host_stale));
     if (rc) return rc;
     vks_upper(h);
-    h->host_stale = false;
+    h->host_stale = 0;
     return 0;
 }
 
@@ -1697,7 +1703,7 @@ extern "C" int gral_pf_forward_ckpt(gral_pf_handle *h, int32_t n, int32_t quanti
     h->adj_n = n;
     h->mom_comp = -1;
     h->mom_vjp_ok = false;
-    h->host_stale = true;
+    h->host_stale = all_fields(h);
     h->gff_ok = false;
     return GRAL_PF_OK;
 }
@@ -1712,7 +1718,7 @@ extern "C" int gral_pf_restore_ckpt(gral_pf_handle *h) {
     HIPCHK(h, hipMemcpyAsync(h->d.vk, ck + n3, n3 * sizeof(float), hipMemcpyDeviceToDevice, h->stream));
     HIPCHK(h, hipMemcpyAsync(h->d.wk, ck + 2 * n3, n3 * sizeof(float), hipMemcpyDeviceToDevice, h->stream));
     HIPCHK(h, hipStreamSynchronize(h->stream));
-    h->host_stale = true;
+    h->host_stale = all_fields(h);
     h->gff_ok = false;
     h->mom_vjp_ok = false;
     return GRAL_PF_OK;
@@ -1835,7 +1841,7 @@ extern "C" int gral_pf_momentum_sweep(gral_pf_handle *h, int32_t comp) {
     h->mom_js = JS;
     h->mom_vjp_ok = true;
     h->adj_n = 0;
-    h->host_stale = true;
+    h->host_stale = all_fields(h);
     h->gff_ok = false;
     return GRAL_PF_OK;
 }
@@ -1900,24 +1906,29 @@ extern "C" int gral_pf_download_fields(gral_pf_handle *h, float *uk, float *vk, 
     if (!h) return GRAL_PF_EINVAL;
     if (!h->prepared && !h->fields) return fail(h, GRAL_PF_ESTATE, "download: upload fields first");
     const size_t n3 = h->n2() * (size_t)h->nkh;
-    const Dom &d = h->d;
-    struct { float *dst; std::vector<float> *src; const float *dev; } f[10] = {
-        {uk, &h->uk, d.uk}, {vk, &h->vk, d.vk}, {wk, &h->wk, d.wk}, {uks, &h->uks, d.uks}, {vks, &h->vks, d.vks},
-        {wks, &h->wks, d.wks}, {dpm, &h->dpm, d.dpm}, {dpmnew, &h->dpmnew, d.dpmnew}, {turb, &h->turb, d.turb},
-        {tdiss, &h->tdiss, d.tdiss}};
-    const int nf = h->host_stale ? (h->prm.turbulence_model != 1 ? 10 : 8) : 0;
-    // fields newer on the device: straight into the caller's array, the levels
-    // above the device's from the host copy
-    std::vector<Move> mv;
-    if (nf && vks) vks_upper(h);
-    for (int q = 0; q < nf; ++q)
-        if (f[q].dst) mv.push_back(field_move(h, f[q].dev, f[q].dst, f[q].src->data()));
+    float *dst[10] = {uk, vk, wk, uks, vks, wks, dpm, dpmnew, turb, tdiss};
+    std::vector<float> *src[10] = {&h->uk, &h->vk, &h->wk, &h->uks, &h->vks, &h->wks, &h->dpm, &h->dpmnew, &h->turb, &h->tdiss};
+    // fields newer on the device: into the caller's array and the host copy at
+    // once, the levels above the device's from the host copy
+    unsigned now = 0;
+    for (int q = 0; q < 10; ++q)
+        if (dst[q]) now |= h->host_stale & (1u << q);
+    std::vector<Move> mv = solver_fields(h, now);
+    for (int q = 0, m = 0; q < 10; ++q) {
+        if (!(now & (1u << q))) continue;
+        Move &x = mv[m++];
+        x.also = x.host;
+        x.rest = x.host;
+        x.host = (char *)dst[q];
+    }
+    if (h->host_stale && vks) vks_upper(h);
     const int rc = move_all(h, false, mv);
     if (rc) return rc;
-    for (int q = nf; q < 10; ++q) {
-        if (!f[q].dst) continue;
-        if (f[q].src->size() == n3) par_copy(f[q].dst, f[q].src->data(), n3 * sizeof(float));
-        else std::memset(f[q].dst, 0, n3 * sizeof(float));
+    h->host_stale &= ~now;
+    for (int q = 0; q < 10; ++q) {
+        if (!dst[q] || (now & (1u << q))) continue;
+        if (src[q]->size() == n3) par_copy(dst[q], src[q]->data(), n3 * sizeof(float));
+        else std::memset(dst[q], 0, n3 * sizeof(float));
     }
     return GRAL_PF_OK;
 }
@@ -2282,7 +2293,7 @@ extern "C" int gral_pf_diagnostic(gral_pf_handle *h, int32_t flow_field_level, i
     if ((rc = move_all(h, false, mv))) { cleanup(); return rc; }
     cleanup();
     h->diag_dtime = dt;
-    h->host_stale = false;
+    h->host_stale = 0;
     h->gff_ok = false;
     if (h->prepared) {
         // keep the solver's device state (levels below nkp) equal to the host's
