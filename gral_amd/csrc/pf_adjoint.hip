@@ -79,7 +79,7 @@ __global__ void k_adj_correction(const Dom *__restrict__ ds, AdjArgs a) {
 
 // S^T runs on strips (pf_launch_adjoint_sweep: 256 x 256 columns of up to 47 levels
 // 1.37 ms, with one launch per anti-diagonal 2.5 ms), whose columns hold 256 levels.  For
-// taller ones: anti-diagonal t of the sweep (a = j1 outer, b = i1 inner, mirrored
+// taller ones, and where the hand-off words find no memory: anti-diagonal t of the sweep (a = j1 outer, b = i1 inner, mirrored
 // by IS/JS as in the forward), launched from the last diagonal to the first.
 // One wave per column: the lanes stage the column's vectors and its P, TERMP
 // and ATP in LDS, lane 0 runs the transposed recurrences over LDS in blocks of

@@ -1273,8 +1273,10 @@ struct StreamGroup {
 };
 
 // groups a lock-step batch of n situations may run in: at most n / 2 and 4
-// (one stream per hardware queue).  Measured on the 8-direction city batch:
-// 24.30 ms per iteration in one group, 23.28 in two, 23.09 in four.
+// (one stream per hardware queue).  Measured on the 8-direction city batch, five
+// runs each: 13.80-13.82 ms per iteration in one group, 13.20-13.26 in two,
+// 12.73-12.79 in four (k-eps 20.5, 20.2-20.3, 20.0-20.5); 32 situations 46.6 in one,
+// 43.7 in four.
 static int max_groups(size_t n) { return (int)std::max<size_t>(1, std::min<size_t>(n / 2, (size_t)kMaxGroups)); }
 // GRAL_PF_GROUPS (1 to 4) fixes the count; 0 if unset
 static int forced_groups() {

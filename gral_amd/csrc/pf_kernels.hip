@@ -3570,13 +3570,13 @@ static StripKernel tke_strip(const Dom *hd, int nsit) {
 // Rows of a strip.  A strip is a workgroup of rows + 2 waves; fewer rows mean
 // less work per step and CU, more strips and (a sweep's path is its column
 // range plus rows per strip) about the same number of steps.  Ten rows while
-// all strips of the launch find a CU of their own (400 x 400 city, one
-// situation: pressure, U and V sweeps 1.33, 1.41 and 1.38 ms against 1.42, 1.48
-// and 1.48 with 14), else 14 (eight situations: 1.62, 2.04 and 1.71 ms against
-// 1.80, 2.16 and 1.91 with ten).  Short sweeps, whose path is mostly the fill of
-// their first strips, take seven (25 rows: 60 against 65 us).  swap: the
-// pressure sweep, whose rows run along i; lds: the kernel's LDS at a row count
-// (tall columns take fewer rows).
+// all strips of the launch find a CU of their own, not counting those of stream
+// groups that run beside it (400 x 400 city, one situation: pressure, U and V
+// sweeps 1.33, 1.41 and 1.38 ms against 1.42, 1.48 and 1.48 with 14), else 14
+// (eight situations: 1.62, 2.04 and 1.71 ms against 1.80, 2.16 and 1.91 with ten).
+// Short sweeps, whose path is mostly the fill of their first strips, take seven
+// (25 rows: 60 against 65 us).  swap: the pressure sweep, whose rows run along i;
+// lds: the kernel's LDS at a row count (tall columns take fewer rows).
 #define LDS_BYTES (160 * 1024)
 static int strip_rows(const Dom *hd, int nsit, bool swap, size_t (*lds)(const Dom *, int, int)) {
     long n = 0, longest = 0;
@@ -3593,7 +3593,9 @@ template <int COMP, int WFIX, int KIND>
 static StripKernel ml_strip(const Dom *hd, int nsit) {
     int n = 0;
     for (int q = 0; q < nsit; ++q) n = max(n, (COMP == 2 ? hd[q].nlow : 0) + hd[q].nact + 1);
-    if constexpr (COMP == 2)                                  // buildings add to the W sweep's columns
+    // buildings add to the W sweep's columns; with 4 groups (from 193 levels) it spills 76 to 156
+    // bytes a lane at the 128 registers that 16 waves leave, the 16-wide one with 3 groups 20
+    if constexpr (COMP == 2)
         if (n > 2 * WAVE) return n <= 3 * WAVE ? k_ml_strip<COMP, WFIX, KIND, 3> : k_ml_strip<COMP, WFIX, KIND, 4>;
     return n <= WAVE ? k_ml_strip<COMP, WFIX, KIND, 1> : k_ml_strip<COMP, WFIX, KIND, 2>;
 }

@@ -117,7 +117,9 @@ int gral_pf_set_met_profile(gral_pf_handle *h, int32_t istatistics, int32_t n_pr
 int gral_pf_upload_fields(gral_pf_handle *h, const float *uk, const float *vk, const float *wk);
 
 /* Prologue of Calculate() (PrognosticFlowfield.cs:145-579) and transfer of the
- * solver state to the GPU. */
+ * solver state to the GPU.  Where the device has no memory left, it takes what
+ * situations of more than 126 levels can do without, which then iterate slower to
+ * the same results, and may wait for a running call on one of them to end. */
 int gral_pf_prepare(gral_pf_handle *h, const gral_pf_params *p);
 
 /* Runs up to n SIMPLE iterations (PrognosticFlowfield.cs:584-1178) on the
@@ -421,7 +423,8 @@ int gral_pf_wind_at_particles(gral_pf_handle *h, int32_t topo, int32_t ikooagral
  * batch when the reference's stop test (PrognosticFlowfield.cs:1149-1166)
  * ends it (early retirement); its results are bit-identical to a plain
  * gral_pf_solve of the same situation.  Situations of one batch must use the
- * same turbulence model.  The handles stay owned by the caller and must
+ * same turbulence model, and columns of more than 126 levels (KADVMAX + 2 > 128)
+ * are not batched with lower ones.  The handles stay owned by the caller and must
  * outlive the batch; after the batch, gral_pf_finish/download_fields work on
  * each handle as after gral_pf_iterate. */
 typedef struct gral_pf_batch gral_pf_batch;
